@@ -193,9 +193,10 @@ typedef struct {
     const double* x0;    /* optional warm start (n+m-1), host; NULL = reference init */
     int bcd_batch;       /* BCD iterations enqueued per batch (two in flight); <= 0: 8 */
     /* BCD iteration form.  0: two passes over M per iteration (row pass,
-     * column pass); nonzero (default 1): one pass per iteration when M is
-     * FP32, 1024 < m <= 16384, at most 1024 rows fall to each compute unit
-     * and min a min b >= 2^-60 sum a sum b; the two-pass form otherwise. */
+     * column pass); nonzero (default 1): one pass per iteration when
+     * m <= 8192 (FP32 bulk in FP32 arithmetic: m <= 16384), at most 1024 rows
+     * fall to each compute unit and min a min b >= 2^-60 sum a sum b; the
+     * two-pass form otherwise. */
     int bcd_fused;
     double tau;          /* QROT gradient descent / L-BFGS: extra term tau/2 (1'alpha - 1'beta)^2
                             (QROTSolverOpts::tau, src/qrot_solvers.h:15-30); default 0 */
@@ -405,7 +406,8 @@ int regot_qrot_primal_val(regot_problem* p, const double* gamma, double* value);
 
 /* Device-side timing of the hot kernels (HIP events on the handle's stream).
  * kind: 0 = row pass, 1 = column pass (partial + combine), 2 = single-read
- * BCD pass, 3 = its column-sum combine.  Enabled by regot_profile_enable(p, 1);
+ * BCD pass, 3 = its column-sum combine (FP32 arithmetic), 4 and 5 = the same
+ * two in FP64 arithmetic.  Enabled by regot_profile_enable(p, 1);
  * totals accumulate until reset. */
 int regot_profile_enable(regot_problem* p, int on);
 int regot_profile_get(regot_problem* p, int kind, long long* launches, double* total_ms);

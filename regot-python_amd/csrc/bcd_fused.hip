@@ -1,4 +1,6 @@
-// bcd_fused.hip -- one BCD iteration in one read of the cost matrix (FP32 bulk).
+// bcd_fused.hip -- one BCD iteration in one read of the cost matrix (FP32 bulk,
+// 8192 < m <= 16384; narrower matrices and FP64: bcd_rows.hip, where several
+// rows share a barrier).
 //
 // A BCD iteration is alpha <- optimal_alpha(beta), then beta <-
 // optimal_beta(alpha) (src/sinkhorn_bcd.cpp:65-103).  Both half-steps need a
@@ -107,7 +109,7 @@ __global__ __launch_bounds__(kFThreads) void k_bcd_fused(
     const float* __restrict__ M, long ldm, int n, int m, const double* __restrict__ beta,
     double k, double reg, const double* __restrict__ loga, const double* __restrict__ a,
     const double* __restrict__ alpha, double* __restrict__ alpha_out, int rpw,
-    double* __restrict__ part, double* __restrict__ rpart, double* __restrict__ bm,
+    double* __restrict__ part, long pitch, double* __restrict__ rpart,
     const int* __restrict__ ctl, int nt)
 {
     if (ctl[0] != 0) return;
@@ -240,7 +242,7 @@ __global__ __launch_bounds__(kFThreads) void k_bcd_fused(
         }
     }
 
-    double* pw = part + static_cast<long>(blockIdx.x) * m;
+    double* pw = part + static_cast<long>(blockIdx.x) * pitch;
 #pragma unroll
     for (int c = 0; c < NC; c++)
 #pragma unroll
@@ -272,8 +274,6 @@ __global__ __launch_bounds__(kFThreads) void k_bcd_fused(
         if (t == 0) rpart[3 * blockIdx.x + q] = tq;
         __syncthreads();
     }
-    // beta_k[m-1] for the objective (the combine overwrites beta)
-    if (t == 0 && blockIdx.x == 0) bm[0] = beta[m - 1];
 }
 
 // Two rows in flight (PF = 2) wherever that fits the 256 VGPRs of a wave
@@ -281,17 +281,17 @@ __global__ __launch_bounds__(kFThreads) void k_bcd_fused(
 template <int NC>
 void fused_launch(bool full, dim3 grid, hipStream_t s, const float* M, long ldm, int n, int m,
                   const double* beta, double k, double reg, const double* loga, const double* a,
-                  const double* alpha, double* alpha_out, int rpw, double* part, double* rpart,
-                  double* bm, const int* ctl, int nt)
+                  const double* alpha, double* alpha_out, int rpw, double* part, long pitch,
+                  double* rpart, const int* ctl, int nt)
 {
     constexpr int PFR = NC <= 6 ? 2 : 1;
     if (full)
         hipLaunchKernelGGL((k_bcd_fused<NC, true, 2>), grid, dim3(kFThreads), 0, s, M, ldm, n,
-                           m, beta, k, reg, loga, a, alpha, alpha_out, rpw, part, rpart, bm, ctl,
+                           m, beta, k, reg, loga, a, alpha, alpha_out, rpw, part, pitch, rpart, ctl,
                            nt);
     else
         hipLaunchKernelGGL((k_bcd_fused<NC, false, PFR>), grid, dim3(kFThreads), 0, s, M, ldm,
-                           n, m, beta, k, reg, loga, a, alpha, alpha_out, rpw, part, rpart, bm,
+                           n, m, beta, k, reg, loga, a, alpha, alpha_out, rpw, part, pitch, rpart,
                            ctl, nt);
 }
 
@@ -307,17 +307,17 @@ int bcd_fused_blocks(int n, int ncu)
 
 bool bcd_fused_shape_ok(int n, int m, int ncu)
 {
-    if (n < 1 || m <= 1024 || m > kFMaxNC * kFSpan) return false;
+    if (n < 1 || m <= 8192 || m > kFMaxNC * kFSpan) return false;
     return ceil_div(n, bcd_fused_blocks(n, ncu)) <= kFMaxRows;
 }
 
 void launch_bcd_fused(const void* M, long ldm, int n, int m, const double* beta, double k,
                       double reg, const double* loga, const double* a, const double* alpha,
-                      double* alpha_out, int nblk, double* part, double* rpart, double* bm,
+                      double* alpha_out, int nblk, double* part, long pitch, double* rpart,
                       const int* ctl, hipStream_t s)
 {
     const int rpw = ceil_div(n, nblk);
-    if (n < 1 || m <= 1024 || m > kFMaxNC * kFSpan || rpw > kFMaxRows)
+    if (n < 1 || m <= 8192 || m > kFMaxNC * kFSpan || rpw > kFMaxRows)
         fail(E_INTERNAL, "single-read BCD pass: shape %d x %d over %d workgroups", n, m, nblk);
     if (static_cast<long>(rpw) * (nblk - 1) >= n)
         fail(E_INTERNAL, "single-read BCD pass: %d workgroups for %d rows", nblk, n);
@@ -327,37 +327,21 @@ void launch_bcd_fused(const void* M, long ldm, int n, int m, const double* beta,
     const float* Mf = static_cast<const float*>(M);
     const dim3 grid(nblk);
     switch (NC) {
-    case 1:
-        fused_launch<1>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
-        break;
-    case 2:
-        fused_launch<2>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
-        break;
-    case 3:
-        fused_launch<3>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
-        break;
-    case 4:
-        fused_launch<4>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
-        break;
     case 5:
-        fused_launch<5>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
+        fused_launch<5>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out, rpw,
+                        part, pitch, rpart, ctl, nt);
         break;
     case 6:
-        fused_launch<6>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
+        fused_launch<6>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out, rpw,
+                        part, pitch, rpart, ctl, nt);
         break;
     case 7:
-        fused_launch<7>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
+        fused_launch<7>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out, rpw,
+                        part, pitch, rpart, ctl, nt);
         break;
     default:
-        fused_launch<8>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out,
-                        rpw, part, rpart, bm, ctl, nt);
+        fused_launch<8>(full, grid, s, Mf, ldm, n, m, beta, k, reg, loga, a, alpha, alpha_out, rpw,
+                        part, pitch, rpart, ctl, nt);
         break;
     }
     KERNEL_CHECK();

@@ -37,7 +37,8 @@ struct ColEpi {
     double* resid = nullptr;
     // Per combine workgroup t (j < m-1 only): [2t] = sum resid_j^2,
     // [2t+1] = sum beta_j b_j with beta = beta_out if set, else colpot.
-    // In BCD mode the half selected by the parity of k+1 is written.
+    // In BCD mode the half selected by the parity of k+1 is written.  Tiles
+    // are of col_combine_blocks(m) workgroups in every mode.
     double* tilepart = nullptr;
     double reg = 1.0;
 };
@@ -65,15 +66,15 @@ void launch_col_pass(int bulk, const void* M, long ldm, int n, int m, const doub
 void launch_plan(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
                  const double* beta, double reg, double* plan, long r0, int nr, hipStream_t s);
 
-// On-device BCD bookkeeping.  The row pass (FIN) publishes per-workgroup sums
-// of (g^2, r, alpha a); every combine workgroup of the same iteration then
+// On-device BCD bookkeeping.  The row pass publishes per-workgroup sums of
+// (g^2, r, alpha a); one workgroup of the same iteration's combine then
 // reduces them (with the column-tile sums of the previous update,
-// double-buffered by the parity of k) to the same f_k and ||g_k|| and takes
-// the same stop decision.  k is the iteration the launch belongs to (the host
+// double-buffered by the parity of k) to f_k and ||g_k|| and takes the stop
+// decision, while the others write beta_{k+1} to its own buffer.  k is the iteration the launch belongs to (the host
 // enqueues iterations in order; launches past the stop return at once).
 struct BcdState {
     const double* a;
-    const double* beta;
+    const double* beta;     // beta_k (the update writes another buffer)
     int k;                  // iteration of this launch
     int* ctl;               // [0] done, [1] iterations completed, [2] niter
     double* hist_f;         // rings of hist_cap entries (device-visible)
@@ -81,7 +82,6 @@ struct BcdState {
     long long* hist_ts;
     int hist_cap;
     double* rpart;          // per row-pass workgroup: sum g^2, sum r, sum alpha a
-    double* bm;             // beta_k[m-1], stored by the row pass of iteration k
     const double* cpart;    // 2 x ntiles x (sum resid^2, sum beta_j b_j), j < m-1
     int nrb;                // row-pass workgroups
     int ntiles;             // combine workgroups
@@ -106,20 +106,42 @@ void launch_row_pass_bcd(int bulk, const void* M, long ldm, int n, int m, const 
                          bool precise = false);
 int row_pass_blocks(int bulk, int n);
 
-// Single-read BCD iteration (FP32 bulk; bcd_fused.hip): per workgroup of whole
-// rows, alpha_out = optimal_alpha(beta) for its rows, the row partials of
-// BcdState (g^2, r, alpha'a at iterate k) and the FP64 column sums of
-// exp((alpha_out_i + beta_j - M_ij) / reg) over its rows into part[blk * m + j].
-// launch_col_combine_sums then finishes the iteration like the two-pass
-// combine (epi.colpot = beta).
+// Single-read BCD iteration: per workgroup of whole rows, alpha_out =
+// optimal_alpha(beta) for its rows, the row partials of BcdState (g^2, r,
+// alpha'a at iterate k) and the FP64 column sums of exp((alpha_out_i + beta_j -
+// M_ij) / reg) over its rows into part[blk * pitch + j] (pitch from
+// bcd_part_pitch).  launch_col_combine_sums then finishes the iteration like
+// the two-pass combine (epi.colpot = beta).
+// m <= 8192 (bcd_rows.hip, FP32 or FP64; precise: FP64 arithmetic over FP32 M):
+struct BcdRowsArgs {
+    const void* M;
+    long ldm;
+    int n, m;
+    const double* beta;
+    double k, reg;
+    const double* loga;
+    const double* a;
+    const double* alpha;
+    double* alpha_out;
+    int nblk;               // workgroups (bcd_fused_blocks)
+    double* part;
+    long pitch;
+    double* rpart;
+    const int* ctl;
+    int rpw, nt;            // set by the launcher
+};
+bool bcd_rows_shape_ok(int n, int m, int ncu);
+long bcd_part_pitch(int m);
+void launch_bcd_rows(int bulk, bool precise, BcdRowsArgs g, hipStream_t s);
+// 8192 < m <= 16384, FP32 (bcd_fused.hip):
 bool bcd_fused_shape_ok(int n, int m, int ncu);
 int bcd_fused_blocks(int n, int ncu);
 void launch_bcd_fused(const void* M, long ldm, int n, int m, const double* beta, double k,
                       double reg, const double* loga, const double* a, const double* alpha,
-                      double* alpha_out, int nblk, double* part, double* rpart, double* bm,
+                      double* alpha_out, int nblk, double* part, long pitch, double* rpart,
                       const int* ctl, hipStream_t s);
-void launch_col_combine_sums(const double* part, int nblk, int m, double k, const ColEpi& epi,
-                             const BcdState& st, hipStream_t s);
+void launch_col_combine_sums(const double* part, long pitch, int nblk, int m, double k,
+                             const ColEpi& epi, const BcdState& st, hipStream_t s);
 
 void launch_fill(double* p, double v, long count, hipStream_t s);
 void launch_fill_int(int* p, int v, long count, hipStream_t s);

@@ -112,11 +112,30 @@ __device__ __forceinline__ double dpp_f64(double v)
     return __hiloint2double(hi, lo);
 }
 
+// x[lane] + x[lane ^ 16] and x[lane] + x[lane ^ 32] on every lane, without LDS:
+// v_permlane16_swap of x with itself leaves the even rows' values in one result
+// and the odd rows' in the other (v_permlane32_swap: the two halves).
+__device__ __forceinline__ double xor16_sum(double x)
+{
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(x), __double2loint(x), false,
+                                                     false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(x), __double2hiint(x), false,
+                                                     false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double xor32_sum(double x)
+{
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(x), false,
+                                                     false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(x), false,
+                                                     false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
 // R wave sums together: lane pairs xor 1 and xor 2 (quad permutes), then the
 // mirrored halves of each 8 and each 16 lanes (DPP), then xor 16 and xor 32
-// (shuffles issued for all R values before their adds).  Each step adds two
-// values that are equal on every lane of a group in either order, so every
-// lane ends with the same bits.
+// (lane swaps).  Each step adds two values that are equal on every lane of a
+// group in either order, so every lane ends with the same bits.
 template <int R>
 __device__ __forceinline__ void wave_sums(double (&x)[R])
 {
@@ -128,20 +147,15 @@ __device__ __forceinline__ void wave_sums(double (&x)[R])
     for (int r = 0; r < R; r++) x[r] += dpp_f64<0x141>(x[r]);   // row_half_mirror
 #pragma unroll
     for (int r = 0; r < R; r++) x[r] += dpp_f64<0x140>(x[r]);   // row_mirror
-    double y[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) y[r] = __shfl_xor(x[r], 16);
+    for (int r = 0; r < R; r++) x[r] = xor16_sum(x[r]);
 #pragma unroll
-    for (int r = 0; r < R; r++) x[r] += y[r];
-#pragma unroll
-    for (int r = 0; r < R; r++) y[r] = __shfl_xor(x[r], 32);
-#pragma unroll
-    for (int r = 0; r < R; r++) x[r] += y[r];
+    for (int r = 0; r < R; r++) x[r] = xor32_sum(x[r]);
 }
 
 // Sum over each group of L consecutive lanes (L a power of two <= 64), the
 // same bits on every lane of the group: DPP steps inside rows of 16 lanes,
-// shuffles across rows.
+// lane swaps across rows.
 template <int L>
 __device__ __forceinline__ double group_sum(double x)
 {
@@ -149,8 +163,8 @@ __device__ __forceinline__ double group_sum(double x)
     if (L >= 4) x += dpp_f64<0x4E>(x);    // quad_perm [2,3,0,1]
     if (L >= 8) x += dpp_f64<0x141>(x);   // row_half_mirror
     if (L >= 16) x += dpp_f64<0x140>(x);  // row_mirror
-    if (L >= 32) x += __shfl_xor(x, 16);
-    if (L >= 64) x += __shfl_xor(x, 32);
+    if (L >= 32) x = xor16_sum(x);
+    if (L >= 64) x = xor32_sum(x);
     return x;
 }
 

@@ -74,9 +74,6 @@ __global__ __launch_bounds__(256) void k_row_pass(const TM* __restrict__ M, long
 #pragma unroll
             for (int q = 0; q < 3; q++)
                 fin.rpart[3 * blockIdx.x + q] = ((red[0][q] + red[1][q]) + red[2][q]) + red[3][q];
-            // beta_k[m-1] for the objective: the combine kernel of this
-            // iteration overwrites beta while other workgroups still decide
-            if (blockIdx.x == 0) fin.bm[0] = beta[m - 1];
         }
     }
 }
@@ -101,17 +98,26 @@ __global__ __launch_bounds__(256) void k_col_partial(
                              part + static_cast<long>(blockIdx.y) * m, nt != 0);
 }
 
-constexpr int kCombineCols = 64;   // columns per combine workgroup (4 threads each)
+// Columns per combine workgroup.  16 columns x 16 threads each: every load of
+// a partial row is one full 128-byte line, and a thread has at most 16 partials
+// of the single-read pass (one per CU), all in flight.  Latency bound: at m =
+// 4096 with 256 partials (8.4 MB) 64 columns x 4 threads, which ran on m / 64
+// workgroups, took 14.6 us (events around the kernel) and this split with the
+// stop decision off the update's path 7.0; at m = 16384 14.3 and 10.6.
+constexpr int kCombineCols = 16;
+constexpr int kCombineSubs = 256 / kCombineCols;
 
-// Stop test of the on-device BCD loop for iterate k = st.k, computed
-// identically (same data, same order) by every combine workgroup:
+// Stop test of the on-device BCD loop for iterate k = st.k, by one workgroup:
 // g_k = [r - a ; column residual of the update that produced beta_k],
 // f_k = reg sum r - (alpha_k + beta_{k,m-1})'a - (beta_k - beta_{k,m-1})'b over
-// j < m-1.  The test order is that of src/sinkhorn_bcd.cpp:65-79.
-__device__ void bcd_decide(const BcdState& st, int kk, double* f_out, double* g_out,
-                           bool* done_out, bool* stall_out)
+// j < m-1.  The test order is that of src/sinkhorn_bcd.cpp:65-79.  Records the
+// history entry and advances or stops the loop.
+__device__ void bcd_decide(const BcdState& st)
 {
+    const int kk = st.k;
     const double* cp = st.cpart + 2L * st.ntiles * (kk & 1);
+    const double bm = st.beta[st.m - 1];
+    const double* sv = st.stall + 2 * (kk & 1);
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     for (int q = threadIdx.x; q < st.nrb; q += 256) {
         v[0] += st.rpart[3 * q];
@@ -123,126 +129,156 @@ __device__ void bcd_decide(const BcdState& st, int kk, double* f_out, double* g_
         v[4] += cp[2 * q + 1];
     }
     block_sums_256<5>(v);
-    const double bm = st.bm[0];
+    if (threadIdx.x != 0) return;
     const double gnorm = sqrt(v[0] + v[3]);
     const double da = v[2] + bm * st.sum_a;
     const double db = v[4] - bm * st.sum_b1;
-    *f_out = st.reg * v[1] - da - db;
-    *g_out = gnorm;
-    *done_out = (gnorm < st.tol) || (kk >= st.max_iter);
-    *stall_out = false;
-    if (!*done_out && st.stall_window > 0) {
-        const double* sv = st.stall + 2 * (kk & 1);
-        *stall_out = !(gnorm < sv[0]) && (kk - static_cast<int>(sv[1]) >= st.stall_window);
+    const bool done = (gnorm < st.tol) || (kk >= st.max_iter);
+    bool stall = false;
+    if (st.stall_window > 0) {
+        stall = !done && !(gnorm < sv[0]) && (kk - static_cast<int>(sv[1]) >= st.stall_window);
+        // running minimum for the next iteration (other parity slot)
+        double* nx = st.stall + 2 * ((kk + 1) & 1);
+        const bool better = gnorm < sv[0];
+        nx[0] = better ? gnorm : sv[0];
+        nx[1] = better ? static_cast<double>(kk) : sv[1];
+    }
+    const int h = kk % st.hist_cap;
+    st.hist_f[h] = st.reg * v[1] - da - db;
+    st.hist_g[h] = gnorm;
+    st.hist_ts[h] = static_cast<long long>(wall_clock64());
+    if (done || stall) {
+        st.ctl[2] = kk;
+        st.ctl[0] = stall ? 2 : 1;
+    } else {
+        st.ctl[1] = kk + 1;
     }
 }
 
-// Combine the nblk partials of each column (4 threads per column, fixed
-// order), then the column epilogue.  With BCD, first take the stop decision
-// for iterate st.k; when it stops, beta is left untouched (beta_k is the
-// result), otherwise beta <- beta_{k+1} and the tile sums of the new column
-// residual go to the other parity half of cpart.  Workgroup 0 records the
-// history entry and advances or stops the loop.
+// Sum (or maximum) over the kCombineSubs threads of each column, in a fixed
+// order; the result is on every thread of the column.  x[sub][col] in LDS.
+template <bool MAX>
+__device__ __forceinline__ double combine_subs(double v, double (*x)[kCombineCols], int sub,
+                                               int col)
+{
+    x[sub][col] = v;
+    __syncthreads();
+    double y[kCombineSubs];
+#pragma unroll
+    for (int q = 0; q < kCombineSubs; q++) y[q] = x[q][col];
+#pragma unroll
+    for (int o = kCombineSubs / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < o; q++) y[q] = MAX ? fmax(y[q], y[q + o]) : y[q] + y[q + o];
+    return y[0];
+}
+
+// Combine the nblk partials of each column (16 threads per column, fixed
+// order), then the column epilogue.  With BCD (iterate st.k), the extra last
+// workgroup takes the stop decision while the others write beta_{k+1}: the
+// loop keeps beta double-buffered by parity, so the update does not wait for
+// the decision, and when the loop stops at k, beta_k is still in its buffer.
+// (Every workgroup taking the decision itself before its update put two more
+// memory round trips on the critical path.)  The tile sums of the new column
+// residual go to the other parity half of cpart.
 // SUMS: the partials are plain FP64 column sums of exp((alpha_i + colpot_j -
 // M_ij) / reg) (the single-read BCD pass), so log2 sum_i 2^((alpha_i - M_ij) k)
 // = log2(sum) - colpot_j k.
 template <bool BCD, bool SUMS>
-__global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ part, int nblk,
-                                                     int m, double k, ColEpi epi, BcdState st,
-                                                     const int* __restrict__ ctl)
+__global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ part, long pitch,
+                                                     int nblk, int m, double k, ColEpi epi,
+                                                     BcdState st, const int* __restrict__ ctl)
 {
-    int kk = 0;
-    double f = 0.0, gnorm = 0.0;
-    bool done = false, stall = false;
-    if (BCD) {
-        if (st.ctl[0] != 0) return;
-        kk = st.k;
-        bcd_decide(st, kk, &f, &gnorm, &done, &stall);
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            const int h = kk % st.hist_cap;
-            st.hist_f[h] = f;
-            st.hist_g[h] = gnorm;
-            st.hist_ts[h] = static_cast<long long>(wall_clock64());
-            if (st.stall_window > 0) {
-                // running minimum for the next iteration (other parity slot)
-                const double* sv = st.stall + 2 * (kk & 1);
-                double* nx = st.stall + 2 * ((kk + 1) & 1);
-                const bool better = gnorm < sv[0];
-                nx[0] = better ? gnorm : sv[0];
-                nx[1] = better ? static_cast<double>(kk) : sv[1];
-            }
-        }
-        done = done || stall;
-    } else if (ctl != nullptr && ctl[0] != 0) {
+    if (ctl != nullptr && ctl[0] != 0) return;
+    if (BCD && blockIdx.x == gridDim.x - 1) {
+        bcd_decide(st);
         return;
     }
-
-    const int sub = threadIdx.x & 3;
-    const int j = blockIdx.x * kCombineCols + (threadIdx.x >> 2);
-    double r2 = 0.0, bb = 0.0;
-    if (!done) {
-        double L;
-        if (SUMS) {
-            // 32 loads in flight per thread, then added in order p = sub, sub + 4, ...
-            double cs = 0.0;
-            if (j < m) {
-                int p = sub;
-                for (; p + 124 < nblk; p += 128) {
-                    double x[32];
+    __shared__ double xs[kCombineSubs][kCombineCols];
+    const int col = threadIdx.x & (kCombineCols - 1);
+    const int sub = threadIdx.x / kCombineCols;
+    const int j = blockIdx.x * kCombineCols + col;
+    const bool valid = j < m;
+    double cp = 0.0, bj = 0.0, lb = 0.0;
+    if (valid && sub == 0) {
+        if (epi.colpot) cp = epi.colpot[j];
+        if (epi.b) bj = epi.b[j];
+        if (epi.logb) lb = epi.logb[j];
+    }
+    // every thread's partials of one chunk in flight at once, added in order
+    constexpr int U = 16;
+    const double* pj = part + j;
+    double L;
+    if (SUMS) {
+        double cs = 0.0;
+        if (valid) {
+            int p = sub;
+            for (; p + (U - 1) * kCombineSubs < nblk; p += U * kCombineSubs) {
+                double x[U];
 #pragma unroll
-                    for (int u = 0; u < 32; u++) x[u] = part[static_cast<long>(p + 4 * u) * m + j];
+                for (int u = 0; u < U; u++) x[u] = pj[(p + u * kCombineSubs) * pitch];
 #pragma unroll
-                    for (int u = 0; u < 32; u++) cs += x[u];
+                for (int u = 0; u < U; u++) cs += x[u];
+            }
+            if (p < nblk) {
+                double x[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int pu = p + u * kCombineSubs;
+                    x[u] = (pu < nblk) ? pj[pu * pitch] : 0.0;
                 }
-                for (; p < nblk; p += 4) cs += part[static_cast<long>(p) * m + j];
+#pragma unroll
+                for (int u = 0; u < U; u++) cs += x[u];
             }
-            cs += __shfl_xor(cs, 1);
-            cs += __shfl_xor(cs, 2);
-            // colpot_j is read before sub 0 of the same column writes beta_out_j
-            L = (j < m && cs > 0.0) ? log2(cs) - epi.colpot[j] * k : -INFINITY;
+        }
+        cs = combine_subs<false>(cs, xs, sub, col);
+        L = cs > 0.0 ? log2(cs) - cp * k : -INFINITY;
+    } else {
+        double Lm = -INFINITY;
+        if (valid)
+            for (int p = sub; p < nblk; p += kCombineSubs) Lm = fmax(Lm, pj[p * pitch]);
+        Lm = combine_subs<true>(Lm, xs, sub, col);
+        double S = 0.0;
+        if (valid && Lm != -INFINITY)
+            for (int p = sub; p < nblk; p += kCombineSubs) {
+                const double x = pj[p * pitch];
+                S += (x == -INFINITY) ? 0.0 : exp2(x - Lm);
+            }
+        __syncthreads();
+        S = combine_subs<false>(S, xs, sub, col);
+        L = (Lm == -INFINITY) ? -INFINITY : Lm + log2(S);
+    }
+    if (sub != 0) return;
+    double r2 = 0.0, bb = 0.0;
+    if (valid) {
+        if (epi.lse2) epi.lse2[j] = L;
+        double cs = 0.0;
+        if (epi.colsum || (epi.resid && !epi.beta_out)) {
+            cs = exp2(cp * k + L);
+            if (epi.colsum) epi.colsum[j] = cs;
+        }
+        double pot = cp, g;
+        if (epi.beta_out) {
+            pot = epi.reg * (lb - kLn2 * L);
+            epi.beta_out[j] = pot;
+            g = bj * expm1(pot / epi.reg + kLn2 * L - lb);
         } else {
-            L = combine_partials(part, nblk, m, j, j < m, sub);
+            g = cs - bj;
         }
-        if (sub == 0 && j < m) {
-            if (epi.lse2) epi.lse2[j] = L;
-            double cs = 0.0;
-            if (epi.colsum || (epi.resid && !epi.beta_out)) {
-                cs = exp2(epi.colpot[j] * k + L);
-                if (epi.colsum) epi.colsum[j] = cs;
-            }
-            double bj = epi.colpot ? epi.colpot[j] : 0.0;
-            double g;
-            if (epi.beta_out) {
-                bj = epi.reg * (epi.logb[j] - kLn2 * L);
-                epi.beta_out[j] = bj;
-                g = epi.b[j] * expm1(bj / epi.reg + kLn2 * L - epi.logb[j]);
-            } else {
-                g = cs - epi.b[j];
-            }
-            if (epi.resid) epi.resid[j] = g;
-            if (j < m - 1) {
-                r2 = g * g;
-                bb = bj * epi.b[j];
-            }
-        }
-        if (epi.tilepart) {
-            double v[2] = {r2, bb};
-            block_sums_256<2>(v);
-            r2 = v[0];
-            bb = v[1];
-            if (threadIdx.x == 0) {
-                double* tp = epi.tilepart + (BCD ? 2L * gridDim.x * ((kk + 1) & 1) : 0);
-                tp[2 * blockIdx.x] = r2;
-                tp[2 * blockIdx.x + 1] = bb;
-            }
+        if (epi.resid) epi.resid[j] = g;
+        if (j < m - 1) {
+            r2 = g * g;
+            bb = pot * bj;
         }
     }
-    if (BCD && blockIdx.x == 0 && threadIdx.x == 0) {
-        if (done) {
-            st.ctl[2] = kk;
-            st.ctl[0] = stall ? 2 : 1;
-        } else {
-            st.ctl[1] = kk + 1;
+    if (epi.tilepart) {
+        // the 16 threads of sub 0 are one DPP row of wave 0
+        r2 = group_sum<kCombineCols>(r2);
+        bb = group_sum<kCombineCols>(bb);
+        if (col == 0) {
+            double* tp = epi.tilepart + (BCD ? 2L * st.ntiles * ((st.k + 1) & 1) : 0);
+            tp[2 * blockIdx.x] = r2;
+            tp[2 * blockIdx.x + 1] = bb;
         }
     }
 }
@@ -406,21 +442,22 @@ void launch_col_pass(int bulk, const void* M, long ldm, int n, int m, const doub
                            static_cast<const double*>(M), ldm, n, m, alpha, colpot_guess, logb,
                            k, rpb, part, ctl, nt);
     KERNEL_CHECK();
+    const int tiles = col_combine_blocks(m);
     if (st != nullptr)
-        hipLaunchKernelGGL((k_col_combine<true, false>), dim3(col_combine_blocks(m)), dim3(256),
-                           0, s, part, nblk, m, k, epi, *st, ctl);
+        hipLaunchKernelGGL((k_col_combine<true, false>), dim3(tiles + 1), dim3(256), 0, s, part,
+                           static_cast<long>(m), nblk, m, k, epi, *st, ctl);
     else
-        hipLaunchKernelGGL((k_col_combine<false, false>), dim3(col_combine_blocks(m)),
-                           dim3(256), 0, s, part, nblk, m, k, epi, BcdState{}, ctl);
+        hipLaunchKernelGGL((k_col_combine<false, false>), dim3(tiles), dim3(256), 0, s, part,
+                           static_cast<long>(m), nblk, m, k, epi, BcdState{}, ctl);
     KERNEL_CHECK();
 }
 
-void launch_col_combine_sums(const double* part, int nblk, int m, double k, const ColEpi& epi,
-                             const BcdState& st, hipStream_t s)
+void launch_col_combine_sums(const double* part, long pitch, int nblk, int m, double k,
+                             const ColEpi& epi, const BcdState& st, hipStream_t s)
 {
     if (epi.colpot == nullptr) fail(E_INTERNAL, "column-sum combine needs the column potential");
-    hipLaunchKernelGGL((k_col_combine<true, true>), dim3(col_combine_blocks(m)), dim3(256), 0, s,
-                       part, nblk, m, k, epi, st, st.ctl);
+    hipLaunchKernelGGL((k_col_combine<true, true>), dim3(col_combine_blocks(m) + 1), dim3(256), 0,
+                       s, part, pitch, nblk, m, k, epi, st, st.ctl);
     KERNEL_CHECK();
 }
 

@@ -295,33 +295,59 @@ void regot_problem::row_pass_bcd(const double* beta_full, const RowEpi& epi, con
 }
 
 // The single-read pass forms column sums of the plan at (alpha_{k+1}, beta_k)
-// from row-shifted FP32 terms; they keep full relative accuracy when every
-// column sum is far above the 2^-106 sum a that flushing can drop, which holds
-// when beta_k came out of an exact beta update and the marginals are bounded
-// away from zero as below (see bcd_fused.hip).
-bool regot_problem::bcd_fused_ok() const
+// from row-shifted terms; they keep full relative accuracy when every column
+// sum is far above the 2^-106 sum a that flushing can drop (FP32; far less in
+// FP64), which holds when beta_k came out of an exact beta update and the
+// marginals are bounded away from zero as below (see bcd_fused.hip).  FP64
+// arithmetic (FP64 bulk, or FP32 bulk's precise finish) has the pass of
+// bcd_rows.hip only.
+bool regot_problem::bcd_fused_ok(bool f64) const
 {
-    return bulk == REGOT_F32 && bcd_fused_shape_ok(n, m, ncu) && min_a > 0.0 && min_b > 0.0 &&
-           min_a * min_b >= 0x1p-60 * sum_a * sum_b;
+    const bool shape = bcd_rows_shape_ok(n, m, ncu) ||
+                       (!f64 && bulk == REGOT_F32 && bcd_fused_shape_ok(n, m, ncu));
+    return shape && min_a > 0.0 && min_b > 0.0 && min_a * min_b >= 0x1p-60 * sum_a * sum_b;
 }
 
-void regot_problem::bcd_fused_iteration(const double* alpha_k, double* alpha_out, double* beta_v,
-                                        const ColEpi& epi, const BcdState& st, int nblk_f,
-                                        double* fpart)
+void regot_problem::bcd_fused_iteration(const double* alpha_k, double* alpha_out,
+                                        const double* beta_k, const ColEpi& epi,
+                                        const BcdState& st, int nblk_f, double* fpart)
 {
+    const bool f64 = bulk != REGOT_F32 || bcd_precise;
+    const long pitch = bcd_part_pitch(m);
     hipEvent_t stop;
-    prof_begin(2, &stop);
-    launch_bcd_fused(dM, ldm, n, m, beta_v, k, reg, loga, a, alpha_k, alpha_out, nblk_f, fpart,
-                     st.rpart, st.bm, st.ctl, stream);
-    prof_end(2, stop);
-    prof_begin(3, &stop);
+    prof_begin(f64 ? 4 : 2, &stop);
+    if (bcd_rows_shape_ok(n, m, ncu)) {
+        BcdRowsArgs g{};
+        g.M = dM;
+        g.ldm = ldm;
+        g.n = n;
+        g.m = m;
+        g.beta = beta_k;
+        g.k = k;
+        g.reg = reg;
+        g.loga = loga;
+        g.a = a;
+        g.alpha = alpha_k;
+        g.alpha_out = alpha_out;
+        g.nblk = nblk_f;
+        g.part = fpart;
+        g.pitch = pitch;
+        g.rpart = st.rpart;
+        g.ctl = st.ctl;
+        launch_bcd_rows(bulk, bcd_precise, g, stream);
+    } else {
+        launch_bcd_fused(dM, ldm, n, m, beta_k, k, reg, loga, a, alpha_k, alpha_out, nblk_f,
+                         fpart, pitch, st.rpart, st.ctl, stream);
+    }
+    prof_end(f64 ? 4 : 2, stop);
+    prof_begin(f64 ? 5 : 3, &stop);
     ColEpi e = epi;
     e.reg = reg;
     e.logb = logb;
     e.b = b;
-    e.colpot = beta_v;
-    launch_col_combine_sums(fpart, nblk_f, m, k, e, st, stream);
-    prof_end(3, stop);
+    e.colpot = beta_k;
+    launch_col_combine_sums(fpart, pitch, nblk_f, m, k, e, st, stream);
+    prof_end(f64 ? 5 : 3, stop);
 }
 
 // One-pass FP64 objective (and gradient): the precise mode of FP32 bulk and
@@ -571,7 +597,7 @@ int regot_profile_get(regot_problem* p, int kind, long long* launches, double* t
 {
     CAPI_BEGIN
     check_handle(p);
-    if (kind < 0 || kind > 3) fail(E_INVALID, "profile kind %d", kind);
+    if (kind < 0 || kind > 5) fail(E_INVALID, "profile kind %d", kind);
     p->prof_collect();
     if (launches) *launches = p->prof_slot[kind].launches;
     if (total_ms) *total_ms = p->prof_slot[kind].total_ms;

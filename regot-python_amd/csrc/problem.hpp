@@ -80,7 +80,7 @@ void launch_log_check(const double* x, double* y, long count, hipStream_t s);
 
 // Buffers of the on-device BCD loop, kept across solves on one handle.
 struct BcdWork {
-    DBuf<double> ap0, ap1, beta, gcol, rpart, cpart, bm, stall;
+    DBuf<double> ap0, ap1, be0, be1, gcol, rpart, cpart, stall;
     DBuf<double> fpart;         // column sums of the single-read pass (blocks x m)
     DBuf<int> ctl;
     MappedRing<double> hf, hg;
@@ -161,10 +161,11 @@ struct regot_problem {
     int hess_storage = -1;
 
     // profiling of the hot passes: [0] row pass, [1] column pass (partial +
-    // combine), [2] single-read BCD pass, [3] its column-sum combine
+    // combine), [2] single-read BCD pass, [3] its column-sum combine, [4] and
+    // [5] the same two in FP64 arithmetic
     bool prof = false;
     long prof_tag = -1;         // tag of the passes being enqueued (-1: none)
-    regot::ProfileSlot prof_slot[4];
+    regot::ProfileSlot prof_slot[6];
 
     regot_problem() = default;
     regot_problem(const regot_problem&) = delete;
@@ -183,11 +184,11 @@ struct regot_problem {
     // Row pass with the BCD bookkeeping fused (see BcdState).
     void row_pass_bcd(const double* beta_full, const regot::RowEpi& epi,
                       const regot::BcdState& st);
-    // Single-read BCD iteration k (bcd_fused.hip): alpha_k -> alpha_out and the
-    // column sums into the BCD workspace, then the stop decision and beta_{k+1}
-    // (beta is both the input beta_k and the output).
-    bool bcd_fused_ok() const;
-    void bcd_fused_iteration(const double* alpha_k, double* alpha_out, double* beta,
+    // Single-read BCD iteration k: alpha_k -> alpha_out and the column sums
+    // into the BCD workspace, then the stop decision and beta_{k+1} (epi's
+    // beta_out, another buffer than beta_k).  f64: in FP64 arithmetic.
+    bool bcd_fused_ok(bool f64) const;
+    void bcd_fused_iteration(const double* alpha_k, double* alpha_out, const double* beta_k,
                              const regot::ColEpi& epi, const regot::BcdState& st, int nblk_f,
                              double* fpart);
 

@@ -37,16 +37,15 @@ void normalise_host(int n, int m, const double* alpha, const double* beta, doubl
 //                   iterate k; each workgroup writes its partials of
 //                   ||r - a||^2, sum r and alpha'a;
 //   column partial  per-tile log2 sums of column j at alpha_{k+1};
-//   column combine  every workgroup reduces the row partials and takes the
-//                   stop decision for iterate k itself (same data, same
-//                   order); unless stopping it writes beta_{k+1} and the
-//                   tile sums of the new column residual (g_{k+1}'s column
-//                   part, zero up to FP64 rounding).  Workgroup 0 records
+//   column combine  writes beta_{k+1} (double buffer) and the tile sums of
+//                   the new column residual (g_{k+1}'s column part, zero up to
+//                   FP64 rounding); one extra workgroup reduces the row
+//                   partials, takes the stop decision for iterate k, records
 //                   f_k, ||g_k|| and a timestamp and stops or advances k.
 // Once the stop flag is set every later kernel returns at once, so the host
 // keeps two batches of iterations in flight and only polls the flag.
 //
-// Single-read form (bcd_fused.hip, FP32 bulk): the row pass and the column
+// Single-read form (bcd_rows.hip, bcd_fused.hip): the row pass and the column
 // partial become one pass whose workgroups hold whole rows; the combine then
 // sums plain column sums.  It needs beta_k to come from an exact beta update,
 // so with a warm start iteration 0 keeps the two-pass form.
@@ -59,8 +58,8 @@ void normalise_host(int n, int m, const double* alpha, const double* beta, doubl
 // it also stops when ||g|| has made no new minimum for kStallWindow
 // iterations (ctl[0] = 2: an unexpected floor).  Either way the driver then
 // re-projects beta_k = optimal_beta(alpha_k) with FP64 exp and sums and
-// continues from iterate k (its history entry re-evaluated) with the
-// two-pass iteration in FP64 arithmetic over the FP32 M, to tol or max_iter,
+// continues from iterate k (its history entry re-evaluated) in FP64
+// arithmetic over the FP32 M, to tol or max_iter,
 // as the reference runs FP64 throughout after its upcast
 // (src/solvers.cpp:359-373).
 constexpr int kStallWindow = 24;
@@ -81,17 +80,17 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     const int nrb = row_pass_blocks(p->bulk, n);
     // measured faster than the two-pass form at every eligible shape tried
     // (2048^2: 1.3x, 8192^2 and 32768 x 8192: 1.8x per solve)
-    const bool fused_ok = o.bcd_fused != 0 && p->bcd_fused_ok();
-    const int nfb = fused_ok ? bcd_fused_blocks(n, p->ncu) : 0;
-    if (fused_ok) w.fpart.ensure(static_cast<size_t>(nfb) * m);
+    const bool fused_any = o.bcd_fused != 0 && p->bcd_fused_ok(false);
+    const int nfb = fused_any ? bcd_fused_blocks(n, p->ncu) : 0;
+    if (fused_any) w.fpart.ensure(static_cast<size_t>(nfb) * bcd_part_pitch(m));
     w.ap0.ensure(n);
     w.ap1.ensure(n);
-    w.beta.ensure(m);
+    w.be0.ensure(m);
+    w.be1.ensure(m);
     w.gcol.ensure(m);
     w.rpart.ensure(3L * std::max(nrb, nfb));
     w.cpart.ensure(4L * p->ntiles);
     w.ctl.ensure(4);
-    w.bm.ensure(1);
     w.stall.ensure(4);
     w.hf.ensure(cap);
     w.hg.ensure(cap);
@@ -121,12 +120,12 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
         if (o.x0) {
             HIP_CHECK(hipMemcpyAsync(p->gamma, o.x0, (n + m - 1) * sizeof(double),
                                      hipMemcpyHostToDevice, s));
-            launch_split_gamma(p->gamma, n, m, w.ap0, w.beta, s);
-            c0.colpot = w.beta;
-            p->col_pass(w.ap0, w.beta, c0);
+            launch_split_gamma(p->gamma, n, m, w.ap0, w.be0, s);
+            c0.colpot = w.be0;
+            p->col_pass(w.ap0, w.be0, c0);
         } else {
             launch_fill(w.ap0, 0.0, n, s);
-            c0.beta_out = w.beta;
+            c0.beta_out = w.be0;
             p->col_pass(w.ap0, nullptr, c0);
         }
     }
@@ -134,14 +133,12 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
 
     BcdState st{};
     st.a = p->a;
-    st.beta = w.beta;
     st.ctl = w.ctl;
     st.hist_f = w.hf.d;
     st.hist_g = w.hg.d;
     st.hist_ts = w.hts.d;
     st.hist_cap = cap;
     st.rpart = w.rpart;
-    st.bm = w.bm;
     st.cpart = w.cpart;
     st.nrb = nrb;
     st.ntiles = p->ntiles;
@@ -165,10 +162,10 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     // terms).  The events use the profiling slots; without profiling on, they
     // are dropped after the solve.
     const bool user_prof = p->prof;
-    size_t cur[4] = {0, 0, 0, 0};
+    size_t cur[6] = {0, 0, 0, 0, 0, 0};
     if (verbose >= 2) {
         p->prof = true;
-        for (int q = 0; q < 4; q++) cur[q] = p->prof_slot[q].tagged.size();
+        for (int q = 0; q < 6; q++) cur[q] = p->prof_slot[q].tagged.size();
     }
     auto pass_ms = [&](int kind, int it) {
         const auto& tg = p->prof_slot[kind].tagged;
@@ -182,7 +179,8 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
         printf("[timing]=================================================\n"
                "║ alpha = %g, beta = %g, grad = %g\n"
                "=========================================================\n\n",
-               pass_ms(0, it) + pass_ms(2, it), pass_ms(1, it) + pass_ms(3, it), 0.0);
+               pass_ms(0, it) + pass_ms(2, it) + pass_ms(4, it),
+               pass_ms(1, it) + pass_ms(3, it) + pass_ms(5, it), 0.0);
     };
 
     // Whether an FP32 loop that stopped at iterate k with status ctl[0] hands
@@ -194,7 +192,7 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     // One run of the on-device loop from iterate k0 until its stop decision;
     // returns ctl[0] (1: converged or max_iter, 2: stalled).
     auto run_loop = [&](int k0) -> int {
-        const bool fused = fused_ok && !precise;
+        const bool fused = fused_any && p->bcd_fused_ok(precise);
         FlagScope fs(p->bcd_precise, precise);
         st.stall_window = (fp32 && !precise) ? kStallWindow : 0;
         st.tol = precise ? tol : tol_fp32;
@@ -205,21 +203,25 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
         launch_fill(w.stall, static_cast<double>(k0), 4, s);
         launch_fill(w.stall.p, HUGE_VAL, 1, s);
         launch_fill(w.stall.p + 2, HUGE_VAL, 1, s);
-        // alpha_k lives in ap[k & 1]; iteration k writes alpha_{k+1} to the other
+        // alpha_k and beta_k live in the buffers of parity k & 1; iteration k
+        // writes alpha_{k+1} and beta_{k+1} to the others
         int k_enq = k0;
         auto enqueue_iteration = [&]() {
             const int kk = k_enq++;
             p->prof_tag = kk;
             double* ak = (kk & 1) ? w.ap1.p : w.ap0.p;
             double* ak1 = (kk & 1) ? w.ap0.p : w.ap1.p;
+            double* bk = (kk & 1) ? w.be1.p : w.be0.p;
+            double* bk1 = (kk & 1) ? w.be0.p : w.be1.p;
             st.k = kk;
+            st.beta = bk;
             ColEpi c;
-            c.beta_out = w.beta;
+            c.beta_out = bk1;
             c.resid = w.gcol;
             c.tilepart = w.cpart;
             if (fused && (kk > 0 || !o.x0)) {
                 st.nrb = nfb;
-                p->bcd_fused_iteration(ak, ak1, w.beta, c, st, nfb, w.fpart);
+                p->bcd_fused_iteration(ak, ak1, bk, c, st, nfb, w.fpart);
                 return;
             }
             st.nrb = nrb;
@@ -227,8 +229,8 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             e.loga = p->loga;
             e.rowpot = ak;
             e.alpha_out = ak1;
-            p->row_pass_bcd(w.beta, e, st);
-            p->col_pass(ak1, w.beta, c, w.ctl, &st);
+            p->row_pass_bcd(bk, e, st);
+            p->col_pass(ak1, bk, c, w.ctl, &st);
         };
         auto launch_batch = [&](int slot) {
             for (int it = 0; it < K && k_enq <= max_iter; it++) enqueue_iteration();
@@ -292,15 +294,16 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             if (p->prof) {
                 // the FP32 launches past iterate k0 returned at once
                 p->prof_drop_after(k0);
-                for (int q = 0; q < 4; q++)
+                for (int q = 0; q < 6; q++)
                     cur[q] = std::min(cur[q], p->prof_slot[q].tagged.size());
             }
             FlagScope fs(p->precise, true);
+            double* bk = (k0 & 1) ? w.be1.p : w.be0.p;
             ColEpi c;
-            c.beta_out = w.beta;
+            c.beta_out = bk;
             c.resid = w.gcol;
             c.tilepart = w.cpart + 2L * p->ntiles * (k0 & 1);
-            p->col_pass((k0 & 1) ? w.ap1.p : w.ap0.p, w.beta, c);
+            p->col_pass((k0 & 1) ? w.ap1.p : w.ap0.p, bk, c);
         }
     } catch (...) {
         p->prof_tag = -1;
@@ -318,7 +321,8 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
 
     HIP_CHECK(hipMemcpyAsync(ah.data(), (niter & 1) ? w.ap1.p : w.ap0.p, n * sizeof(double),
                              hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(bh.data(), w.beta.p, m * sizeof(double), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(bh.data(), (niter & 1) ? w.be1.p : w.be0.p, m * sizeof(double),
+                             hipMemcpyDeviceToHost, s));
     p->sync();
     res->niter = niter;
     res->dual.resize(n + m - 1);

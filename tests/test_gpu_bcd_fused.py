@@ -198,3 +198,87 @@ def test_fp32_bulk_finishes_below_its_resolution(gpu_lib, n, m, reg, tol, unifor
     np.testing.assert_allclose(r.obj_vals[:k], o["obj_vals"][:k], rtol=1e-8)
     np.testing.assert_allclose(r.obj_vals[pf:k], o["obj_vals"][pf:k], rtol=1e-11)
     assert rel_err(r.dual, o["dual"]) < 1e-8
+
+
+# --- several rows per step (m <= 8192, FP32 and FP64 arithmetic) ---------------
+
+def fixed_iterations(gpu_lib, M, a, b, reg, iters, bulk, fused=1):
+    """The iterates of a fixed number of iterations and the passes that ran:
+    (result, FP32 single-read passes, FP64 single-read passes)."""
+    with gpu_lib.Problem(M, a, b, reg, bulk=bulk) as P:
+        P.profile(True)
+        r = P.solve(0, tol=0.0, max_iter=iters, compute_plan=False, bcd_fused=fused)
+        return r, P.profile_stats(2)[0], P.profile_stats(4)[0]
+
+
+# FP64: one thread per 2 columns, 512 threads: NC = ceil(m / 1024); 256 threads
+# up to m = 512.  Rows per workgroup from 1 to 79 (more than one wave's lanes).
+@pytest.mark.parametrize("n,m", [(1, 1), (7, 2), (300, 80), (50, 511), (50, 512), (700, 513),
+                                 (40, 1024), (1030, 1025), (70, 2049), (260, 3073), (33, 4096),
+                                 (33, 5121), (9, 6145), (300, 7169), (5, 8192), (20000, 20),
+                                 (10, 8193)])
+def test_fp64_single_read_iterates(gpu_lib, n, m):
+    # The iterates are those of the oracle's FP64 iteration; sums run in
+    # another order: a relative 1e-15 per sum and step, 12 steps.
+    M, a, b = cloud_problem(n, m, seed=n + m)
+    reg = 0.03
+    print("fp64 single read %dx%d" % (n, m), flush=True)
+    r, _, passes = fixed_iterations(gpu_lib, M, a, b, reg, 12, "fp64")
+    assert passes == (13 if m <= 8192 else 0) and r.niter == 12
+    o = O.sinkhorn_bcd(M, a, b, reg, tol=0.0, max_iter=12)
+    assert rel_err(r.dual, o["dual"]) < 1e-12
+    np.testing.assert_allclose(r.obj_vals, o["obj_vals"], rtol=1e-11, atol=1e-15)
+    np.testing.assert_allclose(r.mar_errs, o["mar_errs"], rtol=1e-7, atol=1e-14)
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (300, 80), (1300, 1024), (40, 1025), (520, 2047),
+                                 (1025, 4096), (11, 6143), (600, 8192)])
+def test_fp32_single_read_iterates(gpu_lib, n, m):
+    # FP32 terms: 2^-24 per exponential and per product, sums of FP32 partials
+    M, a, b = cloud_problem(n, m, seed=n + m, dtype=np.float32)
+    reg = 0.05
+    print("fp32 single read %dx%d" % (n, m), flush=True)
+    tol_floor = 0.5 * 2.0 ** -22 * np.sqrt((a * a).sum() + (b * b).sum())
+    with gpu_lib.Problem(M, a, b, reg) as P:
+        P.profile(True)
+        r = P.solve(0, tol=2 * tol_floor, max_iter=5, compute_plan=False)
+        passes = P.profile_stats(2)[0]
+    o = O.sinkhorn_bcd(M.astype(np.float64), a, b, reg, tol=0.0, max_iter=r.niter)
+    assert passes == r.niter + 1
+    assert rel_err(r.dual, o["dual"]) < 1e-6
+
+
+@pytest.mark.parametrize("m", [700, 1024, 1025, 3000, 5000, 8000])
+def test_fp64_finish_runs_single_read(gpu_lib, m):
+    # an FP32 solve below its resolution: the FP64 finish reads M once per
+    # iteration too, and reaches the oracle's iterate
+    n, reg, tol = 90, 0.05, 1e-11
+    M, a, b = cloud_problem(n, m, seed=m, dtype=np.float32)
+    print("fp64 finish m=%d" % m, flush=True)
+    with gpu_lib.Problem(M, a, b, reg) as P:
+        P.profile(True)
+        r = P.solve(0, tol=tol, max_iter=2000, compute_plan=False, verify=True)
+        fine = P.profile_stats(4)[0]
+    pf = r.stats["precise_from"]
+    o = O.sinkhorn_bcd(M.astype(np.float64), a, b, reg, tol=tol, max_iter=2000)
+    assert pf >= 0 and fine == r.niter - pf + 1
+    assert r.mar_err_fp64 < 1.05 * tol and abs(r.niter - o["niter"]) <= 1
+    assert rel_err(r.dual, o["dual"]) < 1e-10
+
+
+def test_fp64_row_range_fallback(gpu_lib):
+    # at reg 1e-4 the terms span 2^-14000: rows leave [2^-400, 2^400] at first
+    n, m, reg = 70, 900, 1e-4
+    M, a, b = cloud_problem(n, m, seed=2)
+    M[0, :] = 0.0
+    M[1, :] = 1.0
+    a[0] = 1e-7
+    a /= a.sum()
+    print("fp64 range fallback", flush=True)
+    r, _, passes = fixed_iterations(gpu_lib, M, a, b, reg, 20, "fp64")
+    t, _, none = fixed_iterations(gpu_lib, M, a, b, reg, 20, "fp64", fused=0)
+    assert passes == 21 and none == 0 and np.all(np.isfinite(r.dual))
+    o = O.sinkhorn_bcd(M, a, b, reg, tol=0.0, max_iter=20)
+    # arguments of 1e4 carry 1e-12 absolute: duals to reg times that and more
+    assert rel_err(r.dual, o["dual"]) < 1e-11 and rel_err(t.dual, o["dual"]) < 1e-11
+    np.testing.assert_allclose(r.mar_errs, o["mar_errs"], rtol=1e-6, atol=1e-12)
