@@ -10,6 +10,7 @@
 
 #include "driver_work.hpp"
 #include "qrot.hpp"
+#include "sparse.hpp"
 
 namespace regot {
 
@@ -50,6 +51,37 @@ double qrot_obj_grad(regot_problem* p, const double* gamma, double* grad, double
     return w.hout.p[0];
 }
 
+namespace {
+
+// M' for the column roots of the running call (2 n m elements moved once per
+// call, against a strided read of M per Newton step); false when there is no
+// room for it.
+bool form_transpose(regot_problem* p, QrotScratch& w)
+{
+    if (w.mt_state != 0) return w.mt_state > 0;
+    const long esz = p->bulk == REGOT_F32 ? 4 : 8, al = 256 / esz;
+    w.ldt = (p->n + al - 1) / al * al;
+    try {
+        w.mt.ensure(static_cast<size_t>(p->m) * w.ldt * esz);
+    } catch (const Error&) {
+        (void)hipGetLastError();
+        w.mt_state = -1;
+        return false;
+    }
+    launch_transpose(p->bulk, p->dM, p->ldm, p->n, p->m, w.mt.p, w.ldt, p->stream);
+    w.mt_state = 1;
+    return true;
+}
+
+}  // namespace
+
+void qrot_begin_call(regot_problem* p)
+{
+    if (p->qrot) p->qrot->mt_state = 0;
+}
+
+// Roots in one read of M or its transpose (qrot_root.hip); for rows or columns
+// longer than that kernel holds, or with no room for the transpose:
 // Newton's method from the right on sum_k (x - y_k)_+ = reg w per column
 // (cols) or row: the first step takes every y (x = mean + reg w / count), each
 // later one the y below the current x, until the active set stops shrinking.
@@ -64,6 +96,14 @@ void qrot_optimal(regot_problem* p, bool cols, const double* pot, double* out)
     const int n = p->n, m = p->m;
     hipStream_t s = p->stream;
     QrotScratch& w = scratch(p);
+    if (!cols && qrot_row_root_ok(m)) {
+        launch_qrot_row_root(p->bulk, p->dM, p->ldm, n, m, pot, p->a, p->reg, out, p->ncu, s);
+        return;
+    }
+    if (cols && qrot_row_root_ok(n) && form_transpose(p, w)) {
+        launch_qrot_row_root(p->bulk, w.mt.p, w.ldt, m, n, pot, p->b, p->reg, out, p->ncu, s);
+        return;
+    }
     const int count = cols ? m : n;
     const int nbreak = cols ? n : m;
     launch_qrot_pl_init(out, w.kprev, w.done, count, w.open, s);
@@ -728,6 +768,7 @@ static void solve_qrot_semi_dual(regot_problem* p, double tol, int max_iter, int
     res->niter = lbfgs_minimize(w, tol, tol, max_iter, iterate, &xfinal);
     vec_copy(gfull, xfinal, n, s);
     qrot_optimal(p, true, gfull, gfull.p + n);
+    p->sync();
     w.report(res);
     res->dual.resize(N);
     HIP_CHECK(hipMemcpy(res->dual.data(), gfull.p, N * sizeof(double), hipMemcpyDeviceToHost));
@@ -1016,6 +1057,7 @@ int regot_qrot_solve(regot_problem* p, int solver, double tol, int max_iter, int
     res->solver = 100 + solver;
     res->n = p->n;
     res->m = p->m;
+    qrot_begin_call(p);
     solve_qrot(p, solver, tol, max_iter, verbose, o, res.get());
     *out = res.release();
     CAPI_END
@@ -1042,7 +1084,9 @@ int regot_qrot_optimal_beta(regot_problem* p, const double* alpha, double* beta)
     HIP_CHECK(hipSetDevice(p->device));
     DBuf<double> a(p->n), b(p->m);
     HIP_CHECK(hipMemcpyAsync(a.p, alpha, p->n * sizeof(double), hipMemcpyHostToDevice, p->stream));
+    qrot_begin_call(p);
     qrot_optimal(p, true, a.p, b.p);
+    p->sync();
     HIP_CHECK(hipMemcpy(beta, b.p, p->m * sizeof(double), hipMemcpyDeviceToHost));
     CAPI_END
 }
@@ -1054,7 +1098,9 @@ int regot_qrot_optimal_alpha(regot_problem* p, const double* beta, double* alpha
     HIP_CHECK(hipSetDevice(p->device));
     DBuf<double> a(p->n), b(p->m);
     HIP_CHECK(hipMemcpyAsync(b.p, beta, p->m * sizeof(double), hipMemcpyHostToDevice, p->stream));
+    qrot_begin_call(p);
     qrot_optimal(p, false, b.p, a.p);
+    p->sync();
     HIP_CHECK(hipMemcpy(alpha, a.p, p->n * sizeof(double), hipMemcpyDeviceToHost));
     CAPI_END
 }

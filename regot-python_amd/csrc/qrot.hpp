@@ -52,6 +52,12 @@ struct QrotScratch {
     HBuf<double> hout;
     HBuf<int> hopen;
     std::unique_ptr<QrotHess> hess;
+    // M transposed (m x n, pitch ldt) for the column roots: a workspace of the
+    // call that is running (mt_state 0: not formed, 1: formed, -1: no room),
+    // formed again by each call since the caller may own M
+    DBuf<unsigned char> mt;
+    long ldt = 0;
+    int mt_state = 0;
     QrotScratch(int n, int m)
     {
         const int rows = qrot_rows(n, m);
@@ -98,6 +104,13 @@ void launch_qrot_round(int bulk, const void* M, long ldm, int n, int m, const do
                        const double* beta, double reg, const double* x, const double* y,
                        const double* ea, const double* eb, const double* l1, double* P,
                        long ldp, double* scal, hipStream_t s);
+// Roots of every row in one read of M (m <= 16384, qrot_root.hip):
+// out_i = the x with sum_j (x - (M_ij - pot_j))_+ = reg w_i.
+bool qrot_row_root_ok(int m);
+void launch_qrot_row_root(int bulk, const void* M, long ldm, int n, int m, const double* pot,
+                          const double* w, double reg, double* out, int ncu, hipStream_t s);
+// The same roots by Newton passes over M (wider matrices, or no room for the
+// transpose):
 void launch_qrot_pl_init(double* xc, int* kprev, int* done, int count, int* open, hipStream_t s);
 // One Newton step of the per-column (cols) or per-row roots; *open counts the
 // entries still moving.
@@ -162,6 +175,8 @@ void apply_qrot_hess(regot_problem* p, QrotHess& H, const double* x, double tau,
 // gamma (n + m), src/qrot_problem.cpp:226-258.
 double qrot_obj_grad(regot_problem* p, const double* gamma, double* grad, double tau,
                      double* gnorm2);
+// Forget the transpose of the last call (its M may have changed since).
+void qrot_begin_call(regot_problem* p);
 // optimal_beta (cols = true: out = beta (m) given alpha = pot) or
 // optimal_alpha (cols = false: out = alpha (n) given beta = pot), device.
 void qrot_optimal(regot_problem* p, bool cols, const double* pot, double* out);

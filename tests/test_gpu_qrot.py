@@ -300,3 +300,66 @@ def test_qrot_pdaam(gpu_lib):
     full = np.sqrt(((P.sum(1) - a) ** 2).sum() + ((P.sum(0) - b) ** 2).sum())
     assert full <= tol and abs(full - r.mar_errs[-1]) < 1e-12
     np.testing.assert_allclose(P, o["plan"], rtol=1e-5, atol=1e-8)
+
+
+# --- roots in one read of M (rows and columns up to 16384 entries) --------------
+
+def roots_oracle(Z, c):
+    """x_i with sum_j (x_i - Z_ij)_+ = c_i by sorting, FP64."""
+    S = np.sort(Z, axis=1)
+    k = np.arange(1, S.shape[1] + 1)
+    cand = (np.cumsum(S, axis=1) + c[:, None]) / k
+    last = (cand > S).sum(1) - 1
+    return np.take_along_axis(cand, np.maximum(last, 0)[:, None], 1)[:, 0]
+
+
+# threads per row double at 1024, 2048, 4096, 8192 entries; more than 16384
+# takes the Newton passes; reg from a lone active entry to all of them
+@pytest.mark.parametrize("n,m", [(1, 1), (3, 1024), (5, 1025), (40, 2049), (2049, 33), (7, 4097),
+                                 (3000, 17), (4, 8193), (3, 16384), (16384, 2), (2, 16385)])
+@pytest.mark.parametrize("reg", [1e-6, 0.05, 1e4])
+@pytest.mark.parametrize("bulk", ["fp32", "fp64"])
+def test_qrot_roots_all_lengths(gpu_lib, n, m, reg, bulk):
+    M, a, b = cloud_problem(n, m, d=4, seed=n + m, dtype=np.float32)
+    M64 = M.astype(np.float64)
+    rng = np.random.default_rng(n)
+    alpha, beta = rng.uniform(-0.1, 0.1, n), rng.uniform(-0.1, 0.1, m)
+    print("qrot roots %dx%d reg %g %s" % (n, m, reg, bulk), flush=True)
+    with gpu_lib.Problem(M, a, b, reg, bulk=bulk) as P:
+        got_b = P.qrot_optimal_beta(alpha)
+        got_a = P.qrot_optimal_alpha(beta)
+    # sums of up to 16384 entries below 1e4 in another order
+    for got, ref in ((got_b, roots_oracle(M64.T - alpha, reg * b)),
+                     (got_a, roots_oracle(M64 - beta, reg * a))):
+        np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-13)
+
+
+def test_qrot_roots_ties_infinities_and_updates(gpu_lib):
+    # equal entries, a zero marginal, infinite costs, and a cost matrix that its
+    # owner changes between calls
+    import torch
+    n, m, reg = 300, 700, 0.3
+    rng = np.random.default_rng(5)
+    M = rng.integers(0, 4, size=(n, m)).astype(np.float32)
+    M[:, 0] = np.inf
+    M[0, 1:] = np.inf
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    a[1] = 0.0
+    dM = torch.from_numpy(M).to("cuda:0")
+    torch.cuda.synchronize()
+    with gpu_lib.Problem.from_device(dM.data_ptr(), n, m, np.float32, a, b, reg) as P:
+        beta, alpha = np.zeros(m), np.zeros(n)
+        x = P.qrot_optimal_alpha(beta)
+        with np.errstate(invalid="ignore"):
+            ref = roots_oracle(M[1:].astype(np.float64), reg * a[1:])
+        assert x[0] == np.inf and x[1] == 0.0
+        np.testing.assert_allclose(x[1:], ref, rtol=1e-12, atol=1e-14)
+        y = P.qrot_optimal_beta(alpha)
+        assert y[0] == np.inf
+        np.testing.assert_allclose(y[1:], roots_oracle(M[1:, 1:].T.astype(np.float64),
+                                                       reg * b[1:]), rtol=1e-12, atol=1e-14)
+        M2 = rng.uniform(0, 1, size=(n, m)).astype(np.float32)
+        dM.copy_(torch.from_numpy(M2))
+        torch.cuda.synchronize()
+        y = P.qrot_optimal_beta(alpha)
+        np.testing.assert_allclose(y, roots_oracle(M2.T.astype(np.float64), reg * b), rtol=1e-12)
