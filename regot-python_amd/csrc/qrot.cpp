@@ -26,31 +26,6 @@ QrotScratch& scratch(regot_problem* p)
 
 }  // namespace
 
-double qrot_obj_grad(regot_problem* p, const double* gamma, double* grad, double tau,
-                     double* gnorm2)
-{
-    const int n = p->n, m = p->m;
-    hipStream_t s = p->stream;
-    QrotScratch& w = scratch(p);
-    const int rows = qrot_rows(n, m);
-    const int nstrip = ceil_div(m, 256), nblk = ceil_div(n, rows);
-    const double* alpha = gamma;
-    const double* beta = gamma + n;
-    launch_qrot_tile(p->bulk, p->dM, p->ldm, n, m, alpha, beta, 1.0, nullptr, nullptr,
-                     grad ? w.rowpart.p : nullptr, grad ? w.colpart.p : nullptr, w.sqpart, s);
-    if (grad) {
-        launch_qrot_fold(w.rowpart, nstrip, n, n, w.rsum, s);
-        launch_qrot_fold(w.colpart, nblk, m, m, w.csum, s);
-    }
-    launch_qrot_sum1(w.sqpart, nstrip * nblk, w.sq, s);
-    launch_qrot_finish(alpha, beta, p->a, p->b, n, m, p->reg, tau, w.sq, w.rsum, w.csum, grad,
-                       w.fpart, w.gpart, w.out, s);
-    HIP_CHECK(hipMemcpyAsync(w.hout.p, w.out.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    if (gnorm2) *gnorm2 = w.hout.p[1];
-    return w.hout.p[0];
-}
-
 namespace {
 
 // M' for the column roots of the running call (2 n m elements moved once per
@@ -106,6 +81,12 @@ void qrot_optimal(regot_problem* p, bool cols, const double* pot, double* out)
     }
     const int count = cols ? m : n;
     const int nbreak = cols ? n : m;
+    {
+        const size_t rows = qrot_rows(n, m);
+        const size_t a = (n + rows - 1) / rows * m, b = static_cast<size_t>(ceil_div(m, 256)) * n;
+        w.spart.ensure(a > b ? a : b);
+        w.kpart.ensure(a > b ? a : b);
+    }
     launch_qrot_pl_init(out, w.kprev, w.done, count, w.open, s);
     const double* wt = cols ? p->b.p : p->a.p;
     for (int step = 0; step <= nbreak + 1; step++) {
@@ -335,7 +316,8 @@ static void solve_qrot_grssn(regot_problem* p, double tol, int max_iter, int ver
     Timer timer;
     timer.tic();
     auto record = [&](const double* x, double f, double gnorm) {
-        const double prim = qrot_round_plan(p, x, x + n, nullptr, 0);
+        // recorded right after the gradient at x
+        const double prim = qrot_primal(p, x, x + n, true);
         const double dur = timer.toc();
         res->obj_vals.push_back(f);
         res->prim_vals.push_back(prim);
@@ -407,7 +389,8 @@ static void solve_qrot_assn(regot_problem* p, double tol, int max_iter, int verb
     Timer timer;
     timer.tic();
     auto record = [&](const double* x, double f, double gnorm) {
-        const double prim = qrot_round_plan(p, x, x + n, nullptr, 0);
+        // recorded right after the gradient at x
+        const double prim = qrot_primal(p, x, x + n, true);
         const double dur = timer.toc();
         res->obj_vals.push_back(f);
         res->prim_vals.push_back(prim);
@@ -504,7 +487,7 @@ static void solve_qrot_s5n(regot_problem* p, double tol, int max_iter, int verbo
     Timer timer;
     timer.tic();
     auto record = [&](const double* x, double f, double gnorm) {
-        const double prim = qrot_round_plan(p, x, x + n, nullptr, 0);
+        const double prim = qrot_primal(p, x, x + n, false);
         const double dur = timer.toc();
         res->obj_vals.push_back(f);
         res->prim_vals.push_back(prim);
@@ -652,7 +635,7 @@ static void solve_qrot_pdaam(regot_problem* p, double tol, int max_iter, int ver
     double f = w.obj_grad(gamma, grad, &gnorm);
     double dur = timer.toc();
     res->obj_vals.push_back(f);
-    res->prim_vals.push_back(qrot_round_plan(p, gamma, gamma + n, nullptr, 0));
+    res->prim_vals.push_back(qrot_primal(p, gamma, gamma + n, false));
     res->mar_errs.push_back(gnorm / reg);
     res->run_times.push_back(dur);
     double L = 1.0, palpha = 0.0;
@@ -695,7 +678,7 @@ static void solve_qrot_pdaam(regot_problem* p, double tol, int max_iter, int ver
         const double mar_err = std::sqrt(hp.p[2]);
         dur = timer.toc();
         res->obj_vals.push_back(f);
-        res->prim_vals.push_back(qrot_round_plan(p, gamma, gamma + n, nullptr, 0));
+        res->prim_vals.push_back(qrot_primal(p, gamma, gamma + n, false));
         res->mar_errs.push_back(mar_err);
         res->run_times.push_back(res->run_times.back() + dur);
         if (verbose >= 1) {
@@ -752,7 +735,7 @@ static void solve_qrot_semi_dual(regot_problem* p, double tol, int max_iter, int
         const double dur = timer.toc();
         vec_copy(gpr, x, n, s);
         qrot_optimal(p, true, gpr, gpr.p + n);
-        const double prim = qrot_round_plan(p, gpr, gpr.p + n, nullptr, 0);
+        const double prim = qrot_primal(p, gpr, gpr.p + n, false);
         res->obj_vals.push_back(last_f);
         res->prim_vals.push_back(prim);
         res->mar_errs.push_back(gnorm / reg);
@@ -838,7 +821,7 @@ static void solve_qrot_apdagd(regot_problem* p, double tol, int max_iter, int ve
     double f = w.obj_grad(gamma, grad, &gnorm);
     double dur = timer.toc();
     res->obj_vals.push_back(f);
-    res->prim_vals.push_back(qrot_round_plan(p, gamma, gamma + n, nullptr, 0));
+    res->prim_vals.push_back(qrot_primal(p, gamma, gamma + n, false));
     res->mar_errs.push_back(gnorm / reg);
     res->run_times.push_back(dur);
     double L = 1.0, pbeta = 0.0;
@@ -880,7 +863,7 @@ static void solve_qrot_apdagd(regot_problem* p, double tol, int max_iter, int ve
         const double mar_err = std::sqrt(hp.p[2]);
         dur = timer.toc();
         res->obj_vals.push_back(f);
-        res->prim_vals.push_back(qrot_round_plan(p, gamma, gamma + n, nullptr, 0));
+        res->prim_vals.push_back(qrot_primal(p, gamma, gamma + n, false));
         res->mar_errs.push_back(mar_err);
         res->run_times.push_back(res->run_times.back() + dur);
         if (verbose >= 1) {
@@ -942,7 +925,8 @@ void solve_qrot(regot_problem* p, int solver, double tol, int max_iter, int verb
     Timer timer;
     timer.tic();
     auto record = [&](const double* x, double f, double gnorm) {
-        const double prim = qrot_round_plan(p, x, x + n, nullptr, 0);
+        // recorded right after the gradient at x (L-BFGS: after a line search)
+        const double prim = qrot_primal(p, x, x + n, solver != 2);
         const double dur = timer.toc();
         res->obj_vals.push_back(f);
         res->prim_vals.push_back(prim);
@@ -1113,7 +1097,7 @@ int regot_qrot_primal_val(regot_problem* p, const double* gamma, double* value)
     const long N = static_cast<long>(p->n) + p->m;
     DBuf<double> g(N);
     HIP_CHECK(hipMemcpyAsync(g.p, gamma, N * sizeof(double), hipMemcpyHostToDevice, p->stream));
-    *value = qrot_round_plan(p, g.p, g.p + p->n, nullptr, 0);
+    *value = qrot_primal(p, g.p, g.p + p->n, false);
     CAPI_END
 }
 

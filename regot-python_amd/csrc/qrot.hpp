@@ -11,6 +11,9 @@
 namespace regot {
 
 int qrot_rows(int n, int m);
+// scratch of the sweeps (qrot_sweep.hip), in doubles
+void qrot_sweep_sizes(int n, int m, size_t* rowpart, size_t* colpart, size_t* scal);
+bool qrot_row_root_ok(int m);
 
 // The generalised Hessian H = [diag(h1) sigma; sigma' diag(h2)] at one gamma
 // (src/qrot_hess.h:11-36): sigma as a bitmask (launch_qrot_mask), h1 = sigma 1,
@@ -45,9 +48,10 @@ struct QrotHess {
 // Device scratch of the QROT passes and root iterations, sized for a shape;
 // owned by the problem handle.
 struct QrotScratch {
-    DBuf<double> rowpart, colpart, sqpart, rsum, csum, sq, out, spart, fpart, gpart;
-    // rounding (qrot_round_plan): row / column scales, errors, |err_a|_1, totals
-    DBuf<double> x, y, ea, eb, l1part, l1, scal, tot;
+    DBuf<double> rowpart, colpart, sqpart, rsum, csum, out, spart, fpart, gpart;
+    // rounding (qrot_primal): row / column scales, column errors, totals
+    DBuf<double> x, y, eb, scal, tot;
+    DBuf<double> epart, cpart;   // per-workgroup sums of the folds
     DBuf<int> kpart, kprev, done, open;
     HBuf<double> hout;
     HBuf<int> hopen;
@@ -62,16 +66,16 @@ struct QrotScratch {
     {
         const int rows = qrot_rows(n, m);
         const long nstrip = ceil_div(m, 256), nblk = ceil_div(n, rows);
-        rowpart.alloc(static_cast<size_t>(nstrip) * n);
-        colpart.alloc(static_cast<size_t>(nblk) * m);
-        sqpart.alloc(static_cast<size_t>(nstrip) * nblk);
-        const size_t a = static_cast<size_t>(nblk) * m, b = static_cast<size_t>(nstrip) * n;
-        spart.alloc(a > b ? a : b);
-        kpart.alloc(a > b ? a : b);
+        // shared by the 256-column tiles and the sweeps
+        size_t srow, scol, sscal;
+        qrot_sweep_sizes(n, m, &srow, &scol, &sscal);
+        const size_t trow = static_cast<size_t>(nstrip) * n, tcol = static_cast<size_t>(nblk) * m;
+        rowpart.alloc(trow > srow ? trow : srow);
+        colpart.alloc(tcol > scol ? tcol : scol);
+        sqpart.alloc(sscal);
         rsum.alloc(n);
         csum.alloc(m);
-        sq.alloc(1);
-        out.alloc(2);
+        out.alloc(3);
         const int nw = ceil_div(n > m ? n : m, 256);
         fpart.alloc(4 * static_cast<size_t>(nw));
         gpart.alloc(nw);
@@ -83,30 +87,15 @@ struct QrotScratch {
         hopen.ensure(1);
         x.alloc(n);
         y.alloc(m);
-        ea.alloc(n);
         eb.alloc(m);
-        l1part.alloc(ceil_div(n, 256));
-        l1.alloc(1);
-        scal.alloc(2 * static_cast<size_t>(nstrip) * nblk);
+        scal.alloc(sscal);
         tot.alloc(2);
+        epart.alloc(4 * static_cast<size_t>(ceil_div(static_cast<long>(n) + m, 64)));
+        cpart.alloc(ceil_div(m, 64));
     }
 };
-// Row sums (per 256-column strip: rowpart[strip * n + i]), column sums (per
-// row block: colpart[blk * m + j]) and sums of squares (sqpart[blk * strips +
-// strip]) of ((D / div) x_i) y_j, D = (alpha_i + beta_j - M_ij)_+; x, y and
-// any output may be null.
-void launch_qrot_tile(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
-                      const double* beta, double div, const double* x, const double* y,
-                      double* rowpart, double* colpart, double* sqpart, hipStream_t s);
-// P_ij = ((D_ij / reg) x_i) y_j + ea_i eb_j / l1; scal[2 wg] = sum P M,
-// scal[2 wg + 1] = sum P^2 per workgroup; P written when non-null.
-void launch_qrot_round(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
-                       const double* beta, double reg, const double* x, const double* y,
-                       const double* ea, const double* eb, const double* l1, double* P,
-                       long ldp, double* scal, hipStream_t s);
 // Roots of every row in one read of M (m <= 16384, qrot_root.hip):
 // out_i = the x with sum_j (x - (M_ij - pot_j))_+ = reg w_i.
-bool qrot_row_root_ok(int m);
 void launch_qrot_row_root(int bulk, const void* M, long ldm, int n, int m, const double* pot,
                           const double* w, double reg, double* out, int ncu, hipStream_t s);
 // The same roots by Newton passes over M (wider matrices, or no room for the
@@ -146,8 +135,8 @@ void launch_qrot_mask(int bulk, const void* M, long ldm, int n, int m, const dou
                       const double* beta, unsigned long long* mask, hipStream_t s);
 // Row sums of sigma_ij y_j (rows_out) into rowpart[(strip * 4 + k) * n + i]
 // (4 partials per 256-column strip: fold 4 ceil(m / 256) of them) and column
-// sums of sigma_ij x_i (cols_out) into colpart as launch_qrot_tile; null x or
-// y count ones.
+// sums of sigma_ij x_i (cols_out) per block of qrot_rows rows into
+// colpart[blk * m + j]; null x or y count ones.
 void launch_qrot_sig(const unsigned long long* mask, int n, int m, bool rows_out, bool cols_out,
                      const double* x, const double* y, double* rowpart, double* colpart,
                      hipStream_t s);
@@ -182,9 +171,9 @@ void qrot_begin_call(regot_problem* p);
 void qrot_optimal(regot_problem* p, bool cols, const double* pot, double* out);
 
 // <P, M> + reg/2 ||P||^2 of P = approx_proj((alpha (+) beta - M)_+ / reg)
-// for device alpha (n), beta (m); P (device, pitch ldp) written when non-null.
-double qrot_round_plan(regot_problem* p, const double* alpha, const double* beta, double* P,
-                       long ldp);
+// for device alpha (n), beta (m).  fresh: the last sweep on this handle was
+// qrot_obj_grad with a gradient at this very point, whose row scales are taken.
+double qrot_primal(regot_problem* p, const double* alpha, const double* beta, bool fresh);
 // The QROT plan (alpha (+) beta - M)+ / reg of a host dual (n + m) into host memory.
 void qrot_plan_host(regot_problem* p, const double* dual, double* plan);
 

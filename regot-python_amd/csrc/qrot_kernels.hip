@@ -2,14 +2,11 @@
 // (QROT) dual over the cost matrix M (FP32 or FP64 storage, FP64 arithmetic).
 //
 // With D_ij = (alpha_i + beta_j - M_ij)_+ (src/qrot_problem.cpp:37-96):
-//   k_qrot_tile       row sums, column sums and sum of squares of
-//                     W_ij = ((D_ij / div) x_i) y_j (x, y optional weights;
-//                     div = 1 for the dual, reg for the plan D / reg);
-//   k_qrot_round_tile the rounded plan P_ij = W_ij + ea_i eb_j / l1 of
-//                     approx_proj (src/approx_proj.h:6-26) with <P, M> and
-//                     ||P||^2, P optionally written;
+//   (the objective, its gradient and the rounding: qrot_sweep.hip; the roots
+//   of rows that fit a workgroup: qrot_root.hip)
 //   k_qrot_pl_tile    one Newton step of the piecewise-linear roots behind
-//                     optimal_beta / optimal_alpha (src/qrot_problem.cpp:365-418):
+//                     optimal_beta / optimal_alpha (src/qrot_problem.cpp:365-418)
+//                     of longer rows:
 //                     per column (or row) the sum and count of y = M_ij - alpha_i
 //                     (or M_ij - beta_j) below the current iterate;
 //   k_qrot_pl_update  the step x <- (c + S) / K per column or row.
@@ -85,128 +82,6 @@ __device__ __forceinline__ void load4(const double* row, int c0, int m, double* 
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) v[q] = (c0 + q < m) ? row[c0 + q] : 0.0;
-}
-
-// DIV: divide D by div (the plan D / reg of the rounding passes, in the
-// reference's order of operations); without it div is 1 and skipped.
-template <typename TM, bool WT, bool DIV>
-__global__ __launch_bounds__(256) void k_qrot_tile(const TM* __restrict__ M, long ldm, int n,
-                                                   int m, const double* __restrict__ alpha,
-                                                   const double* __restrict__ beta, double div,
-                                                   const double* __restrict__ x,
-                                                   const double* __restrict__ y, int rows,
-                                                   double* __restrict__ rowpart,
-                                                   double* __restrict__ colpart,
-                                                   double* __restrict__ sqpart)
-{
-    __shared__ double red[4][257];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int strip = blockIdx.x, blk = blockIdx.y;
-    const int c0 = strip * 256 + lane * 4;
-    const int r0 = blk * rows;
-    const int r1 = min(n, r0 + rows);
-    double bq[4], yq[4], cs[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        bq[q] = (c0 + q < m) ? beta[c0 + q] : 0.0;
-        yq[q] = (WT && y != nullptr && c0 + q < m) ? y[c0 + q] : 1.0;
-    }
-    double sq = 0.0;
-    for (int r = r0 + wave; r < r1; r += 4) {
-        const double ai = alpha[r];
-        const double xi = (WT && x != nullptr) ? x[r] : 1.0;
-        double mv[4];
-        load4(M + static_cast<long>(r) * ldm, c0, m, mv);
-        double rs = 0.0;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            if (c0 + q < m) {
-                const double c = (ai + bq[q]) - mv[q];
-                double d = c > 0.0 ? c : 0.0;
-                if (DIV) d = d / div;
-                if (WT) {
-                    if (x != nullptr) d = d * xi;
-                    if (y != nullptr) d = d * yq[q];
-                }
-                rs += d;
-                cs[q] += d;
-                sq += d * d;
-            }
-        }
-        rs = wsum64(rs);
-        if (lane == 0 && rowpart) rowpart[static_cast<long>(strip) * n + r] = rs;
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q++) red[wave][lane * 4 + q] = cs[q];
-    sq = wsum64(sq);
-    if (lane == 0) red[wave][256] = sq;
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int j = c0 + q;
-            const double v = ((red[0][lane * 4 + q] + red[1][lane * 4 + q]) +
-                              red[2][lane * 4 + q]) + red[3][lane * 4 + q];
-            if (j < m && colpart) colpart[static_cast<long>(blk) * m + j] = v;
-        }
-        if (lane == 0 && sqpart)
-            sqpart[static_cast<long>(blk) * gridDim.x + strip] =
-                ((red[0][256] + red[1][256]) + red[2][256]) + red[3][256];
-    }
-}
-
-template <typename TM>
-__global__ __launch_bounds__(256) void k_qrot_round_tile(
-    const TM* __restrict__ M, long ldm, int n, int m, const double* __restrict__ alpha,
-    const double* __restrict__ beta, double reg, const double* __restrict__ x,
-    const double* __restrict__ y, const double* __restrict__ ea, const double* __restrict__ eb,
-    const double* __restrict__ l1p, int rows, double* __restrict__ P, long ldp,
-    double* __restrict__ scal)
-{
-    __shared__ double ss[2][4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int strip = blockIdx.x, blk = blockIdx.y;
-    const int c0 = strip * 256 + lane * 4;
-    const int r0 = blk * rows;
-    const int r1 = min(n, r0 + rows);
-    const double l1 = *l1p;
-    double bq[4], yq[4], eq[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const bool in = c0 + q < m;
-        bq[q] = in ? beta[c0 + q] : 0.0;
-        yq[q] = in ? y[c0 + q] : 0.0;
-        eq[q] = in ? eb[c0 + q] : 0.0;
-    }
-    double mp = 0.0, sq = 0.0;
-    for (int r = r0 + wave; r < r1; r += 4) {
-        const double ai = alpha[r], xi = x[r], ei = ea[r];
-        double mv[4];
-        load4(M + static_cast<long>(r) * ldm, c0, m, mv);
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int j = c0 + q;
-            if (j < m) {
-                const double c = (ai + bq[q]) - mv[q];
-                const double v = (((c > 0.0 ? c : 0.0) / reg) * xi) * yq[q] + ei * eq[q] / l1;
-                if (P) P[static_cast<long>(r) * ldp + j] = v;
-                mp += v * mv[q];
-                sq += v * v;
-            }
-        }
-    }
-    mp = wsum64(mp);
-    sq = wsum64(sq);
-    if (lane == 0) {
-        ss[0][wave] = mp;
-        ss[1][wave] = sq;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const long wg = static_cast<long>(blk) * gridDim.x + strip;
-        scal[2 * wg] = ((ss[0][0] + ss[0][1]) + ss[0][2]) + ss[0][3];
-        scal[2 * wg + 1] = ((ss[1][0] + ss[1][1]) + ss[1][2]) + ss[1][3];
-    }
 }
 
 // COLS: per column j, y_i = M_ij - pot_i over the block's rows; else per row
@@ -708,56 +583,6 @@ int qrot_rows(int n, int m)
     int rows = 16;
     while (rows < 256 && static_cast<long>(strips) * ceil_div(n, rows * 2) >= 1024) rows *= 2;
     return rows;
-}
-
-template <typename TM>
-void qrot_tile_launch(dim3 grid, int rows, hipStream_t s, const TM* M, long ldm, int n, int m,
-                      const double* alpha, const double* beta, double div, const double* x,
-                      const double* y, double* rowpart, double* colpart, double* sqpart)
-{
-    const bool wt = x != nullptr || y != nullptr;
-    if (wt)
-        hipLaunchKernelGGL((k_qrot_tile<TM, true, true>), grid, dim3(256), 0, s, M, ldm, n, m,
-                           alpha, beta, div, x, y, rows, rowpart, colpart, sqpart);
-    else if (div != 1.0)
-        hipLaunchKernelGGL((k_qrot_tile<TM, false, true>), grid, dim3(256), 0, s, M, ldm, n, m,
-                           alpha, beta, div, x, y, rows, rowpart, colpart, sqpart);
-    else
-        hipLaunchKernelGGL((k_qrot_tile<TM, false, false>), grid, dim3(256), 0, s, M, ldm, n, m,
-                           alpha, beta, div, x, y, rows, rowpart, colpart, sqpart);
-    KERNEL_CHECK();
-}
-
-void launch_qrot_tile(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
-                      const double* beta, double div, const double* x, const double* y,
-                      double* rowpart, double* colpart, double* sqpart, hipStream_t s)
-{
-    const int rows = qrot_rows(n, m);
-    const dim3 grid(ceil_div(m, 256), ceil_div(n, rows));
-    if (bulk == 0)
-        qrot_tile_launch(grid, rows, s, static_cast<const float*>(M), ldm, n, m, alpha, beta, div,
-                         x, y, rowpart, colpart, sqpart);
-    else
-        qrot_tile_launch(grid, rows, s, static_cast<const double*>(M), ldm, n, m, alpha, beta,
-                         div, x, y, rowpart, colpart, sqpart);
-}
-
-void launch_qrot_round(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
-                       const double* beta, double reg, const double* x, const double* y,
-                       const double* ea, const double* eb, const double* l1, double* P,
-                       long ldp, double* scal, hipStream_t s)
-{
-    const int rows = qrot_rows(n, m);
-    const dim3 grid(ceil_div(m, 256), ceil_div(n, rows));
-    if (bulk == 0)
-        hipLaunchKernelGGL(k_qrot_round_tile<float>, grid, dim3(256), 0, s,
-                           static_cast<const float*>(M), ldm, n, m, alpha, beta, reg, x, y, ea,
-                           eb, l1, rows, P, ldp, scal);
-    else
-        hipLaunchKernelGGL(k_qrot_round_tile<double>, grid, dim3(256), 0, s,
-                           static_cast<const double*>(M), ldm, n, m, alpha, beta, reg, x, y, ea,
-                           eb, l1, rows, P, ldp, scal);
-    KERNEL_CHECK();
 }
 
 void launch_qrot_pl_init(double* xc, int* kprev, int* done, int count, int* open, hipStream_t s)

@@ -363,3 +363,68 @@ def test_qrot_roots_ties_infinities_and_updates(gpu_lib):
         torch.cuda.synchronize()
         y = P.qrot_optimal_beta(alpha)
         np.testing.assert_allclose(y, roots_oracle(M2.T.astype(np.float64), reg * b), rtol=1e-12)
+
+
+# --- the sweeps of the objective and the rounding -------------------------------
+
+def rounded_primal(M, a, b, reg, alpha, beta):
+    """<P, M> + reg/2 ||P||^2 of approx_proj of the plan, element by element."""
+    T = np.maximum(alpha[:, None] + beta[None, :] - M, 0.0) / reg
+    T *= np.minimum(a / T.sum(1), 1.0)[:, None]
+    T *= np.minimum(b / T.sum(0), 1.0)[None, :]
+    ea, eb = a - T.sum(1), b - T.sum(0)
+    P = T + ea[:, None] * eb[None, :] / np.abs(ea).sum()
+    return (P * M).sum() + 0.5 * reg * (P * P).sum()
+
+
+# strips of 256, 512 and 1024 columns begin at m = 1, 320 and 1536; blocks of 16
+# rows, 4 per wave, and their remainders
+@pytest.mark.parametrize("n,m", [(1, 1), (3, 2), (17, 319), (33, 320), (130, 513), (19, 1535),
+                                 (5, 1536), (71, 2051), (2100, 259)])
+@pytest.mark.parametrize("bulk", ["fp32", "fp64"])
+def test_qrot_sweeps_edges(gpu_lib, n, m, bulk):
+    M, a, b = cloud_problem(n, m, d=4, seed=n + m, dtype=np.float32)
+    M64 = M.astype(np.float64)
+    reg = 0.1
+    rng = np.random.default_rng(n * m)
+    alpha, beta = rng.uniform(0.1, 0.4, n), rng.uniform(0.1, 0.4, m)
+    D = np.maximum(alpha[:, None] + beta[None, :] - M64, 0.0)
+    g0 = np.concatenate([D.sum(1) - reg * a, D.sum(0) - reg * b])
+    f0 = 0.5 * (D * D).sum() - reg * (alpha @ a + beta @ b)
+    print("qrot sweeps %dx%d %s" % (n, m, bulk), flush=True)
+    with gpu_lib.Problem(M, a, b, reg, bulk=bulk) as P:
+        gamma = np.concatenate([alpha, beta])
+        f, g = P.qrot_obj_grad(gamma)
+        ft, gt = P.qrot_obj_grad(gamma, tau=0.7)
+        prim = P.qrot_primal_val(gamma)
+        r = P.qrot_solve(0, tol=0.0, max_iter=2, compute_plan=False)
+    # sums of up to 2100 nonnegative terms: 1e-13 relative of their size
+    scale = max(1.0, D.sum(1).max(), D.sum(0).max())
+    assert abs(f - f0) < 1e-13 * max(1.0, abs(f0))
+    assert np.max(np.abs(g - g0)) < 1e-13 * scale
+    d = alpha.sum() - beta.sum()
+    assert abs(ft - (f0 + 0.35 * d * d)) < 1e-12 * max(1.0, abs(ft))
+    t = 0.7 * d * np.concatenate([np.ones(n), -np.ones(m)])
+    assert np.max(np.abs(gt - (g0 + t))) < 1e-12 * max(scale, abs(d))
+    ref = rounded_primal(M64, a, b, reg, alpha, beta)
+    assert abs(prim - ref) < 1e-11 * abs(ref)
+    # the driver's primal values take the row scales of the objective's sweep
+    ref = rounded_primal(M64, a, b, reg, r.dual[:n], r.dual[n:])
+    if np.isfinite(ref):
+        assert abs(r.prim_vals[-1] - ref) < 1e-10 * abs(ref)
+
+
+def test_qrot_primal_infinite_costs(gpu_lib):
+    # an infinite cost forbids its entry: D = 0 there, and the rounding's rank-one
+    # term puts mass on it, as it does element by element
+    n, m, reg = 40, 330, 0.1
+    M, a, b = cloud_problem(n, m, d=4, seed=1)
+    M[3, 5] = np.inf
+    alpha, beta = np.full(n, 0.3), np.full(m, 0.3)
+    with gpu_lib.Problem(M, a, b, reg) as P:
+        f, g = P.qrot_obj_grad(np.concatenate([alpha, beta]))
+        prim = P.qrot_primal_val(np.concatenate([alpha, beta]))
+    D = np.maximum(0.6 - M, 0.0)
+    f0 = 0.5 * (D * D).sum() - reg * (alpha @ a + beta @ b)
+    assert abs(f - f0) < 1e-13 * max(1.0, abs(f0)) and np.all(np.isfinite(g))
+    assert prim == np.inf or np.isnan(prim)
