@@ -191,7 +191,7 @@ typedef struct {
     double cg_tol;       /* <= 0: driver default */
     int cg_max_iter;     /* <= 0: driver default */
     const double* x0;    /* optional warm start (n+m-1), host; NULL = reference init */
-    int bcd_batch;       /* BCD iterations enqueued per batch (two in flight); <= 0: 8 */
+    int bcd_batch;       /* BCD iterations enqueued per batch (two in flight); <= 0: by the iteration's length (1 to 8) */
     /* BCD iteration form.  0: two passes over M per iteration (row pass,
      * column pass); nonzero (default 1): one pass per iteration when
      * m <= 8192 (FP32 bulk in FP32 arithmetic: m <= 16384), at most 1024 rows

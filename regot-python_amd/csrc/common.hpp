@@ -49,21 +49,22 @@ enum Status : int {
 
 #define KERNEL_CHECK() HIP_CHECK(hipGetLastError())
 
-// Owning device allocation (hipMalloc), released on destruction.
+// Device allocation (hipMalloc), released on destruction, or a part of a Slab.
 template <typename T>
 struct DBuf {
     T* p = nullptr;
     size_t n = 0;
+    bool owned = true;
     DBuf() = default;
     explicit DBuf(size_t count) { alloc(count); }
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
-    DBuf(DBuf&& o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DBuf(DBuf&& o) noexcept : p(o.p), n(o.n), owned(o.owned) { o.p = nullptr; o.n = 0; }
     DBuf& operator=(DBuf&& o) noexcept
     {
         if (this != &o) {
             release();
-            p = o.p; n = o.n;
+            p = o.p; n = o.n; owned = o.owned;
             o.p = nullptr; o.n = 0;
         }
         return *this;
@@ -88,11 +89,54 @@ struct DBuf {
     }
     void release()
     {
-        if (p) (void)hipFree(p);
+        if (p && owned) (void)hipFree(p);
         p = nullptr;
         n = 0;
+        owned = true;
+    }
+    // count elements at ptr, which someone else frees.
+    void view(void* ptr, size_t count)
+    {
+        release();
+        p = static_cast<T*>(ptr);
+        n = count;
+        owned = false;
     }
     operator T*() const { return p; }
+};
+
+// Several device buffers in one allocation: a handle's vectors cost one
+// hipMalloc and one hipFree (20 to 40 us each, the bulk of a small handle's
+// life) instead of a dozen.  add() every buffer, then make().
+struct Slab {
+    DBuf<unsigned char> mem;
+    struct Part {
+        void* buf;
+        void (*set)(void*, void*, size_t);
+        size_t at, count;
+    };
+    std::vector<Part> parts;
+    size_t bytes = 0;
+    template <typename T>
+    void add(DBuf<T>& b, size_t count)
+    {
+        if (count == 0) count = 1;
+        parts.push_back({&b,
+                         [](void* buf, void* ptr, size_t c) {
+                             static_cast<DBuf<T>*>(buf)->view(ptr, c);
+                         },
+                         bytes, count});
+        bytes += (count * sizeof(T) + 255) / 256 * 256;
+    }
+    void make()
+    {
+        std::vector<Part> ps;
+        ps.swap(parts);
+        const size_t total = bytes;
+        bytes = 0;
+        mem.alloc(total);
+        for (const Part& q : ps) q.set(q.buf, mem.p + q.at, q.count);
+    }
 };
 
 // Pinned host staging memory (hipHostMalloc), released on destruction.
@@ -136,6 +180,7 @@ struct MappedRing {
     {
         if (h && c <= cap) return;
         release();
+        if (c < 1) c = 1;
         HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&h), sizeof(T) * c, hipHostMallocMapped));
         HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&d), h, 0));
         cap = c;

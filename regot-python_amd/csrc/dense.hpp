@@ -77,6 +77,7 @@ struct BcdState {
     const double* beta;     // beta_k (the update writes another buffer)
     int k;                  // iteration of this launch
     int* ctl;               // [0] done, [1] iterations completed, [2] niter
+    unsigned long long* stop;   // host-visible: 0, or status << 32 | niter once stopped
     double* hist_f;         // rings of hist_cap entries (device-visible)
     double* hist_g;
     long long* hist_ts;
@@ -144,8 +145,11 @@ void launch_col_combine_sums(const double* part, long pitch, int nblk, int m, do
                              const ColEpi& epi, const BcdState& st, hipStream_t s);
 
 void launch_fill(double* p, double v, long count, hipStream_t s);
-void launch_fill_int(int* p, int v, long count, hipStream_t s);
-void launch_stamp(long long* dst, hipStream_t s);
+// dst = src (either may be device-mapped host memory)
+void launch_copy(const double* src, double* dst, long count, hipStream_t s);
+// Start state of the BCD loop at iteration k0: ctl = {0, k0, 0, 0}, both stall
+// slots {+inf, k0}; stamp (nullable) <- the device clock.
+void launch_bcd_begin(int* ctl, double* stall, int k0, long long* stamp, hipStream_t s);
 // gamma -> (alpha, beta) with beta_{m-1} = 0 and the given scale: out = x * k.
 void launch_split_gamma(const double* gamma, int n, int m, double* alpha, double* beta,
                         hipStream_t s);

@@ -150,26 +150,29 @@ __device__ void bcd_decide(const BcdState& st)
     if (done || stall) {
         st.ctl[2] = kk;
         st.ctl[0] = stall ? 2 : 1;
+        // one 8-byte store: the host may look before this launch is complete
+        st.stop[0] = (stall ? 2ull : 1ull) << 32 | static_cast<unsigned>(kk);
     } else {
         st.ctl[1] = kk + 1;
     }
 }
 
-// Sum (or maximum) over the kCombineSubs threads of each column, in a fixed
-// order; the result is on every thread of the column.  x[sub][col] in LDS.
-template <bool MAX>
+// Sum (or maximum) over the NS threads of each column, neighbours first; the
+// result is on every thread of the column.  x[sub][col] in LDS.
+template <bool MAX, int NS>
 __device__ __forceinline__ double combine_subs(double v, double (*x)[kCombineCols], int sub,
                                                int col)
 {
     x[sub][col] = v;
     __syncthreads();
-    double y[kCombineSubs];
+    double y[NS];
 #pragma unroll
-    for (int q = 0; q < kCombineSubs; q++) y[q] = x[q][col];
+    for (int q = 0; q < NS; q++) y[q] = x[q][col];
 #pragma unroll
-    for (int o = kCombineSubs / 2; o > 0; o >>= 1)
+    for (int o = 1; o < NS; o <<= 1)
 #pragma unroll
-        for (int q = 0; q < o; q++) y[q] = MAX ? fmax(y[q], y[q + o]) : y[q] + y[q + o];
+        for (int q = 0; q < NS; q += 2 * o)
+            y[q] = MAX ? fmax(y[q], y[q + o]) : y[q] + y[q + o];
     return y[0];
 }
 
@@ -180,7 +183,10 @@ __device__ __forceinline__ double combine_subs(double v, double (*x)[kCombineCol
 // the decision, and when the loop stops at k, beta_k is still in its buffer.
 // (Every workgroup taking the decision itself before its update put two more
 // memory round trips on the critical path.)  The tile sums of the new column
-// residual go to the other parity half of cpart.
+// residual go to the other parity half of cpart.  Without BCD (one call, not a
+// loop) four threads per column add the partials p = sub, sub + 4, ...: that
+// order is the one the solvers started from optimal_beta have always had, and
+// an L-BFGS path follows its last bit.
 // SUMS: the partials are plain FP64 column sums of exp((alpha_i + colpot_j -
 // M_ij) / reg) (the single-read BCD pass), so log2 sum_i 2^((alpha_i - M_ij) k)
 // = log2(sum) - colpot_j k.
@@ -194,6 +200,7 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
         bcd_decide(st);
         return;
     }
+    constexpr int NS = BCD ? kCombineSubs : 4;
     __shared__ double xs[kCombineSubs][kCombineCols];
     const int col = threadIdx.x & (kCombineCols - 1);
     const int sub = threadIdx.x / kCombineCols;
@@ -231,21 +238,21 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
                 for (int u = 0; u < U; u++) cs += x[u];
             }
         }
-        cs = combine_subs<false>(cs, xs, sub, col);
+        cs = combine_subs<false, NS>(cs, xs, sub, col);
         L = cs > 0.0 ? log2(cs) - cp * k : -INFINITY;
     } else {
         double Lm = -INFINITY;
-        if (valid)
-            for (int p = sub; p < nblk; p += kCombineSubs) Lm = fmax(Lm, pj[p * pitch]);
-        Lm = combine_subs<true>(Lm, xs, sub, col);
+        if (valid && sub < NS)
+            for (int p = sub; p < nblk; p += NS) Lm = fmax(Lm, pj[p * pitch]);
+        Lm = combine_subs<true, NS>(Lm, xs, sub, col);
         double S = 0.0;
-        if (valid && Lm != -INFINITY)
-            for (int p = sub; p < nblk; p += kCombineSubs) {
+        if (valid && sub < NS && Lm != -INFINITY)
+            for (int p = sub; p < nblk; p += NS) {
                 const double x = pj[p * pitch];
                 S += (x == -INFINITY) ? 0.0 : exp2(x - Lm);
             }
         __syncthreads();
-        S = combine_subs<false>(S, xs, sub, col);
+        S = combine_subs<false, NS>(S, xs, sub, col);
         L = (Lm == -INFINITY) ? -INFINITY : Lm + log2(S);
     }
     if (sub != 0) return;
@@ -308,16 +315,25 @@ __global__ void k_fill(double* p, double v, long count)
         p[i] = v;
 }
 
-__global__ void k_fill_int(int* p, int v, long count)
+__global__ void k_copy(const double* __restrict__ src, double* __restrict__ dst, long count)
 {
     for (long i = static_cast<long>(blockIdx.x) * 256 + threadIdx.x; i < count;
          i += static_cast<long>(gridDim.x) * 256)
-        p[i] = v;
+        dst[i] = src[i];
 }
 
-__global__ void k_stamp(long long* dst)
+__global__ void k_bcd_begin(int* ctl, double* stall, int k0, long long* stamp)
 {
-    if (threadIdx.x == 0) dst[0] = static_cast<long long>(wall_clock64());
+    if (threadIdx.x != 0) return;
+    ctl[0] = 0;
+    ctl[1] = k0;
+    ctl[2] = 0;
+    ctl[3] = 0;
+    for (int q = 0; q < 2; q++) {
+        stall[2 * q] = INFINITY;
+        stall[2 * q + 1] = static_cast<double>(k0);
+    }
+    if (stamp) stamp[0] = static_cast<long long>(wall_clock64());
 }
 
 __global__ void k_split_gamma(const double* gamma, int n, int m, double* alpha, double* beta)
@@ -483,16 +499,16 @@ void launch_fill(double* p, double v, long count, hipStream_t s)
     KERNEL_CHECK();
 }
 
-void launch_fill_int(int* p, int v, long count, hipStream_t s)
+void launch_copy(const double* src, double* dst, long count, hipStream_t s)
 {
     if (count <= 0) return;
-    hipLaunchKernelGGL(k_fill_int, dim3(grid_for(count)), dim3(256), 0, s, p, v, count);
+    hipLaunchKernelGGL(k_copy, dim3(grid_for(count)), dim3(256), 0, s, src, dst, count);
     KERNEL_CHECK();
 }
 
-void launch_stamp(long long* dst, hipStream_t s)
+void launch_bcd_begin(int* ctl, double* stall, int k0, long long* stamp, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, s, dst);
+    hipLaunchKernelGGL(k_bcd_begin, dim3(1), dim3(64), 0, s, ctl, stall, k0, stamp);
     KERNEL_CHECK();
 }
 

@@ -38,8 +38,6 @@ struct Work {
     long N;
     hipStream_t s;
     DBuf<double> gamma, g, direc, step, Hstep, x, xg, rhs, y, sv, g_pre, gamma_pre, lr0, lr1;
-    DBuf<double> dscal;
-    HBuf<double> hscal;
     long long cg_iters = 0;
     // algorithmic HBM bytes of the work done: n m s per objective or gradient
     // evaluation (one logical read of M), n m s + 2 nnz 12 per Hessian build
@@ -59,8 +57,6 @@ struct Work {
         for (DBuf<double>* b : {&gamma, &g, &direc, &step, &Hstep, &x, &xg, &rhs, &y, &sv, &g_pre,
                                 &gamma_pre, &lr0, &lr1})
             b->alloc(N);
-        dscal.alloc(8);
-        hscal.ensure(8);
     }
 
     // Reference init (e.g. src/sinkhorn_ssns.cpp:53-62): alpha = 0,
@@ -82,19 +78,17 @@ struct Work {
     {
         const double* xs[1] = {a};
         const double* ys[1] = {b};
-        vec_dots(xs, ys, N, 1, dscal, s);
-        HIP_CHECK(hipMemcpyAsync(hscal.p, dscal.p, sizeof(double), hipMemcpyDeviceToHost, s));
+        vec_dots(xs, ys, N, 1, p->mscal.d + 8, s);
         HIP_CHECK(hipStreamSynchronize(s));
-        return hscal.p[0];
+        return p->mscal.h[8];
     }
 
     // Several dots in one launch.
     void dots(int k, const double* const* a, const double* const* b, double* out)
     {
-        vec_dots(a, b, N, k, dscal, s);
-        HIP_CHECK(hipMemcpyAsync(hscal.p, dscal.p, k * sizeof(double), hipMemcpyDeviceToHost, s));
+        vec_dots(a, b, N, k, p->mscal.d + 8, s);
         HIP_CHECK(hipStreamSynchronize(s));
-        for (int q = 0; q < k; q++) out[q] = hscal.p[q];
+        for (int q = 0; q < k; q++) out[q] = p->mscal.h[8 + q];
     }
 
     // [a; b_0..m-2] . v, for objectives formed from one point's T with
@@ -103,11 +97,10 @@ struct Work {
     {
         const double* xs[2] = {v, v + n};
         const double* ys[2] = {p->a.p, p->b.p};
-        vec_dots(xs, ys, n, 1, dscal, s);
-        vec_dots(xs + 1, ys + 1, m - 1, 1, dscal.p + 1, s);
-        HIP_CHECK(hipMemcpyAsync(hscal.p, dscal.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+        vec_dots(xs, ys, n, 1, p->mscal.d + 8, s);
+        vec_dots(xs + 1, ys + 1, m - 1, 1, p->mscal.d + 9, s);
         HIP_CHECK(hipStreamSynchronize(s));
-        return hscal.p[0] + hscal.p[1];
+        return p->mscal.h[8] + p->mscal.h[9];
     }
 
     // out = x + t d

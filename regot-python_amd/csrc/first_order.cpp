@@ -171,9 +171,7 @@ int lbfgs_minimize(Work& w, double eps_abs, double eps_rel, int max_iter,
     const double eps = std::numeric_limits<double>::epsilon();
     const long N = w.N;
     DBuf<double> S(static_cast<size_t>(mm) * N), Y(static_cast<size_t>(mm) * N);
-    DBuf<double> dpart(vec_mdots_scratch(N)), dout(32);
-    HBuf<double> hout;
-    hout.ensure(32);
+    DBuf<double> dpart(vec_mdots_scratch(N));
     auto slot_s = [&](int i) { return S.p + static_cast<long>(i) * N; };
     auto slot_y = [&](int i) { return Y.p + static_cast<long>(i) * N; };
     // Gram matrices of the correction pairs (by ring slot): SY[i][j] = s_i'y_j,
@@ -243,11 +241,9 @@ int lbfgs_minimize(Work& w, double eps_abs, double eps_rel, int max_iter,
                 i_Sv[i] = add(slot_s(i), v);
                 i_Yv[i] = add(slot_y(i), v);
             }
-            vec_mdots(xs, zs, np, N, dpart, dout, w.s);
-            HIP_CHECK(hipMemcpyAsync(hout.p, dout.p, np * sizeof(double), hipMemcpyDeviceToHost,
-                                     w.s));
+            vec_mdots(xs, zs, np, N, dpart, w.p->mscal.d + 8, w.s);
             HIP_CHECK(hipStreamSynchronize(w.s));
-            const double* d = hout.p;
+            const double* d = w.p->mscal.h + 8;
             double Sv[6] = {}, Yv[6] = {};
             for (int i : act) {
                 Sv[i] = d[i_Sv[i]];
@@ -390,17 +386,15 @@ void solve_apdagd(regot_problem* p, double tol, int max_iter, int verbose, const
     res->plan_device = p->device;
     long nrp, ncp, nsc, npt;
     apd_scratch_sizes(n, m, &nrp, &ncp, &nsc, &npt);
-    DBuf<double> rowpart(nrp), colpart(ncp), scal(nsc), part(npt), out(3);
-    HBuf<double> hout;
-    hout.ensure(3);
+    DBuf<double> rowpart(nrp), colpart(ncp), scal(nsc), part(npt);
+    const double* const hout = p->mscal.h + 40;   // written by the plan pass
     DBuf<double> alpha(n), beta(m);
     auto plan_pass = [&](double tau, bool init) {
         launch_split_gamma(x, n, m, alpha, beta, w.s);
         launch_apd_plan(p->bulk, p->dM, p->ldm, n, m, alpha, beta, p->a, p->b, p->reg, tau, init,
-                        res->plan, ldp, rowpart, colpart, scal, part, out, w.s);
+                        res->plan, ldp, rowpart, colpart, scal, part, p->mscal.d + 40, w.s);
         // read M (and P unless init), write P
         w.alg_bytes += static_cast<double>(n) * m * ((p->bulk == 0 ? 4.0 : 8.0) + (init ? 8 : 16));
-        HIP_CHECK(hipMemcpyAsync(hout.p, out.p, 3 * sizeof(double), hipMemcpyDeviceToHost, w.s));
         HIP_CHECK(hipStreamSynchronize(w.s));
     };
     plan_pass(1.0, true);   // result.get_plan(gamma) at the initial point
@@ -453,8 +447,8 @@ void solve_apdagd(regot_problem* p, double tol, int max_iter, int verbose, const
         }
         vec_axpby(x, -1.0, dt, 0.0, nullptr, w.N, w.s);
         plan_pass(ptau, false);
-        const double primal_obj = hout.p[1] - p->reg * hout.p[2];
-        const double mar_err = std::sqrt(hout.p[0]);
+        const double primal_obj = hout[1] - p->reg * hout[2];
+        const double mar_err = std::sqrt(hout[0]);
         res->obj_vals.push_back(f);
         res->mar_errs.push_back(mar_err);
         res->run_times.push_back(res->run_times.back() + timer.toc());

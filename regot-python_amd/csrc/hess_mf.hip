@@ -398,6 +398,7 @@ __global__ __launch_bounds__(TH) void k_mf_pass(MfArgs a)
             if (stop) {
                 a.ctl[1] = a.it;   // the converged update is not counted
                 a.ctl[0] = 1;
+                a.rep[0] = 1.0;
             }
         }
         if (stop) return;

@@ -41,6 +41,7 @@ struct MfArgs {
     const double* rr_part = nullptr;
     int rr_n = 0;
     double* scal = nullptr;
+    double* rep = nullptr;          // host-visible: rep[0] = 1 on stop
     int it = 0;
     int rpw = 0;                    // rows per workgroup (set by the launcher)
     int nt = 0;                     // nontemporal loads (set by the launcher)

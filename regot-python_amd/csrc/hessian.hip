@@ -86,6 +86,7 @@ struct CgArgs {
     int nbc;        // column workgroups
     int nbu;        // update workgroups (256 entries each)
     const double* dinv;   // Jacobi preconditioner, or null
+    double* rep;          // host-visible: rep[0] = 1 on stop
 };
 
 // dinv_j = 1 / (h2_j + shift - sum_i sigma_ij^2 / (h1_i + shift)), the diagonal
@@ -117,17 +118,27 @@ __global__ __launch_bounds__(256) void k_delta_diag(const int* __restrict__ colp
 }
 
 // u = dinv .* r (or r), partials of r.u and r.r per 1024 entries.
-__global__ __launch_bounds__(256) void k_pcg_start(const double* __restrict__ r,
+// r as given, or (rhs set) r = rhs from a zero start: then also x = 0.  p = s =
+// 0, u = D^-1 r (or r); part = the workgroup's sums of r.u and r.r.
+__global__ __launch_bounds__(256) void k_pcg_start(double* __restrict__ r,
+                                                   const double* __restrict__ rhs,
                                                    const double* __restrict__ dinv, int m1,
-                                                   double* __restrict__ u,
+                                                   double* __restrict__ u, double* __restrict__ x,
+                                                   double* __restrict__ p, double* __restrict__ s,
                                                    double* __restrict__ part)
 {
     __shared__ double sm[2][256];
     double rz = 0.0, rr = 0.0;
     for (int j = blockIdx.x * 1024 + threadIdx.x; j < (blockIdx.x + 1) * 1024 && j < m1;
          j += 256) {
-        const double rj = r[j];
+        const double rj = rhs ? rhs[j] : r[j];
         const double zj = dinv ? rj * dinv[j] : rj;
+        if (rhs) {
+            r[j] = rj;
+            x[j] = 0.0;
+        }
+        p[j] = 0.0;
+        s[j] = 0.0;
         u[j] = zj;
         rz += rj * zj;
         rr += rj * rj;
@@ -146,6 +157,56 @@ __global__ __launch_bounds__(256) void k_pcg_start(const double* __restrict__ r,
         part[2 * blockIdx.x] = sm[0][0];
         part[2 * blockIdx.x + 1] = sm[1][0];
     }
+}
+
+// Scalars of a CG's first iteration from the set-up partials (nbs pairs of r.u,
+// r.r) and scal[6] = rhs.rhs, scal[7] = w.u, with no host round trip before
+// the iterations: scal = {alpha_0, 0, gamma_0, 0, r.r, threshold}.  ctl =
+// {stopped, 0, how}: a zero right-hand side (1) or a start that already meets
+// the rule (2: tol >= 1 without a guess, an exact guess, or no iterations
+// allowed) stops the CG at once.
+struct CgBegin {
+    const double* part;
+    double* scal;
+    int* ctl;
+    double* rep;
+};
+
+__global__ void k_cg_begin(CgBegin b0, CgBegin b1, int nbs, double tol, int max_iter)
+{
+    const CgBegin b = blockIdx.x == 0 ? b0 : b1;
+    if (threadIdx.x != 0) return;
+    double rz = 0.0, rr = 0.0;
+    for (int q = 0; q < nbs; q++) {
+        rz += b.part[2 * q];
+        rr += b.part[2 * q + 1];
+    }
+    const double norm2 = b.scal[6], delta = b.scal[7];
+    double thr = tol * tol * norm2;
+    if (thr < 2.2250738585072014e-308) thr = 2.2250738585072014e-308;
+    b.scal[0] = rz / delta;
+    b.scal[1] = 0.0;
+    b.scal[2] = rz;
+    b.scal[3] = 0.0;
+    b.scal[4] = rr;
+    b.scal[5] = thr;
+    const int how = norm2 == 0.0 ? 1 : (rr < thr || max_iter <= 0) ? 2 : 0;
+    b.ctl[1] = 0;
+    b.ctl[2] = how;
+    b.ctl[0] = how != 0;
+    if (how != 0) b.rep[0] = 1.0;
+}
+
+// The outcome where the host reads it: {stopped, iterations, how, r.r, rhs.rhs}.
+__global__ void k_cg_end(CgBegin b0, CgBegin b1)
+{
+    const CgBegin b = blockIdx.x == 0 ? b0 : b1;
+    if (threadIdx.x != 0) return;
+    b.rep[0] = b.ctl[0];
+    b.rep[1] = b.ctl[1];
+    b.rep[2] = b.ctl[2];
+    b.rep[3] = b.scal[4];
+    b.rep[4] = b.scal[6];
 }
 
 // Fixed-order sums of NV values over the 256 threads: each wave's by DPP and
@@ -297,6 +358,7 @@ __global__ __launch_bounds__(256) void k_cg_cols(CgArgs a0, CgArgs a1, int it)
             a.scal[4] = rr;
             a.ctl[1] = it;   // the converged update is not counted (Eigen's convention)
             a.ctl[0] = 1;
+            a.rep[0] = 1.0;
         }
         return;
     }
@@ -728,11 +790,7 @@ struct CgSide {
     const double* x0 = nullptr;    // device, m-1, or null (start from 0)
     DBuf<double>*r, *pv, *q, *sv, *u, *y, *part, *scal;
     DBuf<int>* ctl;
-    HBuf<int>* hctl;
-    HBuf<double>* hbuf;
-    std::vector<double> hpart;
-    bool active = false;
-    double rhs_norm2 = 0.0;
+    MappedRing<double>* rep;
     int iters = 0;
     double tol_error = 0.0;
     CgArgs a;
@@ -791,61 +849,21 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
         c.part->ensure(std::max(2L * nbc + nbu, 2L * nbs));
         c.scal->ensure(8);
         c.ctl->ensure(4);
-        c.hctl->ensure(16);
-        c.hbuf->ensure(8);
+        c.rep->ensure(8);
+        c.rep->h[0] = 0.0;   // the stream holds no launch that writes it
         if (c.x0) {
             vec_copy(c.x, c.x0, m1, s);
             hess_apply_delta(p, c.x0, shift, *c.q);
             vec_axpby(*c.r, 1.0, c.rhs, -1.0, *c.q, m1, s);
-        } else {
-            launch_fill(c.x, 0.0, m1, s);
-            vec_copy(*c.r, c.rhs, m1, s);
         }
-        hipLaunchKernelGGL(k_pcg_start, dim3(nbs), dim3(256), 0, s, c.r->p, dinv, m1, c.u->p,
+        hipLaunchKernelGGL(k_pcg_start, dim3(nbs), dim3(256), 0, s, c.r->p,
+                           c.x0 ? nullptr : c.rhs, dinv, m1, c.u->p, c.x, c.pv->p, c.sv->p,
                            c.part->p);
         KERNEL_CHECK();
         hess_apply_delta(p, *c.u, shift, *c.q);
         const double* xs[2] = {c.rhs, c.q->p};
         const double* ys[2] = {c.rhs, c.u->p};
         vec_dots(xs, ys, m1, 2, c.scal->p + 6, s);
-        c.hpart.assign(2L * nbs, 0.0);
-        HIP_CHECK(hipMemcpyAsync(c.hpart.data(), c.part->p, 2L * nbs * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipMemcpyAsync(c.hbuf->p, c.scal->p + 6, 2 * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
-        launch_fill(*c.pv, 0.0, m1, s);
-        launch_fill(*c.sv, 0.0, m1, s);
-    }
-    HIP_CHECK(hipStreamSynchronize(s));
-    int act[2] = {0, 0};
-    int na = 0;
-    for (int k = 0; k < nr; k++) {
-        CgSide& c = S[k];
-        c.rhs_norm2 = c.hbuf->p[0];
-        const double delta0 = c.hbuf->p[1];
-        double rz0 = 0.0, rr0 = 0.0;
-        for (int b = 0; b < nbs; b++) {
-            rz0 += c.hpart[2 * b];
-            rr0 += c.hpart[2 * b + 1];
-        }
-        c.iters = 0;
-        c.active = false;
-        if (c.rhs_norm2 == 0.0) {
-            if (c.x0) launch_fill(c.x, 0.0, m1, s);
-            c.tol_error = 0.0;
-            continue;
-        }
-        double thr = tol * tol * c.rhs_norm2;
-        if (thr < 2.2250738585072014e-308) thr = 2.2250738585072014e-308;
-        // converged at the start (tol >= 1 without a guess, or an exact guess)
-        if (rr0 < thr || max_iter <= 0) {
-            c.tol_error = std::sqrt(rr0 / c.rhs_norm2);
-            continue;
-        }
-        double hs[7] = {rz0 / delta0, 0.0, rz0, 0.0, rr0, thr, c.rhs_norm2};
-        HIP_CHECK(hipMemcpyAsync(c.scal->p, hs, 7 * sizeof(double), hipMemcpyHostToDevice, s));
-        int hc[4] = {0, 0, 0, 0};
-        HIP_CHECK(hipMemcpyAsync(c.ctl->p, hc, 4 * sizeof(int), hipMemcpyHostToDevice, s));
         CgArgs& a = c.a;
         a.rowptr = H.rowptr;
         a.colind = H.colind;
@@ -871,20 +889,24 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
         a.nbc = nbc;
         a.nbu = nbu;
         a.dinv = dinv;
-        c.active = true;
-        act[na++] = k;
+        a.rep = c.rep->d;
     }
-    if (na == 0) return;
-    const CgArgs& a0 = S[act[0]].a;
-    const CgArgs& a1 = S[act[na - 1]].a;
+    const CgArgs& a0 = S[0].a;
+    const CgArgs& a1 = S[nr - 1].a;
+    auto begin_of = [](const CgArgs& a) { return CgBegin{a.part, a.scal, a.ctl, a.rep}; };
+    const CgBegin b0 = begin_of(a0), b1 = begin_of(a1);
+    hipLaunchKernelGGL(k_cg_begin, dim3(nr), dim3(64), 0, s, b0, b1, nbs, tol, max_iter);
+    KERNEL_CHECK();
 
     // batches of K iterations, two in flight; iteration indices run 0 ..
-    // max_iter - 1 and nothing is enqueued past them
-    const int K = 16;
+    // max_iter - 1 and nothing is enqueued past them.  What runs past the stop
+    // returns at once but still drains (three launches of some 2 us each); a
+    // batch of 8 iterations of 17 us covers the host's turn-round.
+    const int K = 8;
     int k_enq = 0;
-    hipEvent_t ev[2];
-    HIP_CHECK(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming));
-    HIP_CHECK(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming));
+    for (auto& e : H.cg_ev)
+        if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    hipEvent_t* const ev = H.cg_ev;
     // matrix-free: the pass over M makes the stop test and y = (sigma u) /
     // (h1 + shift) and sigma' y in one read; k_cg_cols_mf folds its partials
     MfArgs ma;
@@ -897,66 +919,64 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
         ma.rr_part = a0.part + 2 * nbc;
         ma.rr_n = nbu;
         ma.scal = a0.scal;
+        ma.rep = a0.rep;
     }
     auto launch_batch = [&](int slot) {
         for (int q = 0; q < K && k_enq < max_iter; q++, k_enq++) {
-            hipLaunchKernelGGL(k_cg_update, dim3(nbu, na), dim3(256), 0, s, a0, a1, k_enq);
+            hipLaunchKernelGGL(k_cg_update, dim3(nbu, nr), dim3(256), 0, s, a0, a1, k_enq);
             if (H.mf) {
                 ma.it = k_enq;
                 launch_mf_pass(MF_CG, ma, H.mf_nwg, s);
                 hipLaunchKernelGGL(k_cg_cols_mf, dim3(nbc), dim3(256), 0, s, a0, H.mf_part.p,
                                    H.mf_nwg);
             } else {
-                cg_rows(lpr_r, a0, a1, na, s);
-                cg_cols(lpr_c, a0, a1, na, k_enq, s);
+                cg_rows(lpr_r, a0, a1, nr, s);
+                cg_cols(lpr_c, a0, a1, nr, k_enq, s);
             }
         }
         KERNEL_CHECK();
-        for (int j = 0; j < na; j++) {
-            CgSide& c = S[act[j]];
-            HIP_CHECK(hipMemcpyAsync(c.hctl->p + 4 * slot, c.ctl->p, 4 * sizeof(int),
-                                     hipMemcpyDeviceToHost, s));
-        }
         HIP_CHECK(hipEventRecord(ev[slot], s));
     };
-    auto all_done = [&](int slot) {
-        for (int j = 0; j < na; j++)
-            if (!S[act[j]].hctl->p[4 * slot]) return false;
+    auto all_done = [&]() {
+        for (int k = 0; k < nr; k++)
+            if (*static_cast<volatile double*>(S[k].rep->h) == 0.0) return false;
         return true;
     };
     try {
         std::deque<int> qu;
-        launch_batch(0);
-        qu.push_back(0);
-        if (k_enq < max_iter) {
-            launch_batch(1);
-            qu.push_back(1);
+        for (int slot = 0; slot < 2 && k_enq < max_iter; slot++) {
+            launch_batch(slot);
+            qu.push_back(slot);
         }
         while (!qu.empty()) {
             const int slot = qu.front();
             qu.pop_front();
             HIP_CHECK(hipEventSynchronize(ev[slot]));
-            if (all_done(slot)) break;
+            if (all_done()) break;
             if (k_enq < max_iter) {
                 launch_batch(slot);
                 qu.push_back(slot);
             }
         }
+        hipLaunchKernelGGL(k_cg_end, dim3(nr), dim3(64), 0, s, b0, b1);
+        KERNEL_CHECK();
         HIP_CHECK(hipStreamSynchronize(s));
     } catch (...) {
         (void)hipStreamSynchronize(s);
-        (void)hipEventDestroy(ev[0]);
-        (void)hipEventDestroy(ev[1]);
         throw;
     }
-    HIP_CHECK(hipEventDestroy(ev[0]));
-    HIP_CHECK(hipEventDestroy(ev[1]));
-    for (int j = 0; j < na; j++) {
-        CgSide& c = S[act[j]];
-        HIP_CHECK(hipMemcpy(c.hctl->p + 8, c.ctl->p, 4 * sizeof(int), hipMemcpyDeviceToHost));
-        HIP_CHECK(hipMemcpy(c.hbuf->p, c.scal->p, 5 * sizeof(double), hipMemcpyDeviceToHost));
-        c.iters = c.hctl->p[8] ? c.hctl->p[9] : max_iter;
-        c.tol_error = std::sqrt(c.hbuf->p[4] / c.rhs_norm2);
+    for (int k = 0; k < nr; k++) {
+        CgSide& c = S[k];
+        const double* rep = c.rep->h;
+        const int how = static_cast<int>(rep[2]);
+        if (how == 1) {   // a zero right-hand side: x = 0
+            if (c.x0) launch_fill(c.x, 0.0, m1, s);
+            c.iters = 0;
+            c.tol_error = 0.0;
+        } else {
+            c.iters = how != 0 ? 0 : rep[0] != 0.0 ? static_cast<int>(rep[1]) : max_iter;
+            c.tol_error = std::sqrt(rep[3] / rep[4]);
+        }
     }
 }
 
@@ -974,8 +994,7 @@ static CgSide cg_side(SparseHessian& H, int k)
         c.part = &H.cg_part;
         c.scal = &H.cg_scal;
         c.ctl = &H.cg_ctl;
-        c.hctl = &H.cg_hctl;
-        c.hbuf = &H.hbuf;
+        c.rep = &H.cg_rep;
     } else {
         c.r = &H.cg1_r;
         c.pv = &H.cg1_p;
@@ -986,8 +1005,7 @@ static CgSide cg_side(SparseHessian& H, int k)
         c.part = &H.cg1_part;
         c.scal = &H.cg1_scal;
         c.ctl = &H.cg1_ctl;
-        c.hctl = &H.cg1_hctl;
-        c.hbuf = &H.hbuf1;
+        c.rep = &H.cg1_rep;
     }
     return c;
 }
@@ -1130,8 +1148,7 @@ static void hess_check(regot_problem* p, bool need_built)
 static void upload_and_grad(regot_problem* p, const double* gamma)
 {
     const long N = p->n + p->m - 1;
-    HIP_CHECK(hipMemcpyAsync(p->gamma, gamma, N * sizeof(double), hipMemcpyHostToDevice,
-                             p->stream));
+    launch_copy(p->stage(gamma, N), p->gamma, N, p->stream);
     (void)p->dev_obj_grad(p->gamma, p->grad, nullptr);
 }
 
@@ -1210,11 +1227,10 @@ int regot_hess_apply_delta(regot_problem* p, const double* x, double shift, doub
     CAPI_BEGIN
     hess_check(p, true);
     const int m1 = p->m - 1;
-    DBuf<double> dx(m1), dr(m1);
-    HIP_CHECK(hipMemcpyAsync(dx, x, m1 * sizeof(double), hipMemcpyHostToDevice, p->stream));
-    hess_apply_delta(p, dx, shift, dr);
-    HIP_CHECK(hipMemcpyAsync(res, dr, m1 * sizeof(double), hipMemcpyDeviceToHost, p->stream));
-    p->sync();
+    p->cin.ensure(m1);
+    launch_copy(p->stage(x, m1), p->cin, m1, p->stream);
+    hess_apply_delta(p, p->cin, shift, p->stage_out(m1));
+    p->unstage(res, m1);
     CAPI_END
 }
 
@@ -1223,11 +1239,12 @@ int regot_hess_apply_hs(regot_problem* p, const double* x, double* res)
     CAPI_BEGIN
     hess_check(p, true);
     const long N = p->n + p->m - 1;
-    DBuf<double> dx(N), dr(N);
-    HIP_CHECK(hipMemcpyAsync(dx, x, N * sizeof(double), hipMemcpyHostToDevice, p->stream));
-    hess_apply_hs(p, dx, dr);
-    HIP_CHECK(hipMemcpyAsync(res, dr, N * sizeof(double), hipMemcpyDeviceToHost, p->stream));
-    p->sync();
+    p->cin.ensure(N);
+    p->cout.ensure(N);
+    launch_copy(p->stage(x, N), p->cin, N, p->stream);
+    hess_apply_hs(p, p->cin, p->cout);
+    launch_copy(p->cout, p->stage_out(N), N, p->stream);
+    p->unstage(res, N);
     CAPI_END
 }
 
@@ -1260,12 +1277,13 @@ int regot_hess_cg(regot_problem* p, const double* rhs, double shift, double tol,
     CAPI_BEGIN
     hess_check(p, true);
     const long N = p->n + p->m - 1;
-    DBuf<double> dx(N), dr(N);
-    HIP_CHECK(hipMemcpyAsync(dx, rhs, N * sizeof(double), hipMemcpyHostToDevice, p->stream));
+    p->cin.ensure(N);
+    p->cout.ensure(N);
+    launch_copy(p->stage(rhs, N), p->cin, N, p->stream);
     double te = 0.0;
-    const int it = hess_cg(p, dx, shift, tol, max_iter, dr, &te);
-    HIP_CHECK(hipMemcpyAsync(res, dr, N * sizeof(double), hipMemcpyDeviceToHost, p->stream));
-    p->sync();
+    const int it = hess_cg(p, p->cin, shift, tol, max_iter, p->cout, &te);
+    launch_copy(p->cout, p->stage_out(N), N, p->stream);
+    p->unstage(res, N);
     if (iters) *iters = it;
     if (tol_error) *tol_error = te;
     CAPI_END

@@ -117,7 +117,8 @@ void regot_problem::setup(int n_, int m_, const void* M, int M_dtype, int bulk_,
             KERNEL_CHECK();
         } else {
             // Host source: convert/pad row chunks in pinned staging, then copy.
-            const long rows_per = std::max<long>(1, (32L << 20) / (ldm * esz));
+            const long rows_per =
+                std::min<long>(n, std::max<long>(1, (32L << 20) / (ldm * static_cast<long>(esz))));
             HBuf<unsigned char> stage;
             stage.ensure(static_cast<size_t>(rows_per) * ldm * esz);
             for (long r0 = 0; r0 < n; r0 += rows_per) {
@@ -164,33 +165,56 @@ void regot_problem::setup(int n_, int m_, const void* M, int M_dtype, int bulk_,
     HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
     HIP_CHECK(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, device));
 
-    a.alloc(n);
-    b.alloc(m);
-    loga.alloc(n);
-    logb.alloc(m);
+    nblk = col_pass_blocks(n, m);
+    ntiles = col_combine_blocks(m);
+    slab.add(a, n);
+    slab.add(b, m);
+    slab.add(loga, n);
+    slab.add(logb, m);
+    slab.add(alpha, n);
+    slab.add(beta, m);
+    slab.add(rsum, n);
+    slab.add(csum, m);
+    slab.add(gamma, static_cast<size_t>(n) + m);
+    slab.add(grad, static_cast<size_t>(n) + m);
+    slab.add(scal, 64);
+    slab.add(ctl, 16);
+    slab.add(part, static_cast<size_t>(nblk) * m);
+    slab.make();
     HIP_CHECK(hipMemcpyAsync(a, a_h, n * sizeof(double), hipMemcpyHostToDevice, stream));
     HIP_CHECK(hipMemcpyAsync(b, b_h, m * sizeof(double), hipMemcpyHostToDevice, stream));
     hipLaunchKernelGGL(k_log, dim3(ceil_div(n, 256)), dim3(256), 0, stream, a.p, loga.p, n);
     hipLaunchKernelGGL(k_log, dim3(ceil_div(m, 256)), dim3(256), 0, stream, b.p, logb.p, m);
     KERNEL_CHECK();
 
-    alpha.alloc(n);
-    beta.alloc(m);
-    rsum.alloc(n);
-    csum.alloc(m);
-    gamma.alloc(n + m);
-    grad.alloc(n + m);
-    scal.alloc(64);
-    ctl.alloc(16);
-    nblk = col_pass_blocks(n, m);
-    part.alloc(static_cast<size_t>(nblk) * m);
-    ntiles = col_combine_blocks(m);
-    hscal.ensure(64);
-    hctl.ensure(16);
+    // scalars, then room for a vector each way: one pinned allocation
+    mscal.ensure(64 + 2 * (n + m));
+    hout = mscal.h + 64 + (n + m);
     HIP_CHECK(hipStreamSynchronize(stream));
 }
 
 void regot_problem::sync() { HIP_CHECK(hipStreamSynchronize(stream)); }
+
+const double* regot_problem::stage(const double* host, long count)
+{
+    if (count > static_cast<long>(n) + m) fail(E_INTERNAL, "staging %ld values", count);
+    if (count > 0 && !host) fail(E_INVALID, "null input vector");
+    std::memcpy(mscal.h + 64, host, count * sizeof(double));
+    return mscal.d + 64;
+}
+
+double* regot_problem::stage_out(long count)
+{
+    if (count > static_cast<long>(n) + m) fail(E_INTERNAL, "staging %ld values", count);
+    return mscal.d + 64 + (n + m);
+}
+
+void regot_problem::unstage(double* host, long count)
+{
+    if (count > 0 && !host) fail(E_INVALID, "null output vector");
+    sync();
+    std::memcpy(host, hout, count * sizeof(double));
+}
 
 void regot_problem::prof_begin(int kind, hipEvent_t* stop_out)
 {
@@ -362,11 +386,10 @@ double regot_problem::dev_obj_fused(const double* d_gamma, double* d_grad, doubl
     launch_split_gamma(d_gamma, n, m, alpha, beta, stream);
     const bool with_grad = d_grad != nullptr;
     launch_objgrad_fused(bulk, dM, ldm, n, m, alpha, beta, a, b, reg, with_grad, d_grad, s_row,
-                         s_col, s_part, scal, stream);
-    HIP_CHECK(hipMemcpyAsync(hscal.p, scal.p, 2 * sizeof(double), hipMemcpyDeviceToHost, stream));
+                         s_col, s_part, mscal.d, stream);
     sync();
-    if (gnorm2) *gnorm2 = hscal.p[1];
-    return hscal.p[0];
+    if (gnorm2) *gnorm2 = mscal.h[1];
+    return mscal.h[0];
 }
 
 double regot_problem::dev_obj(const double* d_gamma)
@@ -378,10 +401,9 @@ double regot_problem::dev_obj(const double* d_gamma)
     e.rowpot = alpha;
     e.rowsum = rsum;
     row_pass(beta, e);
-    vec_obj_finish(rsum, a, b, d_gamma, n, m, reg, scal, stream);
-    HIP_CHECK(hipMemcpyAsync(hscal.p, scal.p, sizeof(double), hipMemcpyDeviceToHost, stream));
+    vec_obj_finish(rsum, a, b, d_gamma, n, m, reg, mscal.d, stream);
     sync();
-    return hscal.p[0];
+    return mscal.h[0];
 }
 
 double regot_problem::dev_obj_grad(const double* d_gamma, double* d_grad, double* gnorm2)
@@ -397,11 +419,10 @@ double regot_problem::dev_obj_grad(const double* d_gamma, double* d_grad, double
     c.colpot = beta;
     c.colsum = csum;
     col_pass(alpha, beta, c);
-    vec_objgrad_finish(rsum, csum, a, b, d_gamma, n, m, reg, d_grad, scal, stream);
-    HIP_CHECK(hipMemcpyAsync(hscal.p, scal.p, 2 * sizeof(double), hipMemcpyDeviceToHost, stream));
+    vec_objgrad_finish(rsum, csum, a, b, d_gamma, n, m, reg, d_grad, mscal.d, stream);
     sync();
-    if (gnorm2) *gnorm2 = hscal.p[1];
-    return hscal.p[0];
+    if (gnorm2) *gnorm2 = mscal.h[1];
+    return mscal.h[0];
 }
 
 // ---------------------------------------------------------------------------
@@ -508,15 +529,12 @@ int regot_optimal_alpha(regot_problem* p, const double* beta_h, double* alpha_h)
     CAPI_BEGIN
     check_handle(p);
     if (!beta_h || !alpha_h) fail(E_INVALID, "null vector");
-    HIP_CHECK(hipMemcpyAsync(p->beta, beta_h, p->m * sizeof(double), hipMemcpyHostToDevice,
-                             p->stream));
+    launch_copy(p->stage(beta_h, p->m), p->beta, p->m, p->stream);
     RowEpi e;
     e.loga = p->loga;
-    e.alpha_out = p->alpha;
+    e.alpha_out = p->stage_out(p->n);
     p->row_pass(p->beta, e);
-    HIP_CHECK(hipMemcpyAsync(alpha_h, p->alpha, p->n * sizeof(double), hipMemcpyDeviceToHost,
-                             p->stream));
-    p->sync();
+    p->unstage(alpha_h, p->n);
     CAPI_END
 }
 
@@ -525,14 +543,11 @@ int regot_optimal_beta(regot_problem* p, const double* alpha_h, double* beta_h)
     CAPI_BEGIN
     check_handle(p);
     if (!beta_h || !alpha_h) fail(E_INVALID, "null vector");
-    HIP_CHECK(hipMemcpyAsync(p->alpha, alpha_h, p->n * sizeof(double), hipMemcpyHostToDevice,
-                             p->stream));
+    launch_copy(p->stage(alpha_h, p->n), p->alpha, p->n, p->stream);
     ColEpi c;
-    c.beta_out = p->beta;
+    c.beta_out = p->stage_out(p->m);
     p->col_pass(p->alpha, nullptr, c);
-    HIP_CHECK(hipMemcpyAsync(beta_h, p->beta, p->m * sizeof(double), hipMemcpyDeviceToHost,
-                             p->stream));
-    p->sync();
+    p->unstage(beta_h, p->m);
     CAPI_END
 }
 
@@ -542,8 +557,7 @@ int regot_dual_obj(regot_problem* p, const double* gamma_h, double* obj)
     check_handle(p);
     if (!gamma_h || !obj) fail(E_INVALID, "null pointer");
     const long N = p->n + p->m - 1;
-    HIP_CHECK(hipMemcpyAsync(p->gamma, gamma_h, N * sizeof(double), hipMemcpyHostToDevice,
-                             p->stream));
+    launch_copy(p->stage(gamma_h, N), p->gamma, N, p->stream);
     *obj = p->dev_obj(p->gamma);
     CAPI_END
 }
@@ -554,12 +568,9 @@ int regot_dual_obj_grad(regot_problem* p, const double* gamma_h, double* obj, do
     check_handle(p);
     if (!gamma_h || !obj || !grad_h) fail(E_INVALID, "null pointer");
     const long N = p->n + p->m - 1;
-    HIP_CHECK(hipMemcpyAsync(p->gamma, gamma_h, N * sizeof(double), hipMemcpyHostToDevice,
-                             p->stream));
-    *obj = p->dev_obj_grad(p->gamma, p->grad, nullptr);
-    HIP_CHECK(
-        hipMemcpyAsync(grad_h, p->grad, N * sizeof(double), hipMemcpyDeviceToHost, p->stream));
-    p->sync();
+    launch_copy(p->stage(gamma_h, N), p->gamma, N, p->stream);
+    *obj = p->dev_obj_grad(p->gamma, p->stage_out(N), nullptr);
+    std::memcpy(grad_h, p->hout, N * sizeof(double));
     CAPI_END
 }
 

@@ -80,12 +80,13 @@ void launch_log_check(const double* x, double* y, long count, hipStream_t s);
 
 // Buffers of the on-device BCD loop, kept across solves on one handle.
 struct BcdWork {
+    Slab slab;
     DBuf<double> ap0, ap1, be0, be1, gcol, rpart, cpart, stall;
     DBuf<double> fpart;         // column sums of the single-read pass (blocks x m)
     DBuf<int> ctl;
     MappedRing<double> hf, hg;
     MappedRing<long long> hts;
-    HBuf<int> hc;
+    MappedRing<unsigned long long> stop;
     hipEvent_t ev[2] = {nullptr, nullptr};
     ~BcdWork()
     {
@@ -132,6 +133,7 @@ struct regot_problem {
     double sumsq_a = 0.0, sumsq_b = 0.0;   // sum a_i^2, sum b_j^2
     int ncu = 0;                // compute units of the device
     int wall_khz = 0;           // device wall clock rate (timestamps)
+    regot::Slab slab;           // the vectors of a, b, ... part below
     regot::DBuf<double> a, b, loga, logb;
 
     // scratch for the operator entry points and the drivers
@@ -140,8 +142,21 @@ struct regot_problem {
     int nblk = 1;
     int ntiles = 1;
     std::unique_ptr<regot::BcdWork> bcd;
-    regot::HBuf<double> hscal;
-    regot::HBuf<int> hctl;
+    // Results that only the host reads are written by the kernels straight into
+    // pinned, device-mapped memory and read after the stream is idle: no copy
+    // per scalar.  mscal: objective values ([0..3]) and dot products ([8..39]);
+    // from [64] on n + m values of the caller's on their way in, then as many
+    // on their way out (hout).
+    regot::MappedRing<double> mscal;
+    double* hout = nullptr;
+    regot::DBuf<double> cin, cout;   // device side of an operator call's vectors
+    // count doubles of the caller's memory where a kernel can read them (until
+    // the next stage(); the stream is idle when a call begins)
+    const double* stage(const double* host, long count);
+    // device-visible room for count doubles, read at hout after sync() ...
+    double* stage_out(long count);
+    // ... which unstage() does, into the caller's memory
+    void unstage(double* host, long count);
 
     // sparsified Hessian of the Newton-type drivers (sparse.hpp)
     std::unique_ptr<regot::SparseHessian> hess;

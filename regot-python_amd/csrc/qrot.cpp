@@ -619,13 +619,12 @@ static void solve_qrot_pdaam(regot_problem* p, double tol, int max_iter, int ver
     // ||grad_alpha||^2 and ||grad_beta||^2
     auto block_norms = [&](double* lr, double* mr) {
         const double* xs[1] = {grad};
-        vec_dots(xs, xs, n, 1, w.dscal.p, s);
+        vec_dots(xs, xs, n, 1, p->mscal.d + 8, s);
         const double* xt[1] = {grad + n};
-        vec_dots(xt, xt, m, 1, w.dscal.p + 1, s);
-        HIP_CHECK(hipMemcpyAsync(w.hscal.p, w.dscal.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+        vec_dots(xt, xt, m, 1, p->mscal.d + 9, s);
         HIP_CHECK(hipStreamSynchronize(s));
-        *lr = w.hscal.p[0];
-        *mr = w.hscal.p[1];
+        *lr = p->mscal.h[8];
+        *mr = p->mscal.h[9];
     };
     plan_pass(0.0, 1.0, true);
     res->qrot = true;

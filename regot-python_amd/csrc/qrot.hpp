@@ -50,10 +50,9 @@ struct QrotHess {
 struct QrotScratch {
     DBuf<double> rowpart, colpart, sqpart, rsum, csum, out, spart, fpart, gpart;
     // rounding (qrot_primal): row / column scales, column errors, totals
-    DBuf<double> x, y, eb, scal, tot;
+    DBuf<double> x, y, eb, scal;
     DBuf<double> epart, cpart;   // per-workgroup sums of the folds
     DBuf<int> kpart, kprev, done, open;
-    HBuf<double> hout;
     HBuf<int> hopen;
     std::unique_ptr<QrotHess> hess;
     // M transposed (m x n, pitch ldt) for the column roots: a workspace of the
@@ -83,13 +82,11 @@ struct QrotScratch {
         kprev.alloc(c);
         done.alloc(c);
         open.alloc(1);
-        hout.ensure(2);
         hopen.ensure(1);
         x.alloc(n);
         y.alloc(m);
         eb.alloc(m);
         scal.alloc(sscal);
-        tot.alloc(2);
         epart.alloc(4 * static_cast<size_t>(ceil_div(static_cast<long>(n) + m, 64)));
         cpart.alloc(ceil_div(m, 64));
     }

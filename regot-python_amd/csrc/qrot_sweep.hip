@@ -470,15 +470,15 @@ double qrot_obj_grad(regot_problem* p, const double* gamma, double* grad, double
                        grad ? w.rsum.p : nullptr, w.csum.p, w.x.p,
                        grad && !(tau > 0.0) ? grad : nullptr, w.epart.p);
     hipLaunchKernelGGL(k_qrot_obj_total, dim3(1), dim3(256), 0, s, w.epart.p, ne, w.sqpart.p,
-                       g.strips * g.blocks, p->reg, tau, w.out.p);
+                       g.strips * g.blocks, p->reg, tau,
+                       grad && tau > 0.0 ? w.out.p : p->mscal.d);
     KERNEL_CHECK();
     if (grad && tau > 0.0)   // the gradient's tau term needs 1'alpha - 1'beta first
         launch_qrot_finish(alpha, beta, p->a, p->b, n, m, p->reg, tau, w.out.p + 2, w.rsum,
-                           w.csum, grad, w.fpart, w.gpart, w.out, s);
-    HIP_CHECK(hipMemcpyAsync(w.hout.p, w.out.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
+                           w.csum, grad, w.fpart, w.gpart, p->mscal.d, s);
     HIP_CHECK(hipStreamSynchronize(s));
-    if (gnorm2) *gnorm2 = w.hout.p[1];
-    return w.hout.p[0];
+    if (gnorm2) *gnorm2 = p->mscal.h[1];
+    return p->mscal.h[0];
 }
 
 double qrot_primal(regot_problem* p, const double* alpha, const double* beta, bool fresh)
@@ -506,11 +506,10 @@ double qrot_primal(regot_problem* p, const double* alpha, const double* beta, bo
     hipLaunchKernelGGL(k_qrot_rows_fold, dim3(nr), dim3(256), 0, s, w.rowpart.p, g.strips, p->a.p,
                        w.x.p, n, p->reg, w.epart.p);
     hipLaunchKernelGGL(k_qrot_round_total, dim3(1), dim3(256), 0, s, w.scal.p, g.strips * g.blocks,
-                       w.epart.p, nr, w.cpart.p, nc, p->reg, w.tot.p);
+                       w.epart.p, nr, w.cpart.p, nc, p->reg, p->mscal.d);
     KERNEL_CHECK();
-    HIP_CHECK(hipMemcpyAsync(w.hout.p, w.tot.p, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
-    return w.hout.p[0] + 0.5 * p->reg * w.hout.p[1];
+    return p->mscal.h[0] + 0.5 * p->reg * p->mscal.h[1];
 }
 
 }  // namespace regot

@@ -19,13 +19,6 @@ int set_error(int code, const char* what);
 
 namespace {
 
-// gamma = [alpha + beta_{m-1}; beta_{0..m-2} - beta_{m-1}]; src/sinkhorn_bcd.cpp:50-51
-void normalise_host(int n, int m, const double* alpha, const double* beta, double* gamma)
-{
-    for (int i = 0; i < n; i++) gamma[i] = alpha[i] + beta[m - 1];
-    for (int j = 0; j < m - 1; j++) gamma[n + j] = beta[j] - beta[m - 1];
-}
-
 // Plain Sinkhorn / BCD with the whole loop on the GPU.
 //
 // Semantics follow sinkhorn_bcd_internal, src/sinkhorn_bcd.cpp:14-124: init
@@ -72,7 +65,15 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     // With kernel profiling on, the iterations are enqueued exactly as
     // without it; each pass's events carry its iteration, and the launches
     // past the stop decision (which return at once) are dropped at the end.
-    const int K = o.bcd_batch > 0 ? o.bcd_batch : 8;
+    //
+    // Iterations per batch, two batches in flight.  A batch covers the host's
+    // turn-round (an event, two launches per iteration: some 40 us), and what
+    // is enqueued past the stop decision still has to drain, about 5 us per
+    // iteration: 8 iterations of 10 us, 4 of 21 us, 1 of 175 us.
+    const double it_us = 8.0 + static_cast<double>(n) * p->ldm *
+                                   (p->bulk == REGOT_F32 ? 4.0 : 8.0) / 5e6;
+    const int K = o.bcd_batch > 0 ? o.bcd_batch
+                                  : std::max(1, std::min(8, static_cast<int>(90.0 / it_us)));
     const int cap = std::max(4096, 4 * K + 8);
 
     if (!p->bcd) p->bcd = std::make_unique<BcdWork>();
@@ -82,20 +83,26 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     // (2048^2: 1.3x, 8192^2 and 32768 x 8192: 1.8x per solve)
     const bool fused_any = o.bcd_fused != 0 && p->bcd_fused_ok(false);
     const int nfb = fused_any ? bcd_fused_blocks(n, p->ncu) : 0;
+    if (!w.ap0.p) {
+        w.slab.add(w.ap0, n);
+        w.slab.add(w.ap1, n);
+        w.slab.add(w.be0, m);
+        w.slab.add(w.be1, m);
+        w.slab.add(w.gcol, m);
+        w.slab.add(w.rpart, 3L * std::max(nrb, nfb));
+        w.slab.add(w.cpart, 4L * p->ntiles);
+        w.slab.add(w.ctl, 4);
+        w.slab.add(w.stall, 4);
+        if (fused_any) w.slab.add(w.fpart, static_cast<size_t>(nfb) * bcd_part_pitch(m));
+        w.slab.make();
+    }
+    // a later solve may take the single-read form where the first did not
     if (fused_any) w.fpart.ensure(static_cast<size_t>(nfb) * bcd_part_pitch(m));
-    w.ap0.ensure(n);
-    w.ap1.ensure(n);
-    w.be0.ensure(m);
-    w.be1.ensure(m);
-    w.gcol.ensure(m);
     w.rpart.ensure(3L * std::max(nrb, nfb));
-    w.cpart.ensure(4L * p->ntiles);
-    w.ctl.ensure(4);
-    w.stall.ensure(4);
     w.hf.ensure(cap);
     w.hg.ensure(cap);
     w.hts.ensure(cap + 1);
-    w.hc.ensure(8);
+    w.stop.ensure(1);
     for (auto& e : w.ev)
         if (!e) HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 
@@ -110,17 +117,13 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
         ~FlagScope() { f = was; }
     };
 
-    std::vector<double> ah(n), bh(m);
-
     ColEpi c0;
     c0.resid = w.gcol;
     c0.tilepart = w.cpart;
     {
         FlagScope fs(p->precise, precise);
         if (o.x0) {
-            HIP_CHECK(hipMemcpyAsync(p->gamma, o.x0, (n + m - 1) * sizeof(double),
-                                     hipMemcpyHostToDevice, s));
-            launch_split_gamma(p->gamma, n, m, w.ap0, w.be0, s);
+            launch_split_gamma(p->stage(o.x0, n + m - 1L), n, m, w.ap0, w.be0, s);
             c0.colpot = w.be0;
             p->col_pass(w.ap0, w.be0, c0);
         } else {
@@ -129,7 +132,6 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             p->col_pass(w.ap0, nullptr, c0);
         }
     }
-    launch_stamp(w.hts.d + cap, s);
 
     BcdState st{};
     st.a = p->a;
@@ -150,6 +152,7 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     st.n = n;
     st.m = m;
     st.stall = w.stall;
+    st.stop = w.stop.d;
 
     const double tick_ms = p->wall_khz > 0 ? 1.0 / p->wall_khz : 0.0;
     int h_read = 0, niter = 0;
@@ -196,13 +199,9 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
         FlagScope fs(p->bcd_precise, precise);
         st.stall_window = (fp32 && !precise) ? kStallWindow : 0;
         st.tol = precise ? tol : tol_fp32;
-        // ctl = {0, k0, 0, 0}; both stall slots = {+inf, k0} (fill kernels,
-        // no memset nodes and no host synchronisation)
-        launch_fill_int(w.ctl, 0, 4, s);
-        launch_fill_int(w.ctl.p + 1, k0, 1, s);
-        launch_fill(w.stall, static_cast<double>(k0), 4, s);
-        launch_fill(w.stall.p, HUGE_VAL, 1, s);
-        launch_fill(w.stall.p + 2, HUGE_VAL, 1, s);
+        // (the first run also stamps the end of the set-up)
+        w.stop.h[0] = 0;   // the stream holds no launch that writes it
+        launch_bcd_begin(w.ctl, w.stall, k0, precise ? nullptr : w.hts.d + cap, s);
         // alpha_k and beta_k live in the buffers of parity k & 1; iteration k
         // writes alpha_{k+1} and beta_{k+1} to the others
         int k_enq = k0;
@@ -232,10 +231,10 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             p->row_pass_bcd(bk, e, st);
             p->col_pass(ak1, bk, c, w.ctl, &st);
         };
+        int k_end[2] = {k0, k0};   // iterations enqueued up to each batch's event
         auto launch_batch = [&](int slot) {
             for (int it = 0; it < K && k_enq <= max_iter; it++) enqueue_iteration();
-            HIP_CHECK(hipMemcpyAsync(w.hc.p + 4 * slot, w.ctl.p, 4 * sizeof(int),
-                                     hipMemcpyDeviceToHost, s));
+            k_end[slot] = k_enq;
             HIP_CHECK(hipEventRecord(w.ev[slot], s));
         };
         std::deque<int> q;
@@ -248,9 +247,14 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             const int slot = q.front();
             q.pop_front();
             HIP_CHECK(hipEventSynchronize(w.ev[slot]));
-            const int* c = w.hc.p + 4 * slot;
-            const bool done = c[0] != 0;
-            const int avail = done ? c[2] + 1 : c[1];
+            // what this batch has written is visible now; a stop word of a
+            // later one (its history may not be) waits for that batch's event
+            const unsigned long long word =
+                *reinterpret_cast<volatile unsigned long long*>(w.stop.h);
+            const int c[3] = {static_cast<int>(word >> 32), 0,
+                              static_cast<int>(word & 0xffffffffu)};
+            const bool done = word != 0 && c[2] < k_end[slot];
+            const int avail = done ? c[2] + 1 : k_end[slot];
             if (h_read == 0 && avail > 0) ts_init = w.hts.h[cap];
             for (; h_read < avail; h_read++) {
                 const int h = h_read % cap;
@@ -319,14 +323,11 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     }
     if (p->prof) p->prof_commit(niter);
 
-    HIP_CHECK(hipMemcpyAsync(ah.data(), (niter & 1) ? w.ap1.p : w.ap0.p, n * sizeof(double),
-                             hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipMemcpyAsync(bh.data(), (niter & 1) ? w.be1.p : w.be0.p, m * sizeof(double),
-                             hipMemcpyDeviceToHost, s));
+    vec_normalise((niter & 1) ? w.ap1 : w.ap0, (niter & 1) ? w.be1 : w.be0, n, m,
+                  p->stage_out(n + m - 1L), s);
     p->sync();
     res->niter = niter;
-    res->dual.resize(n + m - 1);
-    normalise_host(n, m, ah.data(), bh.data(), res->dual.data());
+    res->dual.assign(p->hout, p->hout + (n + m - 1));
 }
 
 }  // namespace

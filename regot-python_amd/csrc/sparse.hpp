@@ -71,8 +71,7 @@ struct SparseHessian {
     // the second right-hand side of a paired CG (hess_cg2): the same state
     DBuf<double> cg1_r, cg1_p, cg1_q, cg1_s, cg1_u, cg1_y, cg1_part, cg1_scal, cg1_rhs;
     DBuf<int> cg1_ctl;
-    HBuf<int> cg1_hctl;
-    HBuf<double> hbuf1;
+    MappedRing<double> cg1_rep;
     // Matrix-free build (FP32 bulk): no CSR / CSC; the kept entries as the
     // dense FP32 matrix mf_t (K_ij = T_ij where kept, else 0; row pitch
     // mf_ldt) and every product is a pass over it by mf_nwg workgroups,
@@ -82,8 +81,17 @@ struct SparseHessian {
     long mf_ldt = 0;
     DBuf<float> mf_t;
     DBuf<double> mf_part;
-    HBuf<int> cg_hctl;
-    HBuf<double> hbuf;
+    // host-visible outcome of a CG (k_cg_end); [0] is set when it stops
+    MappedRing<double> cg_rep;
+    hipEvent_t cg_ev[2] = {nullptr, nullptr};
+    SparseHessian() = default;
+    SparseHessian(const SparseHessian&) = delete;
+    SparseHessian& operator=(const SparseHessian&) = delete;
+    ~SparseHessian()
+    {
+        for (auto& e : cg_ev)
+            if (e) (void)hipEventDestroy(e);
+    }
     HBuf<long long> hll;
     double density() const
     {

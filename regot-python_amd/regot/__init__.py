@@ -470,7 +470,8 @@ class Problem:
 
     def profile_stats(self, kind):
         """(launches, total ms) of kind 0 = row pass, 1 = column pass, 2 = single-read
-        BCD pass, 3 = its column-sum combine."""
+        BCD pass, 3 = its column-sum combine, 4 and 5 = the same two in FP64
+        arithmetic."""
         cnt = _lib.ctypes.c_longlong()
         ms = _lib.ctypes.c_double()
         check(lib().regot_profile_get(self._h, int(kind), _lib.ctypes.byref(cnt),
