@@ -77,24 +77,30 @@ __device__ __forceinline__ void exp2_tab_load(double* lds)
 // 64 k instead: scaling by a power of two commutes with every rounding (no
 // overflow or underflow at these magnitudes), so y is exactly 64 x and the
 // result is bit for bit dexp2(x).  Then k = rint(y) comes from the
-// 1.5 * 2^52 shifter (one add; |y| < 2^51 after the clamp, ties to even as
-// rint; the low word of the sum is k), and the polynomial runs on
+// 1.5 * 2^52 shifter (one add; |y| < 2^51, ties to even as rint; the low word
+// of the sum is k while |k| < 2^31), and the polynomial runs on
 // d = y - k = 64 f (exact) with the coefficients scaled by 64^-n, which again
 // changes no rounding.
-__device__ __forceinline__ double dexp2_64(double y, const double* tab)
+// The method proper, for |y| < kExp2Fast or a NaN, which comes out as a NaN.
+constexpr double kExp2Fast = 0x1p31;
+__device__ __forceinline__ double dexp2_64_fast(double y, const double* tab)
 {
     constexpr double c1 = 0x1.62e42fefa39efp-1 * 0x1p-6, c2 = 0x1.ebfbdff82c58fp-3 * 0x1p-12;
     constexpr double c3 = 0x1.c6b08d704a0c0p-5 * 0x1p-18, c4 = 0x1.3b2ab6fba4e77p-7 * 0x1p-24;
     constexpr double c5 = 0x1.5d87fe78a6731p-10 * 0x1p-30, c6 = 0x1.430912f86c787p-13 * 0x1p-36;
-    // clamp: beyond +-1100 * 64 the result is already 0 or +inf (NaN last)
-    const double yc = fmin(fmax(y, -70400.0), 70400.0);
-    const double sh = yc + 0x1.8p52;
+    const double sh = y + 0x1.8p52;
     const double kx = sh - 0x1.8p52;
     const int i = __double2loint(sh);
-    const double d = yc - kx;
+    const double d = y - kx;
     const double q = d * (c1 + d * (c2 + d * (c3 + d * (c4 + d * (c5 + d * c6)))));
     const double2 t = *reinterpret_cast<const double2*>(tab + 2 * (i & 63));
-    const double r = ldexp(t.x + fma(t.x, q, t.y), i >> 6);
+    return ldexp(t.x + fma(t.x, q, t.y), i >> 6);
+}
+
+__device__ __forceinline__ double dexp2_64(double y, const double* tab)
+{
+    // clamp: beyond +-1100 * 64 the result is already 0 or +inf (NaN last)
+    const double r = dexp2_64_fast(fmin(fmax(y, -70400.0), 70400.0), tab);
     // a NaN argument gives a quiet NaN (exponent all ones, top mantissa bit set)
     return __hiloint2double((y != y) ? 0x7ff80000 : __double2hiint(r), __double2loint(r));
 }

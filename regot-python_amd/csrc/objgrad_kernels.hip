@@ -13,8 +13,8 @@
 // Tiling: a workgroup owns a 256-column strip of a block of rows; each lane
 // owns 4 adjacent columns and the 4 waves take the block's rows round robin
 // (coalesced row segments).  Row sums are reduced
-// across the wave per row and written per strip, column sums accumulate per
-// lane down the block and are merged through LDS per block; two small
+// across the wave eight rows at a time and written per strip, column sums
+// accumulate per lane down the block and are merged through LDS per block; two small
 // kernels fold strips, blocks and the scalars in a fixed order.
 #include <algorithm>
 
@@ -28,27 +28,49 @@ namespace {
 // Wave sum by DPP and shuffle steps (the same bits on every lane).
 __device__ __forceinline__ double wsum(double v) { return dev::group_sum<64>(v); }
 
-__device__ __forceinline__ void ldm4(const float* p, int c0, int m, double (&v)[4])
+// Columns per lane.  8 would spread each row's wave sum over twice the
+// elements but needs 88 VGPRs, 5 waves per SIMD: measured slower (objective
+// call at 16384^2 316 against 297 us, at 4096^2 61.5 against 51.0 us, with the
+// wave sum per row).
+constexpr int kCPL = 4;
+constexpr int kStrip = 64 * kCPL;     // columns per workgroup strip
+
+// Rows of a wave whose sums are formed together, and the pitch in doubles of
+// their lane sums in LDS: 528 bytes put the 64 reads of 16 bytes of a
+// reduction step on all banks evenly.
+constexpr int kRowsTog = 8;
+constexpr int kLanePitch = 66;
+
+template <bool NT, typename V>
+__device__ __forceinline__ V ldv(const V* p)
 {
-    if (c0 + 3 < m) {
+    return NT ? __builtin_nontemporal_load(p) : *p;
+}
+
+// Four columns of a row from c0 on; FULL: all of them are inside the matrix.
+template <bool FULL, bool NT>
+__device__ __forceinline__ void ldm4(const float* p, int c0, int m, float (&v)[4])
+{
+    if (FULL || c0 + 3 < m) {
         typedef float f4 __attribute__((ext_vector_type(4)));
-        const f4 u = __builtin_nontemporal_load(reinterpret_cast<const f4*>(p + c0));
+        const f4 u = ldv<NT>(reinterpret_cast<const f4*>(p + c0));
         v[0] = u.x;
         v[1] = u.y;
         v[2] = u.z;
         v[3] = u.w;
     } else {
 #pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = (c0 + q < m) ? static_cast<double>(p[c0 + q]) : 0.0;
+        for (int q = 0; q < 4; q++) v[q] = (c0 + q < m) ? p[c0 + q] : 0.f;
     }
 }
 
+template <bool FULL, bool NT>
 __device__ __forceinline__ void ldm4(const double* p, int c0, int m, double (&v)[4])
 {
-    if (c0 + 3 < m) {
+    if (FULL || c0 + 3 < m) {
         typedef double d2 __attribute__((ext_vector_type(2)));
-        const d2 u0 = __builtin_nontemporal_load(reinterpret_cast<const d2*>(p + c0));
-        const d2 u1 = __builtin_nontemporal_load(reinterpret_cast<const d2*>(p + c0 + 2));
+        const d2 u0 = ldv<NT>(reinterpret_cast<const d2*>(p + c0));
+        const d2 u1 = ldv<NT>(reinterpret_cast<const d2*>(p + c0 + 2));
         v[0] = u0.x;
         v[1] = u0.y;
         v[2] = u1.x;
@@ -59,57 +81,99 @@ __device__ __forceinline__ void ldm4(const double* p, int c0, int m, double (&v)
     }
 }
 
-// Columns per lane.  8 would spread each row's wave sum over twice the
-// elements (27.5 instead of 30 VALU instructions per element) but needs 88
-// VGPRs, 5 waves per SIMD instead of 8: measured slower (objective call at
-// 16384^2 316 against 297 us, at 4096^2 61.5 against 51.0 us).
-constexpr int kCPL = 4;
-constexpr int kStrip = 64 * kCPL;     // columns per workgroup strip
+// alpha k64 + bk: one rounding on full strips, two on a ragged last one.  (The
+// two forms agree to an ulp; which one is used is fixed here because an L-BFGS
+// path follows the last bit.)
+template <bool FULL>
+__device__ __forceinline__ double row_col(double alpha, double k64, double bk)
+{
+#pragma clang fp contract(off)
+    if (FULL) return fma(alpha, k64, bk);
+    const double ak = alpha * k64;
+    return ak + bk;
+}
 
-// The rows of one tile: FULL = every column of the strip is inside the
-// matrix (no per-element bounds), WT = weights x, y present.
-template <typename TM, bool FULL, bool WT>
+// The rows r, r + 4, ... < r1 of one tile (r the same on the whole wave):
+// FULL = every column of the strip is inside the matrix (no per-element
+// bounds), WT = weights x, y present.  Eight rows at a time: each lane leaves
+// its four-column sum of every row in the wave's own LDS (lw), then lane 8 q + s
+// adds row q's sums of lanes 8 s .. 8 s + 7 and three DPP steps finish the
+// eight rows together: 16 VALU instructions for what took 18 per row, with
+// the same pairing of lanes (1, 2, 4 apart, then 8, 16, 32) and so the same
+// bits.
+template <typename TM, bool FULL, bool WT, bool NT>
 __device__ __forceinline__ void sums_rows_loop(const TM* __restrict__ M, long ldm, int n, int m,
                                                const double* __restrict__ alpha, double k64,
                                                const double* __restrict__ xw, int c0, int r, int r1,
                                                int strip, const double (&bk)[kCPL],
                                                const double (&yq)[kCPL], const double* tab,
-                                               double (&cs)[kCPL], double* __restrict__ rowpart)
+                                               double* lw, double (&cs)[kCPL],
+                                               double* __restrict__ rowpart)
 {
+    // Two rows per trip take turns in the two buffers.  That costs 10 more VGPRs
+    // (70, 7 waves per SIMD): 210 against 235 us at 16384^2 FP32, where the issue
+    // rate bounds, but 136 against 126 us at 8192^2 FP64, where the read does.
+    constexpr int PAIR = (sizeof(TM) == 4 && !WT) ? 2 : 1;
     const int lane = threadIdx.x & 63;
-    for (; r < r1; r += 4) {
-        double mv[kCPL];
+    TM mv[2][kCPL];   // this row and the wave's next
+    if (r < r1) ldm4<FULL, NT>(M + r * ldm, c0, m, mv[0]);
+    for (; r < r1; r += 4 * kRowsTog) {
+        const int cnt = min(kRowsTog, (r1 - r + 3) >> 2);
+        // alpha of the eight rows on lanes 0 .. 7
+        const double al = alpha[r + 4 * min(lane & 7, cnt - 1)];
+#pragma unroll 1
+        for (int h0 = 0; h0 < cnt; h0 += PAIR)
 #pragma unroll
-        for (int h = 0; h < kCPL; h += 4) {
-            double v4[4];
-            if (FULL && sizeof(TM) == 4) {
-                typedef float f4 __attribute__((ext_vector_type(4)));
-                const f4 u = __builtin_nontemporal_load(reinterpret_cast<const f4*>(
-                    reinterpret_cast<const float*>(M) + r * ldm + c0 + h));
-                v4[0] = u.x;
-                v4[1] = u.y;
-                v4[2] = u.z;
-                v4[3] = u.w;
-            } else {
-                ldm4(M + static_cast<long>(r) * ldm, c0 + h, m, v4);
-            }
+        for (int u = 0; u < PAIR; u++) {
+            const int h = h0 + u;
+            if (h >= cnt) break;   // wave-uniform
+            // (the last row reads itself again)
+            const int i = r + 4 * h;
+            ldm4<FULL, NT>(M + static_cast<long>(i + 4 < r1 ? i + 4 : i) * ldm, c0, m, mv[1 - u]);
+            const double ai = __hiloint2double(
+                __builtin_amdgcn_readlane(__double2hiint(al), h),
+                __builtin_amdgcn_readlane(__double2loint(al), h));
+            double y[kCPL];
+            bool far = false;
 #pragma unroll
-            for (int q = 0; q < 4; q++) mv[h + q] = v4[q];
-        }
-        const double ak = alpha[r] * k64;
-        double rs = 0.0;
-#pragma unroll
-        for (int q = 0; q < kCPL; q++) {
-            if (FULL || c0 + q < m) {
+            for (int q = 0; q < kCPL; q++) {
                 // 64 (alpha_i + beta_j - M_ij) / reg in log2 units
-                double t = dev::dexp2_64(fma(-k64, mv[q], ak + bk[q]), tab);
-                if (WT) t *= (xw ? xw[r] : 1.0) * yq[q];
-                rs += t;
-                cs[q] += t;
+                y[q] = fma(-k64, static_cast<double>(mv[u][q]), row_col<FULL>(ai, k64, bk[q]));
+                far = far || fabs(y[q]) >= dev::kExp2Fast;
             }
+            if (__any(far)) {   // wave-uniform; NaN stays
+#pragma unroll
+                for (int q = 0; q < kCPL; q++) {
+                    const double c = fmin(fmax(y[q], -70400.0), 70400.0);
+                    y[q] = (y[q] != y[q]) ? y[q] : c;
+                }
+            }
+            double rs = 0.0;
+#pragma unroll
+            for (int q = 0; q < kCPL; q++) {
+                if (FULL || c0 + q < m) {
+                    double t = dev::dexp2_64_fast(y[q], tab);
+                    if (WT) t *= (xw ? xw[i] : 1.0) * yq[q];
+                    rs = (q == 0 && !WT) ? t : rs + t;
+                    cs[q] += t;
+                }
+            }
+            lw[h * kLanePitch + lane] = rs;
+            if (PAIR == 1)
+#pragma unroll
+                for (int q = 0; q < kCPL; q++) mv[0][q] = mv[1][q];
         }
-        rs = wsum(rs);
-        if (lane == 0) rowpart[static_cast<long>(strip) * n + r] = rs;
+        // the wave's LDS stores and loads stay in program order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const int row = lane >> 3, seg = lane & 7;
+        const double2* src = reinterpret_cast<const double2*>(lw + row * kLanePitch + 8 * seg);
+        const double2 x0 = src[0], x1 = src[1], x2 = src[2], x3 = src[3];
+        double s = ((x0.x + x0.y) + (x1.x + x1.y)) + ((x2.x + x2.y) + (x3.x + x3.y));
+        s = dev::group_sum<8>(s);
+        if (seg == 0 && row < cnt) rowpart[static_cast<long>(strip) * n + r + 4 * row] = s;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
@@ -117,10 +181,17 @@ __device__ __forceinline__ void sums_rows_loop(const TM* __restrict__ M, long ld
 // beta has m entries (beta_{m-1} = 0).  Sums of w_ij = x_i T_ij y_j (WT:
 // weights given, else 1): rowpart[strip * n + i] = sum of row i over the
 // strip; colpart[block * m + j] (when non-null) = sum of column j over the
-// block.  Each lane owns kCPL adjacent columns.  (Loading the next row's M
-// ahead measured 5% slower: more registers, lower occupancy.)
-template <typename TM, bool WT>
-__global__ __launch_bounds__(256) void k_sums_tile(const TM* __restrict__ M, long ldm, int n, int m,
+// block.  Each lane owns kCPL adjacent columns.
+//
+// Bound by the FP64 issue rate: at 16384^2 FP32 254 us at 30 VALU instructions
+// per element, now 210 at 22.5 (84% of the cycles issue VALU, at the 2.0 GHz the
+// card holds under FP64 load; the read of M alone takes 165 us).  What went: the
+// wave sum per row (4 of the 30; see sums_rows_loop), the clamps and the NaN
+// select of every exponential (3; now one test per row and the clamp on a branch),
+// register moves.  At 4096^2 FP64 (134 MB) an evaluation call takes 53 us, before
+// 72 with 15 us of that host round trips.
+template <typename TM, bool WT, bool NT>
+__global__ __launch_bounds__(256, WT ? 5 : 7) void k_sums_tile(const TM* __restrict__ M, long ldm, int n, int m,
                                                    const double* __restrict__ alpha,
                                                    const double* __restrict__ beta, double k,
                                                    int rows, const double* __restrict__ xw,
@@ -128,11 +199,13 @@ __global__ __launch_bounds__(256) void k_sums_tile(const TM* __restrict__ M, lon
                                                    double* __restrict__ rowpart,
                                                    double* __restrict__ colpart)
 {
-    __shared__ double sm[4][kStrip];
+    // the waves' lane sums (kRowsTog kLanePitch each), then their column sums
+    static_assert(kRowsTog * kLanePitch >= kStrip, "column sums take the same room");
+    __shared__ __align__(16) double sm[4][kRowsTog * kLanePitch];
     __shared__ __align__(16) double tab[128];
     dev::exp2_tab_load(tab);
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int strip = blockIdx.x, blk = blockIdx.y;
     const int c0 = strip * kStrip + lane * kCPL;
     const int r0 = blk * rows;
@@ -142,16 +215,19 @@ __global__ __launch_bounds__(256) void k_sums_tile(const TM* __restrict__ M, lon
     double bk[kCPL], yq[kCPL], cs[kCPL];
 #pragma unroll
     for (int q = 0; q < kCPL; q++) {
-        bk[q] = (c0 + q < m) ? beta[c0 + q] * k64 : 0.0;
-        yq[q] = (WT && yw && c0 + q < m) ? yw[c0 + q] : 1.0;
+        // (clamped, not skipped: the loads go out together)
+        const int j = min(c0 + q, m - 1);
+        const double bj = beta[j];
+        bk[q] = (c0 + q < m) ? bj * k64 : 0.0;
+        yq[q] = (WT && yw) ? yw[j] : 1.0;
         cs[q] = 0.0;
     }
     if ((strip + 1) * kStrip <= m)   // workgroup-uniform
-        sums_rows_loop<TM, true, WT>(M, ldm, n, m, alpha, k64, xw, c0, r0 + wave, r1, strip, bk,
-                                     yq, tab, cs, rowpart);
+        sums_rows_loop<TM, true, WT, NT>(M, ldm, n, m, alpha, k64, xw, c0, r0 + wave, r1, strip,
+                                         bk, yq, tab, sm[wave], cs, rowpart);
     else
-        sums_rows_loop<TM, false, WT>(M, ldm, n, m, alpha, k64, xw, c0, r0 + wave, r1, strip,
-                                      bk, yq, tab, cs, rowpart);
+        sums_rows_loop<TM, false, WT, NT>(M, ldm, n, m, alpha, k64, xw, c0, r0 + wave, r1, strip,
+                                          bk, yq, tab, sm[wave], cs, rowpart);
     if (!colpart) return;   // grid-uniform
 #pragma unroll
     for (int q = 0; q < kCPL; q++) sm[wave][lane * kCPL + q] = cs[q];
@@ -299,6 +375,32 @@ void sums_scratch_sizes(int n, int m, long* rowpart, long* colpart, long* part)
     *part = 4L * ceil_div(std::max(n, m), 256);
 }
 
+// NT: a matrix that does not fit the 256 MB last-level cache is streamed.
+template <typename TM, bool WT>
+static void launch_sums_tile_t(const void* M, long ldm, int n, int m, const double* alpha,
+                               const double* beta, double k, int rows, const double* x,
+                               const double* y, double* rowpart, double* colpart, hipStream_t s)
+{
+    const dim3 grid(ceil_div(m, kStrip), ceil_div(n, rows));
+    const bool nt = static_cast<double>(n) * ldm * sizeof(TM) > 256e6;
+    hipLaunchKernelGGL((nt ? k_sums_tile<TM, WT, true> : k_sums_tile<TM, WT, false>), grid, dim3(256),
+                       0, s, static_cast<const TM*>(M), ldm, n, m, alpha, beta, k, rows, x, y,
+                       rowpart, colpart);
+}
+
+template <bool WT>
+static void launch_sums_tile(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
+                             const double* beta, double k, int rows, const double* x,
+                             const double* y, double* rowpart, double* colpart, hipStream_t s)
+{
+    if (bulk == 0)
+        launch_sums_tile_t<float, WT>(M, ldm, n, m, alpha, beta, k, rows, x, y, rowpart, colpart,
+                                      s);
+    else
+        launch_sums_tile_t<double, WT>(M, ldm, n, m, alpha, beta, k, rows, x, y, rowpart, colpart,
+                                       s);
+}
+
 void launch_objgrad_fused(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
                           const double* beta, const double* a, const double* b, double reg,
                           bool with_grad, double* grad, double* rowpart, double* colpart,
@@ -308,17 +410,10 @@ void launch_objgrad_fused(int bulk, const void* M, long ldm, int n, int m, const
     const int nstrip = ceil_div(m, kStrip);
     const int rows = sums_rows(n, m);
     const int nblk = ceil_div(n, rows);
-    const dim3 grid(nstrip, nblk);
     const double k = 1.4426950408889634074 / reg;
     double* cp = with_grad ? colpart : nullptr;
-    if (bulk == 0)
-        hipLaunchKernelGGL((k_sums_tile<float, false>), grid, dim3(256), 0, s,
-                           static_cast<const float*>(M), ldm, n, m, alpha, beta, k, rows, nullptr,
-                           nullptr, rowpart, cp);
-    else
-        hipLaunchKernelGGL((k_sums_tile<double, false>), grid, dim3(256), 0, s,
-                           static_cast<const double*>(M), ldm, n, m, alpha, beta, k, rows,
-                           nullptr, nullptr, rowpart, cp);
+    launch_sums_tile<false>(bulk, M, ldm, n, m, alpha, beta, k, rows, nullptr, nullptr, rowpart, cp,
+                            s);
     KERNEL_CHECK();
     const int nf = ceil_div(std::max(n, m), 256);
     hipLaunchKernelGGL(k_sums_fold, dim3(nf), dim3(256), 0, s, rowpart, nstrip, cp, nblk, alpha,
@@ -334,25 +429,12 @@ void launch_wsums(int bulk, const void* M, long ldm, int n, int m, const double*
 {
     if (n <= 0 || m <= 0) fail(E_INVALID, "weighted sums on an empty problem");
     const int rows = sums_rows(n, m);
-    const dim3 grid(ceil_div(m, kStrip), ceil_div(n, rows));
     const double k = 1.4426950408889634074 / reg;
-    const bool wt = x || y;
-    if (bulk == 0 && wt)
-        hipLaunchKernelGGL((k_sums_tile<float, true>), grid, dim3(256), 0, s,
-                           static_cast<const float*>(M), ldm, n, m, alpha, beta, k, rows, x, y,
-                           rowpart, colpart);
-    else if (bulk == 0)
-        hipLaunchKernelGGL((k_sums_tile<float, false>), grid, dim3(256), 0, s,
-                           static_cast<const float*>(M), ldm, n, m, alpha, beta, k, rows, x, y,
-                           rowpart, colpart);
-    else if (wt)
-        hipLaunchKernelGGL((k_sums_tile<double, true>), grid, dim3(256), 0, s,
-                           static_cast<const double*>(M), ldm, n, m, alpha, beta, k, rows, x, y,
-                           rowpart, colpart);
+    if (x || y)
+        launch_sums_tile<true>(bulk, M, ldm, n, m, alpha, beta, k, rows, x, y, rowpart, colpart, s);
     else
-        hipLaunchKernelGGL((k_sums_tile<double, false>), grid, dim3(256), 0, s,
-                           static_cast<const double*>(M), ldm, n, m, alpha, beta, k, rows, x, y,
-                           rowpart, colpart);
+        launch_sums_tile<false>(bulk, M, ldm, n, m, alpha, beta, k, rows, nullptr, nullptr, rowpart,
+                                colpart, s);
     KERNEL_CHECK();
 }
 

@@ -204,3 +204,47 @@ def test_device_fp64_log_accuracy(gpu_lib):
     _lib.check(_lib.lib().regot_check_log(_lib.dptr(z), _lib.dptr(w), len(z), 0))
     assert w[0] == -np.inf and w[1] == -np.inf and w[2] == np.inf
     assert np.all(np.isnan(w[3:]))
+
+
+@pytest.mark.parametrize("n,m", [(1, 1), (3, 256), (33, 255), (67, 513), (131, 1024), (257, 1030)])
+def test_obj_grad_tile_edges(gpu_lib, n, m):
+    """The one-pass evaluation at the edges of its tiles (256 columns, 32 rows, 8
+    rows of a wave together), in FP64."""
+    rng = np.random.default_rng(1000 * n + m)
+    M = rng.random((n, m))
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    reg = 0.05
+    gamma = 0.1 * rng.standard_normal(n + m - 1) - 0.2
+    beta = np.append(gamma[n:], 0.0)
+    x = (gamma[:n, None] + beta[None, :] - M) / reg
+    T = np.exp(x.astype(np.longdouble))
+    with gpu_lib.Problem(M, a, b, reg, bulk="fp64") as P:
+        f, g = P.dual_obj_grad(gamma)
+    # three roundings of the argument, an ulp or two of exp, the summation
+    tol = (4.0 * np.abs(x).max() + n + m + 8) * 2.0 ** -52
+    rs, cs = T.sum(1), T.sum(0)
+    assert np.all(np.abs(g[:n] - (rs - a)) <= tol * (rs + a))
+    assert np.all(np.abs(g[n:] - (cs - b)[:-1]) <= tol * (cs + b)[:-1])
+    parts = [reg * T.sum(), gamma[:n] @ a, beta @ b]
+    size = reg * T.sum() + np.abs(gamma[:n]) @ a + np.abs(beta) @ b
+    assert abs(f - (parts[0] - parts[1] - parts[2])) <= tol * size
+
+
+def test_obj_grad_far_arguments(gpu_lib):
+    """Exponents beyond 2^31 / 64 are 0 or inf, as exp gives them, and a NaN stays
+    in its own row and column."""
+    n, m = 40, 300
+    M = np.random.default_rng(0).random((n, m))
+    M[3, :] = 1e12        # far below: this row is 0
+    M[:, 7] = 1e12        # and this column
+    M[5, 11] = -1e12      # far above: inf
+    M[20, 100] = np.nan
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    with gpu_lib.Problem(M, a, b, 1.0, bulk="fp64") as P:
+        _, g = P.dual_obj_grad(np.zeros(n + m - 1))
+    T = np.exp(-M)
+    want = np.concatenate([T.sum(1) - a, (T.sum(0) - b)[:-1]])
+    assert np.array_equal(np.isnan(g), np.isnan(want))
+    assert np.array_equal(np.isinf(g), np.isinf(want))
+    ok = np.isfinite(want)
+    assert np.allclose(g[ok], want[ok], rtol=(n + m) * 2.0 ** -52, atol=1e-13)
