@@ -5,6 +5,7 @@
 #include <deque>
 #include <vector>
 
+#include "cg.hpp"
 #include "dense_device.hpp"
 #include "hess_mf.hpp"
 #include "hessian.hpp"
@@ -62,32 +63,6 @@ __global__ void k_sub_div(const double* w, const double* y, const double* h1, do
 // ctl: [0] done, [1] iterations when done.  scal: [0..1] alpha by parity,
 // [2..3] gamma by parity, [4] r.r of the last update, [5] stop threshold,
 // [6] rhs norm^2.
-struct CgArgs {
-    const int* rowptr;
-    const int* colind;
-    const double* rval;
-    const int* colptr;
-    const int* rowind;
-    const double* cval;
-    const double* h1;
-    const double* h2;
-    double shift;
-    int n, m1;
-    double* x;
-    double* r;
-    double* p;
-    double* s;
-    double* w;
-    double* u;
-    double* y;      // n
-    double* part;   // [2 nbc] r.u, w.u per column workgroup; [nbu] r.r per update workgroup
-    double* scal;
-    int* ctl;
-    int nbc;        // column workgroups
-    int nbu;        // update workgroups (256 entries each)
-    const double* dinv;   // Jacobi preconditioner, or null
-    double* rep;          // host-visible: rep[0] = 1 on stop
-};
 
 // dinv_j = 1 / (h2_j + shift - sum_i sigma_ij^2 / (h1_i + shift)), the diagonal
 // of Delta (>= shift since sigma_ij <= h1_i and sum_i sigma_ij <= h2_j); one
@@ -566,6 +541,7 @@ static void prepare(regot_problem* p, SparseHessian& H, const double* d_gamma, c
     H.rcnt.ensure(n + 1);   // also receives an (n+1)-entry scan
     H.zcnt.ensure(n);
     H.mf = false;
+    H.compact = false;
     launch_split_gamma(d_gamma, n, m, H.vn, H.vm, s);
     hipLaunchKernelGGL(k_hess_diag, dim3(ceil_div(std::max(n, m), 256)), dim3(256), 0, s, d_grad,
                        p->a.p, p->b.p, n, m, p->reg, H.h1.p, H.h2.p);
@@ -796,6 +772,41 @@ struct CgSide {
     CgArgs a;
 };
 
+// Stored entries from which the products keep their vector in LDS.  Below, the
+// copy of the vector costs more than the gathers: a solve of some 20 iterations
+// took per iteration, its set-up and copies included, from global memory and
+// from LDS: 0.72 M entries (6000^2 FP32) 35.8 and 37.0 us, 1.34 M (8192^2) 56.3
+// and 44.7, 1.80 M (6000^2) 49.3 and 38.9, 2.25 M (15000^2) 99.7 and 72.7, in
+// FP64 1.34 M (8192^2) 55.7 and 49.0.
+constexpr long long kCgLdsMin = 1000000;
+
+// What the products of cg_lds.hip read, formed once per build.  False: FP32
+// bulk and no memory for the compact copies (12 bytes per entry).
+static bool cg_entries(regot_problem* p, SparseHessian& H, CgEntries* e)
+{
+    if (p->bulk != 0) return true;
+    if (!H.compact) {
+        try {
+            H.rval32.ensure(H.nnz);
+            H.cval32.ensure(H.nnz);
+            H.colind16.ensure(H.nnz);
+            H.rowind16.ensure(H.nnz);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            return false;
+        }
+        launch_cg_compact(H.rval, H.colind, H.nnz, p->reg, H.rval32, H.colind16, p->stream);
+        launch_cg_compact(H.cval, H.rowind, H.nnz, p->reg, H.cval32, H.rowind16, p->stream);
+        H.compact = true;
+    }
+    e->rval32 = H.rval32;
+    e->cval32 = H.cval32;
+    e->colind16 = H.colind16;
+    e->rowind16 = H.rowind16;
+    e->scale = 1.0 / p->reg;
+    return true;
+}
+
 // CG on Delta for nr (1 or 2) right-hand sides, each to its own stop rule
 // ||r||^2 < max(tol^2 ||rhs||^2, DBL_MIN) and cap (Eigen's counting, the
 // converged update not counted; src/sinkhorn_cg.cpp:29-38).  Two sides run
@@ -835,6 +846,11 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
         }
     }
     const double* dinv = jacobi ? H.cg_dinv.p : nullptr;
+    CgEntries ent;
+    // the kernels of cg_lds.hip are the 64-lane form
+    const bool lds = !H.mf && (lpr_r == 64 || lpr_c == 64) && H.nnz >= kCgLdsMin &&
+                     cg_lds_ok(n, m1, p->ncu) && cg_entries(p, H, &ent);
+    const bool lds_r = lds && lpr_r == 64, lds_c = lds && lpr_c == 64;
 
     // per side: x = x0 (or 0), r = rhs - Delta x, u = D^-1 r (or r),
     // w = Delta u (in q), p = s = 0 (beta_0 = 0)
@@ -930,8 +946,14 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
                 hipLaunchKernelGGL(k_cg_cols_mf, dim3(nbc), dim3(256), 0, s, a0, H.mf_part.p,
                                    H.mf_nwg);
             } else {
-                cg_rows(lpr_r, a0, a1, nr, s);
-                cg_cols(lpr_c, a0, a1, nr, k_enq, s);
+                if (lds_r)
+                    launch_cg_rows_lds(a0, a1, ent, nr, p->ncu, s);
+                else
+                    cg_rows(lpr_r, a0, a1, nr, s);
+                if (lds_c)
+                    launch_cg_cols_lds(a0, a1, ent, nr, k_enq, p->ncu, s);
+                else
+                    cg_cols(lpr_c, a0, a1, nr, k_enq, s);
             }
         }
         KERNEL_CHECK();

@@ -52,6 +52,11 @@ struct SparseHessian {
     DBuf<double> h1, h2;
     DBuf<int> rowptr, colind, colptr, rowind;
     DBuf<double> rval, cval;
+    // the entries as the large CG products read them (CgEntries), valid while
+    // compact is set
+    DBuf<float> rval32, cval32;
+    DBuf<unsigned short> colind16, rowind16;
+    bool compact = false;
     // work
     DBuf<double> tau, rho;
     DBuf<int> rcnt, ccnt, zcnt, csc_work;

@@ -93,3 +93,44 @@ def test_cg_pair_matrix_free_runs_two_solves(gpu_lib):
         pr = P.hess_cg2(r0, r1, shift, tol=1e-10, max_iter=5000)
     same(s0, pr, 0)
     same(s1, pr, 1)
+
+
+@pytest.mark.parametrize("bulk,n,m,density", [("fp32", 3001, 3503, 0.1), ("fp64", 3001, 3503, 0.1),
+                                              ("fp32", 16387, 2050, 0.12),
+                                              ("fp32", 18431, 11000, 0.005)])
+def test_cg_products_with_vector_in_lds(gpu_lib, bulk, n, m, density):
+    """Sets of more than 1 M stored entries, whose products keep the gathered
+    vector in LDS: odd sizes, a last workgroup with few rows, one and two
+    right-hand sides, against the residual formed from the exported entries."""
+    import scipy.sparse as sp
+    reg = 0.02
+    M, a, b = cloud_problem(n, m, d=8, seed=82)
+    if bulk == "fp32":
+        M = M.astype(np.float32)
+    rng = np.random.default_rng(9)
+    N, tol = n + m - 1, 1e-10
+    with gpu_lib.Problem(M, a, b, reg) as P:
+        P.set_hess_storage(0)
+        P.sparsified_hess_with_density(near_optimum(P), density)
+        H = P.hess_export()
+        assert len(H["rval"]) > 1000000
+        S = sp.csr_matrix((H["rval"], H["colind"], H["rowptr"]), shape=(n, m - 1))
+        shift = 1e-3 * H["h2"].max()
+        r0, r1 = rng.standard_normal(N), rng.standard_normal(N)
+        s0 = P.hess_cg(r0, shift, tol=tol, max_iter=2000)
+        s1 = P.hess_cg(r1, shift, tol=tol, max_iter=2000)
+        pr = P.hess_cg2(r0, r1, shift, tol=tol, max_iter=2000)
+        same(s0, pr, 0)
+        same(s1, pr, 1)
+        for r, (x, it, err) in ((r0, s0), (r1, s1)):
+            assert 0 < it < 2000 and err <= tol
+            # the residual of the eliminated system, relative to its right-hand side
+            d1 = H["h1"] + shift
+            rhs = r[n:] - S.T @ (r[:n] / d1)
+            res = rhs - ((H["h2"] + shift) * x[n:] - S.T @ ((S @ x[n:]) / d1))
+            # the recurrence's residual drifts from the true one by rounding:
+            # it steps of 2^-52 times the size of Delta x (|Delta| <= 2 max h2)
+            drift = it * 2.0 ** -50 * 2.0 * H["h2"].max() * np.linalg.norm(x[n:])
+            assert np.linalg.norm(res) <= tol * np.linalg.norm(rhs) + drift
+            top = (r[:n] - S @ x[n:]) / d1
+            assert np.allclose(x[:n], top, rtol=1e-12, atol=1e-12 * np.abs(top).max())
