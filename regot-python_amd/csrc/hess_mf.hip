@@ -530,6 +530,14 @@ __global__ __launch_bounds__(256) void k_mf_fold(const double* __restrict__ part
     if (j >= m1) return;
     double s = 0.0;
     int w = 0;
+    // added in order, the loads far ahead
+    for (; w + 64 <= nwg; w += 64) {
+        double x[64];
+#pragma unroll
+        for (int u = 0; u < 64; u++) x[u] = part[static_cast<long>(w + u) * m1 + j];
+#pragma unroll
+        for (int u = 0; u < 64; u++) s += x[u];
+    }
     for (; w + 8 <= nwg; w += 8) {
         double x[8];
 #pragma unroll

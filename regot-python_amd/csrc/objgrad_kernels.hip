@@ -254,6 +254,29 @@ __device__ __forceinline__ void bsum4(double (&v)[4], double (*sm)[4])
     for (int q = 0; q < 4; q++) v[q] = ((sm[q][0] + sm[q][1]) + sm[q][2]) + sm[q][3];
 }
 
+// x[0] + x[pitch] + ... (cnt of them), 32 and then 8 loads in flight, added in
+// order.  (Eight at a time k_sums_fold took 8.2 us at 16384^2, now 7.3.)
+__device__ __forceinline__ double sum_strided(const double* __restrict__ x, long pitch, int cnt)
+{
+    double r = 0.0;
+    int s = 0;
+    for (; s + 32 <= cnt; s += 32) {
+        double v[32];
+#pragma unroll
+        for (int u = 0; u < 32; u++) v[u] = x[(s + u) * pitch];
+#pragma unroll
+        for (int u = 0; u < 32; u++) r += v[u];
+    }
+    for (; s < cnt; s += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = x[min(s + u, cnt - 1) * pitch];
+#pragma unroll
+        for (int u = 0; u < 8; u++) r += (s + u < cnt) ? v[u] : 0.0;
+    }
+    return r;
+}
+
 // Thread t < n: r_t = sum over strips, grad_t = r_t - a_t; thread t < m - 1:
 // c_t = sum over blocks (when colpart is set), grad_{n+t} = c_t - b_t.
 // part[4 wg + {0..3}] = this workgroup's sum r, sum alpha a, sum betat bt,
@@ -271,17 +294,7 @@ __global__ __launch_bounds__(256) void k_sums_fold(const double* __restrict__ ro
     const int t = blockIdx.x * 256 + threadIdx.x;
     double sr = 0.0, sa = 0.0, sb = 0.0, g2 = 0.0;
     if (t < n) {
-        // eight partials in flight, added in order
-        double r = 0.0;
-        int s = 0;
-        for (; s + 8 <= nstrip; s += 8) {
-            double x[8];
-#pragma unroll
-            for (int u = 0; u < 8; u++) x[u] = rowpart[static_cast<long>(s + u) * n + t];
-#pragma unroll
-            for (int u = 0; u < 8; u++) r += x[u];
-        }
-        for (; s < nstrip; s++) r += rowpart[static_cast<long>(s) * n + t];
+        const double r = sum_strided(rowpart + t, n, nstrip);
         const double g = r - a[t];
         if (grad) grad[t] = g;
         sr = r;
@@ -291,16 +304,7 @@ __global__ __launch_bounds__(256) void k_sums_fold(const double* __restrict__ ro
     if (t < m - 1) {
         sb = beta[t] * b[t];
         if (colpart) {
-            double c = 0.0;
-            int q = 0;
-            for (; q + 8 <= nblk; q += 8) {
-                double x[8];
-#pragma unroll
-                for (int u = 0; u < 8; u++) x[u] = colpart[static_cast<long>(q + u) * m + t];
-#pragma unroll
-                for (int u = 0; u < 8; u++) c += x[u];
-            }
-            for (; q < nblk; q++) c += colpart[static_cast<long>(q) * m + t];
+            const double c = sum_strided(colpart + t, m, nblk);
             const double g = c - b[t];
             if (grad) grad[n + t] = g;
             g2 += g * g;

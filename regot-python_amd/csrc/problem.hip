@@ -203,6 +203,15 @@ const double* regot_problem::stage(const double* host, long count)
     return mscal.d + 64;
 }
 
+const double* regot_problem::stage_gamma(const double* host)
+{
+    const long N = n + m - 1L;
+    const double* g = stage(host, N);
+    if (precise || bulk == 1) return g;
+    launch_copy(g, gamma, N, stream);
+    return gamma;
+}
+
 double* regot_problem::stage_out(long count)
 {
     if (count > static_cast<long>(n) + m) fail(E_INTERNAL, "staging %ld values", count);
@@ -556,9 +565,7 @@ int regot_dual_obj(regot_problem* p, const double* gamma_h, double* obj)
     CAPI_BEGIN
     check_handle(p);
     if (!gamma_h || !obj) fail(E_INVALID, "null pointer");
-    const long N = p->n + p->m - 1;
-    launch_copy(p->stage(gamma_h, N), p->gamma, N, p->stream);
-    *obj = p->dev_obj(p->gamma);
+    *obj = p->dev_obj(p->stage_gamma(gamma_h));
     CAPI_END
 }
 
@@ -568,8 +575,7 @@ int regot_dual_obj_grad(regot_problem* p, const double* gamma_h, double* obj, do
     check_handle(p);
     if (!gamma_h || !obj || !grad_h) fail(E_INVALID, "null pointer");
     const long N = p->n + p->m - 1;
-    launch_copy(p->stage(gamma_h, N), p->gamma, N, p->stream);
-    *obj = p->dev_obj_grad(p->gamma, p->stage_out(N), nullptr);
+    *obj = p->dev_obj_grad(p->stage_gamma(gamma_h), p->stage_out(N), nullptr);
     std::memcpy(grad_h, p->hout, N * sizeof(double));
     CAPI_END
 }

@@ -153,6 +153,10 @@ struct regot_problem {
     // count doubles of the caller's memory where a kernel can read them (until
     // the next stage(); the stream is idle when a call begins)
     const double* stage(const double* host, long count);
+    // gamma (n + m - 1) where dev_obj and dev_obj_grad may read it: the one-pass
+    // form reads it once, to split it, and takes it from the host; the two-pass
+    // form of FP32 bulk reads it again and gets a copy
+    const double* stage_gamma(const double* host);
     // device-visible room for count doubles, read at hout after sync() ...
     double* stage_out(long count);
     // ... which unstage() does, into the caller's memory
