@@ -82,7 +82,9 @@ __device__ __forceinline__ void exp2_tab_load(double* lds)
 // d = y - k = 64 f (exact) with the coefficients scaled by 64^-n, which again
 // changes no rounding.
 // The method proper, for |y| < kExp2Fast or a NaN, which comes out as a NaN.
-constexpr double kExp2Fast = 0x1p31;
+// (Up to 2^31 the bound may not reach: rint(2^31 - 1/2) is 2^31, whose low word
+// reads as -2^31.)
+constexpr double kExp2Fast = 0x1p30;
 __device__ __forceinline__ double dexp2_64_fast(double y, const double* tab)
 {
     constexpr double c1 = 0x1.62e42fefa39efp-1 * 0x1p-6, c2 = 0x1.ebfbdff82c58fp-3 * 0x1p-12;

@@ -248,3 +248,23 @@ def test_obj_grad_far_arguments(gpu_lib):
     assert np.array_equal(np.isinf(g), np.isinf(want))
     ok = np.isfinite(want)
     assert np.allclose(g[ok], want[ok], rtol=(n + m) * 2.0 ** -52, atol=1e-13)
+
+
+def test_obj_grad_arguments_at_the_table_bound(gpu_lib):
+    """Exponents whose table index leaves 32 bits: y = 64 log2(e) (-M) within a unit
+    of +-2^31 (the exponential's integer part there is +-2^31), and of +-2^30, are
+    inf or 0 as exp gives them."""
+    ys = [s * (2.0 ** e + d) for s in (1, -1) for e in (31, 30)
+          for d in (-0.75, -0.5, -0.25, 0.0, 0.5, 1.0)]
+    n, m = len(ys), 300
+    M = np.random.default_rng(1).random((n, m))
+    for i, y in enumerate(ys):
+        M[i, i] = -y / (64.0 * np.log2(np.e))
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    with gpu_lib.Problem(M, a, b, 1.0, bulk="fp64") as P:
+        f, g = P.dual_obj_grad(np.zeros(n + m - 1))
+    assert f == np.inf
+    for i, y in enumerate(ys):
+        assert (g[i] == np.inf) == (y > 0) and (g[n + i] == np.inf) == (y > 0), y
+    T = np.exp(-M[n // 2:])
+    assert np.allclose(g[n // 2:n], T.sum(1) - a[n // 2:], rtol=(n + m) * 2.0 ** -52)
