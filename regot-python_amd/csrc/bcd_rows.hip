@@ -32,7 +32,8 @@
 // Range: e and tot as in bcd_fused.hip; tot_i outside [lo, hi] (FP32
 // arithmetic 2^-+20, FP64 2^-+400) or not a number redoes the row with its
 // largest term as the shift.  A term flushed below the smallest normal drops
-// < 2^-106 (FP32) or < 2^-600 (FP64) of a_i from a column sum.
+// < 2^-106 (FP32) or < 2^-600 (FP64) of a_i from a column sum.  A row of
+// infinite costs has tot 0: alpha = +inf, and no part in the column sums.
 #include "dense.hpp"
 #include "dense_device.hpp"
 #include "dexp2.hpp"
@@ -157,6 +158,13 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
         if (!ONE) load_rows<TM, NC, R, NT>(M, ldm, i0 + R, r1, off, nxt);
         const double la0 = la, al0 = al, av0 = av;
         double shl = row_shift(la, al, k);
+        const bool row_in = lane < NW * R && i0 + lr < r1;
+        // A shift of 1e30 makes every term 0.  The repeats of the last row have
+        // weight 0 and must not have an infinite term; an infinite potential (a
+        // row without a finite cost) or one that is not a number (a warm start's)
+        // says nothing of the row's size, and the range test below finds a shift
+        // if there is a finite term.
+        shl = (row_in && __builtin_isfinite(shl)) ? shl : 1e30;
         if (!ONE) {
             // the next step's row data
             long i = i0 + R + lr;
@@ -165,7 +173,6 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
             al = alpha[i];
             av = a[i];
         }
-        const bool row_in = lane < NW * R && i0 + lr < r1;
         TA e[R][NC][V];
         double tot;
         for (int trial = 0;; trial++) {

@@ -282,3 +282,44 @@ def test_fp64_row_range_fallback(gpu_lib):
     # arguments of 1e4 carry 1e-12 absolute: duals to reg times that and more
     assert rel_err(r.dual, o["dual"]) < 1e-11 and rel_err(t.dual, o["dual"]) < 1e-11
     np.testing.assert_allclose(r.mar_errs, o["mar_errs"], rtol=1e-6, atol=1e-12)
+
+
+# --- infinite costs and non-finite warm starts -----------------------------------
+
+# one and several rows per workgroup, the step's last rows repeated or not
+@pytest.mark.parametrize("bulk,n,m", [("fp64", 30, 20), ("fp64", 300, 33), ("fp64", 30, 3000),
+                                      ("fp32", 60, 700), ("fp32", 1030, 700), ("fp32", 30, 3000),
+                                      ("fp32", 700, 5000)])
+def test_single_read_row_without_finite_cost(gpu_lib, bulk, n, m):
+    # a row of infinite costs has no mass to give: its potential is +inf and the
+    # others' iterates are those of the problem without it
+    M, a, b = cloud_problem(n, m, seed=n + m)
+    M = M.astype(np.float32 if bulk == "fp32" else np.float64)
+    for row in (n // 2, n - 1):
+        M2 = M.copy()
+        M2[row, :] = np.inf
+        print("infinite row %d of %dx%d %s" % (row, n, m, bulk), flush=True)
+        r, f32, f64 = fixed_iterations(gpu_lib, M2, a, b, 0.05, 4, bulk)
+        assert f32 + f64 == 5 and r.niter == 4
+        keep = np.arange(n) != row
+        o = O.sinkhorn_bcd(M[keep].astype(np.float64), a[keep], b, 0.05, tol=0.0, max_iter=4)
+        assert r.dual[row] == np.inf
+        assert rel_err(np.delete(r.dual, row), o["dual"]) < (1e-6 if bulk == "fp32" else 1e-12)
+
+
+@pytest.mark.parametrize("bulk,n,m", [("fp64", 30, 20), ("fp64", 30, 3000), ("fp32", 60, 700),
+                                      ("fp32", 30, 3000), ("fp32", 1030, 3000)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_single_read_recovers_from_a_warm_start(gpu_lib, bulk, n, m, bad):
+    # alpha_0 only guesses the scale of the first row sums; a row whose guess is
+    # not finite is formed again by the next iteration
+    M, a, b = cloud_problem(n, m, seed=n + m)
+    M = M.astype(np.float32 if bulk == "fp32" else np.float64)
+    x0 = 0.01 * np.random.default_rng(3).standard_normal(n + m - 1)
+    x0[n - 1] = bad
+    print("warm start with %s %dx%d %s" % (bad, n, m, bulk), flush=True)
+    with gpu_lib.Problem(M, a, b, 0.05, bulk=bulk) as P:
+        r = P.solve(0, tol=1e-8, max_iter=2000, compute_plan=False, x0=x0)
+        c = P.solve(0, tol=1e-8, max_iter=2000, compute_plan=False)
+    assert r.niter < 2000 and np.all(np.isfinite(r.dual))
+    assert rel_err(r.dual, c.dual) < 1e-5      # both within tol of the one solution
