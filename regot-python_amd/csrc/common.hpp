@@ -171,12 +171,12 @@ template <typename T>
 struct MappedRing {
     T* h = nullptr;
     T* d = nullptr;
-    int cap = 0;
+    size_t cap = 0;
     MappedRing() = default;
     MappedRing(const MappedRing&) = delete;
     MappedRing& operator=(const MappedRing&) = delete;
     ~MappedRing() { release(); }
-    void ensure(int c)
+    void ensure(size_t c)
     {
         if (h && c <= cap) return;
         release();

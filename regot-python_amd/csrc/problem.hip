@@ -188,8 +188,8 @@ void regot_problem::setup(int n_, int m_, const void* M, int M_dtype, int bulk_,
     KERNEL_CHECK();
 
     // scalars, then room for a vector each way: one pinned allocation
-    mscal.ensure(64 + 2 * (n + m));
-    hout = mscal.h + 64 + (n + m);
+    mscal.ensure(stage_size(n, m));
+    hout = mscal.h + stage_out_at(n, m);
     HIP_CHECK(hipStreamSynchronize(stream));
 }
 
@@ -199,13 +199,13 @@ const double* regot_problem::stage(const double* host, long count)
 {
     if (count > static_cast<long>(n) + m) fail(E_INTERNAL, "staging %ld values", count);
     if (count > 0 && !host) fail(E_INVALID, "null input vector");
-    std::memcpy(mscal.h + 64, host, count * sizeof(double));
-    return mscal.d + 64;
+    std::memcpy(mscal.h + kStageAt, host, count * sizeof(double));
+    return mscal.d + kStageAt;
 }
 
 const double* regot_problem::stage_gamma(const double* host)
 {
-    const long N = n + m - 1L;
+    const long N = static_cast<long>(n) + m - 1;
     const double* g = stage(host, N);
     if (precise || bulk == 1) return g;
     launch_copy(g, gamma, N, stream);
@@ -215,7 +215,7 @@ const double* regot_problem::stage_gamma(const double* host)
 double* regot_problem::stage_out(long count)
 {
     if (count > static_cast<long>(n) + m) fail(E_INTERNAL, "staging %ld values", count);
-    return mscal.d + 64 + (n + m);
+    return mscal.d + stage_out_at(n, m);
 }
 
 void regot_problem::unstage(double* host, long count)

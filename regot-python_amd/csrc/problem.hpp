@@ -149,6 +149,9 @@ struct regot_problem {
     // on their way out (hout).
     regot::MappedRing<double> mscal;
     double* hout = nullptr;
+    static constexpr size_t kStageAt = 64;
+    static size_t stage_out_at(int n, int m) { return kStageAt + (static_cast<size_t>(n) + m); }
+    static size_t stage_size(int n, int m) { return kStageAt + 2 * (static_cast<size_t>(n) + m); }
     regot::DBuf<double> cin, cout;   // device side of an operator call's vectors
     // count doubles of the caller's memory where a kernel can read them (until
     // the next stage(); the stream is idle when a call begins)
