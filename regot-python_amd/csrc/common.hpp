@@ -196,4 +196,14 @@ struct MappedRing {
 
 inline int ceil_div(long a, long b) { return static_cast<int>((a + b - 1) / b); }
 
+// Grid of `blocks` workgroups of 256 threads.  A launch holds fewer than 2^32
+// threads along x, so wider ones continue along y; the kernel's block is
+// blockIdx.y gridDim.x + blockIdx.x, and the last few may lie past the end.
+inline dim3 wide_grid(long blocks)
+{
+    constexpr long kX = 1L << 23;
+    if (blocks <= kX) return dim3(static_cast<unsigned>(blocks));
+    return dim3(static_cast<unsigned>(kX), static_cast<unsigned>((blocks + kX - 1) / kX));
+}
+
 }  // namespace regot

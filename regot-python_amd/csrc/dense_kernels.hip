@@ -196,15 +196,17 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
                                                      BcdState st, const int* __restrict__ ctl)
 {
     if (ctl != nullptr && ctl[0] != 0) return;
-    if (BCD && blockIdx.x == gridDim.x - 1) {
-        bcd_decide(st);
+    const int tiles = (m + kCombineCols - 1) / kCombineCols;
+    const int tile = blockIdx.y * gridDim.x + blockIdx.x;   // wide_grid
+    if (tile >= tiles) {
+        if (BCD && tile == tiles) bcd_decide(st);
         return;
     }
     constexpr int NS = BCD ? kCombineSubs : 4;
     __shared__ double xs[kCombineSubs][kCombineCols];
     const int col = threadIdx.x & (kCombineCols - 1);
     const int sub = threadIdx.x / kCombineCols;
-    const int j = blockIdx.x * kCombineCols + col;
+    const int j = tile * kCombineCols + col;
     const bool valid = j < m;
     double cp = 0.0, bj = 0.0, lb = 0.0;
     if (valid && sub == 0) {
@@ -284,8 +286,8 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
         bb = group_sum<kCombineCols>(bb);
         if (col == 0) {
             double* tp = epi.tilepart + (BCD ? 2L * st.ntiles * ((st.k + 1) & 1) : 0);
-            tp[2 * blockIdx.x] = r2;
-            tp[2 * blockIdx.x + 1] = bb;
+            tp[2 * tile] = r2;
+            tp[2 * tile + 1] = bb;
         }
     }
 }
@@ -460,10 +462,10 @@ void launch_col_pass(int bulk, const void* M, long ldm, int n, int m, const doub
     KERNEL_CHECK();
     const int tiles = col_combine_blocks(m);
     if (st != nullptr)
-        hipLaunchKernelGGL((k_col_combine<true, false>), dim3(tiles + 1), dim3(256), 0, s, part,
+        hipLaunchKernelGGL((k_col_combine<true, false>), wide_grid(tiles + 1L), dim3(256), 0, s, part,
                            static_cast<long>(m), nblk, m, k, epi, *st, ctl);
     else
-        hipLaunchKernelGGL((k_col_combine<false, false>), dim3(tiles), dim3(256), 0, s, part,
+        hipLaunchKernelGGL((k_col_combine<false, false>), wide_grid(tiles), dim3(256), 0, s, part,
                            static_cast<long>(m), nblk, m, k, epi, BcdState{}, ctl);
     KERNEL_CHECK();
 }
@@ -472,8 +474,8 @@ void launch_col_combine_sums(const double* part, long pitch, int nblk, int m, do
                              const ColEpi& epi, const BcdState& st, hipStream_t s)
 {
     if (epi.colpot == nullptr) fail(E_INTERNAL, "column-sum combine needs the column potential");
-    hipLaunchKernelGGL((k_col_combine<true, true>), dim3(col_combine_blocks(m) + 1), dim3(256), 0,
-                       s, part, pitch, nblk, m, k, epi, st, st.ctl);
+    hipLaunchKernelGGL((k_col_combine<true, true>), wide_grid(col_combine_blocks(m) + 1L),
+                       dim3(256), 0, s, part, pitch, nblk, m, k, epi, st, st.ctl);
     KERNEL_CHECK();
 }
 

@@ -234,9 +234,11 @@ __global__ __launch_bounds__(256) void k_qrot_obj_fold(
     __shared__ double sm[4][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int e = blockIdx.x * 64 + lane;
+    const long blk = static_cast<long>(blockIdx.y) * gridDim.x + blockIdx.x;   // wide_grid
+    const long e = blk * 64 + lane;
     const bool row = e < n;
-    const bool valid = e < n + m;
+    const bool valid = e < static_cast<long>(n) + m;
+    if (blk * 64 >= static_cast<long>(n) + m) return;
     double v = 0.0;
     if (rsum)
         v = fold64(row ? rowpart + e : colpart + (e - n), row ? nstrip : nblk, row ? n : m, valid,
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(256) void k_qrot_obj_fold(
     wave_sums<4>(w);
     if (lane == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) part[4 * blockIdx.x + q] = w[q];
+        for (int q = 0; q < 4; q++) part[4 * blk + q] = w[q];
     }
 }
 
@@ -311,7 +313,9 @@ __global__ __launch_bounds__(256) void k_qrot_cols_fold(const double* __restrict
     __shared__ double sm[4][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int j = blockIdx.x * 64 + lane;
+    const long blk = static_cast<long>(blockIdx.y) * gridDim.x + blockIdx.x;   // wide_grid
+    const long j = blk * 64 + lane;
+    if (blk * 64 >= m) return;
     const double v = fold64(colpart + j, nblk, m, j < m, wave, lane, sm);
     if (wave != 0) return;
     double w = 0.0;
@@ -324,7 +328,7 @@ __global__ __launch_bounds__(256) void k_qrot_cols_fold(const double* __restrict
         w = e * e;
     }
     w = wave_sum0(w);
-    if (lane == 0) part[blockIdx.x] = w;
+    if (lane == 0) part[blk] = w;
 }
 
 // err_a = a - x A / reg; per workgroup {|err_a|_1, ||err_a||^2,
@@ -337,7 +341,9 @@ __global__ __launch_bounds__(256) void k_qrot_rows_fold(const double* __restrict
     __shared__ double sm[4][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = blockIdx.x * 64 + lane;
+    const long blk = static_cast<long>(blockIdx.y) * gridDim.x + blockIdx.x;   // wide_grid
+    const long i = blk * 64 + lane;
+    if (blk * 64 >= n) return;
     const long plane = static_cast<long>(nstrip) * n;
     const double A = fold64(rowpart + i, nstrip, n, i < n, wave, lane, sm);
     const double B = fold64(rowpart + plane + i, nstrip, n, i < n, wave, lane, sm);
@@ -354,7 +360,7 @@ __global__ __launch_bounds__(256) void k_qrot_rows_fold(const double* __restrict
     wave_sums<4>(w);
     if (lane == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) part[4 * blockIdx.x + q] = w[q];
+        for (int q = 0; q < 4; q++) part[4 * blk + q] = w[q];
     }
 }
 
@@ -465,7 +471,7 @@ double qrot_obj_grad(regot_problem* p, const double* gamma, double* grad, double
         sweep_any<SW_GRAD>(p, alpha, beta, w, w.rowpart, w.colpart, w.sqpart);
     else
         sweep_any<SW_OBJ>(p, alpha, beta, w, nullptr, nullptr, w.sqpart);
-    hipLaunchKernelGGL(k_qrot_obj_fold, dim3(ne), dim3(256), 0, s, w.rowpart.p, g.strips,
+    hipLaunchKernelGGL(k_qrot_obj_fold, wide_grid(ne), dim3(256), 0, s, w.rowpart.p, g.strips,
                        w.colpart.p, g.blocks, alpha, beta, p->a.p, p->b.p, n, m, p->reg,
                        grad ? w.rsum.p : nullptr, w.csum.p, w.x.p,
                        grad && !(tau > 0.0) ? grad : nullptr, w.epart.p);
@@ -491,19 +497,19 @@ double qrot_primal(regot_problem* p, const double* alpha, const double* beta, bo
         const SweepGrid g = sweep_grid(n, m, SW_GRAD);
         sweep_any<SW_GRAD>(p, alpha, beta, w, w.rowpart, w.colpart, w.sqpart);
         const int ne = ceil_div(static_cast<long>(n) + m, 64);
-        hipLaunchKernelGGL(k_qrot_obj_fold, dim3(ne), dim3(256), 0, s, w.rowpart.p, g.strips,
+        hipLaunchKernelGGL(k_qrot_obj_fold, wide_grid(ne), dim3(256), 0, s, w.rowpart.p, g.strips,
                            w.colpart.p, g.blocks, alpha, beta, p->a.p, p->b.p, n, m, p->reg, w.rsum.p,
                            w.csum.p, w.x.p, static_cast<double*>(nullptr), w.epart.p);
         KERNEL_CHECK();
     }
     const int nc = ceil_div(m, 64), nr = ceil_div(n, 64);
     sweep_any<SW_COLS>(p, alpha, beta, w, nullptr, w.colpart, nullptr);
-    hipLaunchKernelGGL(k_qrot_cols_fold, dim3(nc), dim3(256), 0, s, w.colpart.p,
+    hipLaunchKernelGGL(k_qrot_cols_fold, wide_grid(nc), dim3(256), 0, s, w.colpart.p,
                        sweep_grid(n, m, SW_COLS).blocks, p->b.p, m, p->reg, w.y.p, w.eb.p, w.cpart.p);
     KERNEL_CHECK();
     const SweepGrid g = sweep_grid(n, m, SW_LAST);
     sweep_any<SW_LAST>(p, alpha, beta, w, w.rowpart, nullptr, w.scal);
-    hipLaunchKernelGGL(k_qrot_rows_fold, dim3(nr), dim3(256), 0, s, w.rowpart.p, g.strips, p->a.p,
+    hipLaunchKernelGGL(k_qrot_rows_fold, wide_grid(nr), dim3(256), 0, s, w.rowpart.p, g.strips, p->a.p,
                        w.x.p, n, p->reg, w.epart.p);
     hipLaunchKernelGGL(k_qrot_round_total, dim3(1), dim3(256), 0, s, w.scal.p, g.strips * g.blocks,
                        w.epart.p, nr, w.cpart.p, nc, p->reg, p->mscal.d);

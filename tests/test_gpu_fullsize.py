@@ -79,3 +79,30 @@ def test_c3_sparse_newton_and_splr_16384(gpu_lib):
     for key in (("sn", 0.01), ("splr", 0.05)):
         err = cpu_marginal_error(M, a, b, reg, out[key].dual)
         assert err < 1e-8, (key, err)
+
+
+def test_one_row_of_more_columns_than_a_launch_is_wide(gpu_lib):
+    # 16 threads per column in the combine: from 2^28 columns on, more threads than
+    # one launch dimension holds.  With one row the half-steps are closed forms.
+    import torch
+    m, reg = (1 << 28) + 1000, 0.5
+    g = torch.Generator(device="cuda")
+    g.manual_seed(0)
+    M = torch.zeros(1, (m + 63) // 64 * 64, device="cuda")
+    M[:, :m] = torch.rand(1, m, device="cuda", generator=g)
+    b = np.full(m, 1.0 / m)
+    torch.cuda.synchronize()
+    print("1 x %d" % m, flush=True)
+    with gpu_lib.Problem.from_device(M.data_ptr(), 1, m, np.float32, np.ones(1), b, reg,
+                                     ldm=M.shape[1]) as P:
+        beta = torch.from_numpy(P.optimal_beta(np.full(1, 0.25))).to("cuda")
+        # reg log b - 0.25 + M, from FP32 terms
+        beta -= M[0, :m].double() + (reg * np.log(1.0 / m) - 0.25)
+        assert beta.abs().max().item() < 1e-6
+        del beta
+        print("  solve", flush=True)
+        r = P.solve(0, tol=0.5, max_iter=1, compute_plan=False)
+    # beta_0 is the solution: f = -sum b (beta_j + reg log a ...), gauge beta_{m-1} = 0
+    assert r.niter == 0 and r.mar_errs[0] < 1e-3
+    dual = torch.from_numpy(r._dual[1:]).to("cuda")
+    assert (dual - (M[0, :m - 1] - M[0, m - 1]).double()).abs().max().item() < 2e-6

@@ -30,3 +30,8 @@ needs_gxx = pytest.mark.skipif(shutil.which("g++") is None or
 def test_staging_memory_of_wide_problems(tmp_path):
     # n + m values each way, from n + m = 2 up to the largest int sizes
     run_host_check("staging_check", tmp_path)
+
+
+@needs_gxx
+def test_grids_of_wide_problems(tmp_path):
+    run_host_check("grid_check", tmp_path)
