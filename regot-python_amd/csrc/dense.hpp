@@ -35,10 +35,9 @@ struct ColEpi {
     // Column gradient: with beta_out, b_j * expm1(beta_out_j/reg + ln2 lse2 - log b_j)
     // (the FP64 rounding residual of the update); otherwise colsum_j - b_j.
     double* resid = nullptr;
-    // Per combine workgroup t (j < m-1 only): [2t] = sum resid_j^2,
+    // Per tile t of 16 columns (j < m-1 only): [2t] = sum resid_j^2,
     // [2t+1] = sum beta_j b_j with beta = beta_out if set, else colpot.
-    // In BCD mode the half selected by the parity of k+1 is written.  Tiles
-    // are of col_combine_blocks(m) workgroups in every mode.
+    // In BCD mode the half selected by the parity of k+1 is written.
     double* tilepart = nullptr;
     double reg = 1.0;
 };
@@ -53,10 +52,10 @@ void launch_row_pass(int bulk, const void* M, long ldm, int n, int m, const doub
 struct BcdState;
 
 // Column pass: partial log2-sums per (row block, column) into part (nblk * m
-// doubles), then a combine kernel (4 threads per column) with the epilogue.
+// doubles), then a combine kernel (4 or 16 threads per column) with the epilogue.
 // With st, the combine also takes the BCD stop decision (see BcdState).
 int col_pass_blocks(int n, int m);
-int col_combine_blocks(int m);
+int col_combine_tiles(int m);
 void launch_col_pass(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
                      const double* colpot_guess, const double* logb, double k, double* part,
                      int nblk, const ColEpi& epi, const BcdState* st, const int* ctl,
@@ -85,7 +84,7 @@ struct BcdState {
     double* rpart;          // per row-pass workgroup: sum g^2, sum r, sum alpha a
     const double* cpart;    // 2 x ntiles x (sum resid^2, sum beta_j b_j), j < m-1
     int nrb;                // row-pass workgroups
-    int ntiles;             // combine workgroups
+    int ntiles;             // tiles of 16 columns
     double sum_a;           // sum_i a_i
     double sum_b1;          // sum_{j < m-1} b_j
     double tol;

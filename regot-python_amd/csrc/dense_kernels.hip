@@ -104,8 +104,10 @@ __global__ __launch_bounds__(256) void k_col_partial(
 // 4096 with 256 partials (8.4 MB) 64 columns x 4 threads, which ran on m / 64
 // workgroups, took 14.6 us (events around the kernel) and this split with the
 // stop decision off the update's path 7.0; at m = 16384 14.3 and 10.6.
-constexpr int kCombineCols = 16;
-constexpr int kCombineSubs = 256 / kCombineCols;
+// Where a column has at most 4 partials (few rows, or a wide matrix), 16 threads
+// have little to share out: 64 columns x 4 threads, a quarter of the workgroups
+// (131072 columns, 16 rows, FP32: 279 us per two-pass iteration, now 268).
+constexpr int kCombineTile = 16;   // columns per entry of ColEpi::tilepart
 
 // Stop test of the on-device BCD loop for iterate k = st.k, by one workgroup:
 // g_k = [r - a ; column residual of the update that produced beta_k],
@@ -124,9 +126,21 @@ __device__ void bcd_decide(const BcdState& st)
         v[1] += st.rpart[3 * q + 1];
         v[2] += st.rpart[3 * q + 2];
     }
-    for (int q = threadIdx.x; q < st.ntiles; q += 256) {
-        v[3] += cp[2 * q];
-        v[4] += cp[2 * q + 1];
+    // Eight loads in flight, added in order: one at a time, the sum over the tiles
+    // of a wide matrix outlasts the rest of the combine (65536 columns, 16 rows,
+    // FP64: 267 us per iteration, now 264).
+    constexpr int U = 8;
+    const double2* cp2 = reinterpret_cast<const double2*>(cp);
+    for (int q = threadIdx.x; q < st.ntiles; q += 256 * U) {
+        double2 x[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) x[u] = cp2[min(q + 256 * u, st.ntiles - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (q + 256 * u < st.ntiles) {
+                v[3] += x[u].x;
+                v[4] += x[u].y;
+            }
     }
     block_sums_256<5>(v);
     if (threadIdx.x != 0) return;
@@ -160,8 +174,7 @@ __device__ void bcd_decide(const BcdState& st)
 // Sum (or maximum) over the NS threads of each column, neighbours first; the
 // result is on every thread of the column.  x[sub][col] in LDS.
 template <bool MAX, int NS>
-__device__ __forceinline__ double combine_subs(double v, double (*x)[kCombineCols], int sub,
-                                               int col)
+__device__ __forceinline__ double combine_subs(double v, double (*x)[256 / NS], int sub, int col)
 {
     x[sub][col] = v;
     __syncthreads();
@@ -176,7 +189,7 @@ __device__ __forceinline__ double combine_subs(double v, double (*x)[kCombineCol
     return y[0];
 }
 
-// Combine the nblk partials of each column (16 threads per column, fixed
+// Combine the nblk partials of each column (NS threads per column, fixed
 // order), then the column epilogue.  With BCD (iterate st.k), the extra last
 // workgroup takes the stop decision while the others write beta_{k+1}: the
 // loop keeps beta double-buffered by parity, so the update does not wait for
@@ -184,29 +197,29 @@ __device__ __forceinline__ double combine_subs(double v, double (*x)[kCombineCol
 // (Every workgroup taking the decision itself before its update put two more
 // memory round trips on the critical path.)  The tile sums of the new column
 // residual go to the other parity half of cpart.  Without BCD (one call, not a
-// loop) four threads per column add the partials p = sub, sub + 4, ...: that
-// order is the one the solvers started from optimal_beta have always had, and
-// an L-BFGS path follows its last bit.
+// loop) NS = 4, the partials p = sub, sub + 4, ...: that order is the one the
+// solvers started from optimal_beta have always had, and an L-BFGS path follows
+// its last bit.  (With at most 4 partials both NS add in the same order.)
 // SUMS: the partials are plain FP64 column sums of exp((alpha_i + colpot_j -
 // M_ij) / reg) (the single-read BCD pass), so log2 sum_i 2^((alpha_i - M_ij) k)
 // = log2(sum) - colpot_j k.
-template <bool BCD, bool SUMS>
+template <bool BCD, bool SUMS, int NS>
 __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ part, long pitch,
                                                      int nblk, int m, double k, ColEpi epi,
                                                      BcdState st, const int* __restrict__ ctl)
 {
     if (ctl != nullptr && ctl[0] != 0) return;
-    const int tiles = (m + kCombineCols - 1) / kCombineCols;
-    const int tile = blockIdx.y * gridDim.x + blockIdx.x;   // wide_grid
-    if (tile >= tiles) {
-        if (BCD && tile == tiles) bcd_decide(st);
+    constexpr int COLS = 256 / NS;
+    const int wgs = (m + COLS - 1) / COLS;
+    const int wg = blockIdx.y * gridDim.x + blockIdx.x;   // wide_grid
+    if (wg >= wgs) {
+        if (BCD && wg == wgs) bcd_decide(st);
         return;
     }
-    constexpr int NS = BCD ? kCombineSubs : 4;
-    __shared__ double xs[kCombineSubs][kCombineCols];
-    const int col = threadIdx.x & (kCombineCols - 1);
-    const int sub = threadIdx.x / kCombineCols;
-    const int j = tile * kCombineCols + col;
+    __shared__ double xs[NS][COLS];
+    const int col = threadIdx.x & (COLS - 1);
+    const int sub = threadIdx.x / COLS;
+    const int j = wg * COLS + col;
     const bool valid = j < m;
     double cp = 0.0, bj = 0.0, lb = 0.0;
     if (valid && sub == 0) {
@@ -222,10 +235,10 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
         double cs = 0.0;
         if (valid) {
             int p = sub;
-            for (; p + (U - 1) * kCombineSubs < nblk; p += U * kCombineSubs) {
+            for (; p + (U - 1) * NS < nblk; p += U * NS) {
                 double x[U];
 #pragma unroll
-                for (int u = 0; u < U; u++) x[u] = pj[(p + u * kCombineSubs) * pitch];
+                for (int u = 0; u < U; u++) x[u] = pj[(p + u * NS) * pitch];
 #pragma unroll
                 for (int u = 0; u < U; u++) cs += x[u];
             }
@@ -233,7 +246,7 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
                 double x[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const int pu = p + u * kCombineSubs;
+                    const int pu = p + u * NS;
                     x[u] = (pu < nblk) ? pj[pu * pitch] : 0.0;
                 }
 #pragma unroll
@@ -244,11 +257,11 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
         L = cs > 0.0 ? log2(cs) - cp * k : -INFINITY;
     } else {
         double Lm = -INFINITY;
-        if (valid && sub < NS)
+        if (valid)
             for (int p = sub; p < nblk; p += NS) Lm = fmax(Lm, pj[p * pitch]);
         Lm = combine_subs<true, NS>(Lm, xs, sub, col);
         double S = 0.0;
-        if (valid && sub < NS && Lm != -INFINITY)
+        if (valid && Lm != -INFINITY)
             for (int p = sub; p < nblk; p += NS) {
                 const double x = pj[p * pitch];
                 S += (x == -INFINITY) ? 0.0 : exp2(x - Lm);
@@ -281,13 +294,13 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
         }
     }
     if (epi.tilepart) {
-        // the 16 threads of sub 0 are one DPP row of wave 0
-        r2 = group_sum<kCombineCols>(r2);
-        bb = group_sum<kCombineCols>(bb);
-        if (col == 0) {
+        // the threads of sub 0 are lanes of wave 0, 16 columns a DPP row
+        r2 = group_sum<kCombineTile>(r2);
+        bb = group_sum<kCombineTile>(bb);
+        if (col % kCombineTile == 0 && valid) {
             double* tp = epi.tilepart + (BCD ? 2L * st.ntiles * ((st.k + 1) & 1) : 0);
-            tp[2 * tile] = r2;
-            tp[2 * tile + 1] = bb;
+            tp[2 * (j / kCombineTile)] = r2;
+            tp[2 * (j / kCombineTile) + 1] = bb;
         }
     }
 }
@@ -434,7 +447,7 @@ int col_pass_blocks(int n, int m)
     return nblk;
 }
 
-int col_combine_blocks(int m) { return ceil_div(m, kCombineCols); }
+int col_combine_tiles(int m) { return ceil_div(m, kCombineTile); }
 
 void launch_col_pass(int bulk, const void* M, long ldm, int n, int m, const double* alpha,
                      const double* colpot_guess, const double* logb, double k, double* part,
@@ -460,13 +473,17 @@ void launch_col_pass(int bulk, const void* M, long ldm, int n, int m, const doub
                            static_cast<const double*>(M), ldm, n, m, alpha, colpot_guess, logb,
                            k, rpb, part, ctl, nt);
     KERNEL_CHECK();
-    const int tiles = col_combine_blocks(m);
-    if (st != nullptr)
-        hipLaunchKernelGGL((k_col_combine<true, false>), wide_grid(tiles + 1L), dim3(256), 0, s, part,
-                           static_cast<long>(m), nblk, m, k, epi, *st, ctl);
+    // (the stop decision is one more workgroup)
+    const long pitch = m;
+    if (st != nullptr && nblk > 4)
+        hipLaunchKernelGGL((k_col_combine<true, false, 16>), wide_grid(ceil_div(m, 16) + 1L),
+                           dim3(256), 0, s, part, pitch, nblk, m, k, epi, *st, ctl);
+    else if (st != nullptr)
+        hipLaunchKernelGGL((k_col_combine<true, false, 4>), wide_grid(ceil_div(m, 64) + 1L),
+                           dim3(256), 0, s, part, pitch, nblk, m, k, epi, *st, ctl);
     else
-        hipLaunchKernelGGL((k_col_combine<false, false>), wide_grid(tiles), dim3(256), 0, s, part,
-                           static_cast<long>(m), nblk, m, k, epi, BcdState{}, ctl);
+        hipLaunchKernelGGL((k_col_combine<false, false, 4>), wide_grid(ceil_div(m, 64)),
+                           dim3(256), 0, s, part, pitch, nblk, m, k, epi, BcdState{}, ctl);
     KERNEL_CHECK();
 }
 
@@ -474,7 +491,7 @@ void launch_col_combine_sums(const double* part, long pitch, int nblk, int m, do
                              const ColEpi& epi, const BcdState& st, hipStream_t s)
 {
     if (epi.colpot == nullptr) fail(E_INTERNAL, "column-sum combine needs the column potential");
-    hipLaunchKernelGGL((k_col_combine<true, true>), wide_grid(col_combine_blocks(m) + 1L),
+    hipLaunchKernelGGL((k_col_combine<true, true, 16>), wide_grid(ceil_div(m, 16) + 1L),
                        dim3(256), 0, s, part, pitch, nblk, m, k, epi, st, st.ctl);
     KERNEL_CHECK();
 }

@@ -166,7 +166,7 @@ void regot_problem::setup(int n_, int m_, const void* M, int M_dtype, int bulk_,
     HIP_CHECK(hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, device));
 
     nblk = col_pass_blocks(n, m);
-    ntiles = col_combine_blocks(m);
+    ntiles = col_combine_tiles(m);
     slab.add(a, n);
     slab.add(b, m);
     slab.add(loga, n);

@@ -323,3 +323,23 @@ def test_single_read_recovers_from_a_warm_start(gpu_lib, bulk, n, m, bad):
         c = P.solve(0, tol=1e-8, max_iter=2000, compute_plan=False)
     assert r.niter < 2000 and np.all(np.isfinite(r.dual))
     assert rel_err(r.dual, c.dual) < 1e-5      # both within tol of the one solution
+
+
+# four and sixteen threads per column in the combine (4 and 5 row blocks of 16),
+# and 64- and 16-column workgroups with a remainder; 131101 columns: 513 tiles of
+# 256 and so one row block, and more tile sums than eight per thread
+@pytest.mark.parametrize("n,m", [(64, 65), (65, 65), (64, 1007), (65, 1007), (3, 1), (70, 16),
+                                 (17, 131101)])
+@pytest.mark.parametrize("bulk", ["fp32", "fp64"])
+def test_two_pass_combine_splits(gpu_lib, bulk, n, m):
+    M, a, b = cloud_problem(n, m, d=4, seed=n + m)
+    M = M.astype(np.float32 if bulk == "fp32" else np.float64)
+    print("two-pass combine %dx%d %s" % (n, m, bulk), flush=True)
+    r, f32, f64 = fixed_iterations(gpu_lib, M, a, b, 0.05, 4, bulk, fused=0)
+    assert (f32, f64) == (0, 0)
+    o = O.sinkhorn_bcd(M.astype(np.float64), a, b, 0.05, tol=0.0, max_iter=4)
+    assert rel_err(r.dual, o["dual"]) < (1e-6 if bulk == "fp32" else 1e-12)
+    np.testing.assert_allclose(r.obj_vals, o["obj_vals"], rtol=1e-7 if bulk == "fp32" else 1e-11)
+    # FP64: the sums of squares over all tiles; FP32 rounds each row sum to 2^-23
+    np.testing.assert_allclose(r.mar_errs, o["mar_errs"], rtol=1e-2 if bulk == "fp32" else 1e-7,
+                               atol=2e-7 if bulk == "fp32" else 1e-14)
