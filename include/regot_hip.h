@@ -195,8 +195,10 @@ typedef struct {
     /* BCD iteration form.  0: two passes over M per iteration (row pass,
      * column pass); nonzero (default 1): one pass per iteration when
      * m <= 8192 (FP32 bulk in FP32 arithmetic: m <= 16384), at most 1024 rows
-     * fall to each compute unit and min a min b >= 2^-60 sum a sum b; the
-     * two-pass form otherwise. */
+     * fall to each compute unit and min a min b >= 2^-60 sum a sum b, except
+     * for tall, narrow matrices, where two passes are faster (m <= 512, FP64
+     * bulk 256, and more than 192, FP64 arithmetic 128, rows per compute unit
+     * and 256, FP64 bulk 128, columns); the two-pass form otherwise. */
     int bcd_fused;
     double tau;          /* QROT gradient descent / L-BFGS: extra term tau/2 (1'alpha - 1'beta)^2
                             (QROTSolverOpts::tau, src/qrot_solvers.h:15-30); default 0 */

@@ -352,6 +352,24 @@ bool bcd_rows_shape_ok(int n, int m, int ncu)
     return n >= 1 && m >= 1 && m <= kRMaxCols && ceil_div(n, bcd_fused_blocks(n, ncu)) <= kRMaxRows;
 }
 
+// The pass costs a workgroup 0.3 us per row (FP32 storage with FP64 arithmetic:
+// 0.45) however few columns the row has, since its threads past them idle; the
+// two-pass form costs a time per strip of columns (64 lanes x 16 bytes), and with
+// one or two strips that is the smaller.  us per iteration, single read
+// / two passes, at 128, 192, 256 and 512 rows per CU: FP32 x 256 columns 44 / 55,
+// 63 / 65, 81 / 74, 154 / 112; x 512 45 / 59, 63 / 74, 82 / 90, 157 / 151; x 576
+// 45 / 69, 63 / 92, 82 / 112, 157 / 209.  FP64 x 128 50 / 53, 71 / 64, 92 / 74,
+// 175 / 114; x 256 50 / 65, 71 / 79, 93 / 95, 179 / 154; x 320 51 / 67, 72 / 88,
+// 93 / 108, 178 / 198.  FP32 storage with FP64 arithmetic x 256 65 / 65, 92 / 78,
+// 121 / 92; x 512 64 / 77, 92 / 100, 121 / 120, 235 / 209.
+bool bcd_rows_pays(int bulk, bool precise, int n, int m, int ncu)
+{
+    const int strip = bulk == 0 ? 256 : 128;
+    const int limit = bulk == 0 && !precise ? 192 : 128;
+    const int rows = ceil_div(n, bcd_fused_blocks(n, ncu));
+    return m > 2 * strip || rows <= limit * ceil_div(m, strip);
+}
+
 long bcd_part_pitch(int m) { return (static_cast<long>(m) + 15) / 16 * 16; }
 
 void launch_bcd_rows(int bulk, bool precise, BcdRowsArgs g, hipStream_t s)

@@ -131,6 +131,8 @@ struct BcdRowsArgs {
     int rpw, nt;            // set by the launcher
 };
 bool bcd_rows_shape_ok(int n, int m, int ncu);
+// Whether it is faster there than two passes.
+bool bcd_rows_pays(int bulk, bool precise, int n, int m, int ncu);
 long bcd_part_pitch(int m);
 void launch_bcd_rows(int bulk, bool precise, BcdRowsArgs g, hipStream_t s);
 // 8192 < m <= 16384, FP32 (bcd_fused.hip):

@@ -333,11 +333,12 @@ void regot_problem::row_pass_bcd(const double* beta_full, const RowEpi& epi, con
 // FP64), which holds when beta_k came out of an exact beta update and the
 // marginals are bounded away from zero as below (see bcd_fused.hip).  FP64
 // arithmetic (FP64 bulk, or FP32 bulk's precise finish) has the pass of
-// bcd_rows.hip only.
+// bcd_rows.hip only.  Tall, narrow matrices take two passes (bcd_rows_pays).
 bool regot_problem::bcd_fused_ok(bool f64) const
 {
-    const bool shape = bcd_rows_shape_ok(n, m, ncu) ||
-                       (!f64 && bulk == REGOT_F32 && bcd_fused_shape_ok(n, m, ncu));
+    const bool shape =
+        (bcd_rows_shape_ok(n, m, ncu) && bcd_rows_pays(bulk, f64, n, m, ncu)) ||
+        (!f64 && bulk == REGOT_F32 && bcd_fused_shape_ok(n, m, ncu));
     return shape && min_a > 0.0 && min_b > 0.0 && min_a * min_b >= 0x1p-60 * sum_a * sum_b;
 }
 

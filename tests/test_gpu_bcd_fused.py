@@ -343,3 +343,46 @@ def test_two_pass_combine_splits(gpu_lib, bulk, n, m):
     # FP64: the sums of squares over all tiles; FP32 rounds each row sum to 2^-23
     np.testing.assert_allclose(r.mar_errs, o["mar_errs"], rtol=1e-2 if bulk == "fp32" else 1e-7,
                                atol=2e-7 if bulk == "fp32" else 1e-14)
+
+
+# --- tall, narrow matrices -------------------------------------------------------
+
+# (bulk, m, rows per compute unit, single read): the strips of the two-pass form
+# are 256 (FP32) and 128 (FP64) columns wide; one or two strips and more than 192
+# (FP64 arithmetic: 128) rows per unit and strip take two passes
+@pytest.mark.parametrize("bulk,m,rows,single", [
+    ("fp32", 40, 192, True), ("fp32", 40, 193, False), ("fp32", 256, 200, False),
+    ("fp32", 257, 384, True), ("fp32", 257, 385, False), ("fp32", 513, 400, True),
+    ("fp64", 40, 128, True), ("fp64", 40, 129, False), ("fp64", 129, 256, True),
+    ("fp64", 129, 257, False), ("fp64", 257, 300, True)])
+def test_tall_narrow_form(gpu_lib, bulk, m, rows, single):
+    import torch
+    n = rows * torch.cuda.get_device_properties(0).multi_processor_count
+    rng = np.random.default_rng(m)
+    x, y = rng.random((n, 1)), rng.random((1, m))
+    M = ((x - y) ** 2).astype(np.float32 if bulk == "fp32" else np.float64)
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    print("tall %dx%d %s" % (n, m, bulk), flush=True)
+    with gpu_lib.Problem(M, a, b, 0.05, bulk=bulk) as P:
+        P.profile(True)
+        r = P.solve(0, tol=0.0 if bulk == "fp64" else 1e-6, max_iter=3, compute_plan=False)
+        one, two = P.profile_stats(2 if bulk == "fp32" else 4)[0], P.profile_stats(0)[0]
+    assert (one, two) == ((r.niter + 1, 0) if single else (0, r.niter + 1))
+    o = O.sinkhorn_bcd(M.astype(np.float64), a, b, 0.05, tol=0.0, max_iter=r.niter)
+    assert rel_err(r.dual, o["dual"]) < (1e-6 if bulk == "fp32" else 1e-12)
+
+
+def test_tall_narrow_fp64_finish(gpu_lib):
+    # between the two limits: FP32 iterations in one read, their FP64 finish in two
+    import torch
+    n, m = 160 * torch.cuda.get_device_properties(0).multi_processor_count, 40
+    rng = np.random.default_rng(m)
+    M = ((rng.random((n, 1)) - rng.random((1, m))) ** 2).astype(np.float32)
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    with gpu_lib.Problem(M, a, b, 0.05) as P:
+        P.profile(True)
+        r = P.solve(0, tol=1e-12, max_iter=2000, compute_plan=False, verify=True)
+        counts = [P.profile_stats(k)[0] for k in (0, 2, 4)]
+    pf = r.stats["precise_from"]
+    assert pf >= 0 and counts == [r.niter - pf + 1, pf + 1, 0]
+    assert r.mar_err_fp64 < 1.05e-12
