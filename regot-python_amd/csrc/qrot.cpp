@@ -30,12 +30,13 @@ namespace {
 
 // M' for the column roots of the running call (2 n m elements moved once per
 // call, against a strided read of M per Newton step); false when there is no
-// room for it.
+// room for it, or more columns than its launch covers.
 bool form_transpose(regot_problem* p, QrotScratch& w)
 {
     if (w.mt_state != 0) return w.mt_state > 0;
-    const long esz = p->bulk == REGOT_F32 ? 4 : 8, al = 256 / esz;
-    w.ldt = (p->n + al - 1) / al * al;
+    if (p->m >= 1 << 30) return false;
+    const long esz = p->bulk == REGOT_F32 ? 4 : 8;
+    w.ldt = qrot_transpose_pitch(p->bulk, p->n);
     try {
         w.mt.ensure(static_cast<size_t>(p->m) * w.ldt * esz);
     } catch (const Error&) {
@@ -50,9 +51,22 @@ bool form_transpose(regot_problem* p, QrotScratch& w)
 
 }  // namespace
 
-void qrot_begin_call(regot_problem* p)
+// Whole 16-byte vectors, and 256-byte lines where that adds at most a quarter
+// (a 4-row M would grow 16-fold).
+long qrot_transpose_pitch(int bulk, int n)
 {
-    if (p->qrot) p->qrot->mt_state = 0;
+    const long esz = bulk == 0 ? 4 : 8;
+    const long al = (n * esz >= 1024 ? 256 : 16) / esz;
+    return (n + al - 1) / al * al;
+}
+
+QrotCall::~QrotCall()
+{
+    if (!p->qrot) return;
+    QrotScratch& w = *p->qrot;
+    w.mt_state = 0;
+    // (hipFree waits for the device)
+    if (w.mt.n > kQrotKeep) w.mt.release();
 }
 
 // Roots in one read of M or its transpose (qrot_root.hip); for rows or columns
@@ -1040,7 +1054,7 @@ int regot_qrot_solve(regot_problem* p, int solver, double tol, int max_iter, int
     res->solver = 100 + solver;
     res->n = p->n;
     res->m = p->m;
-    qrot_begin_call(p);
+    QrotCall call(p);
     solve_qrot(p, solver, tol, max_iter, verbose, o, res.get());
     *out = res.release();
     CAPI_END
@@ -1067,7 +1081,7 @@ int regot_qrot_optimal_beta(regot_problem* p, const double* alpha, double* beta)
     HIP_CHECK(hipSetDevice(p->device));
     DBuf<double> a(p->n), b(p->m);
     HIP_CHECK(hipMemcpyAsync(a.p, alpha, p->n * sizeof(double), hipMemcpyHostToDevice, p->stream));
-    qrot_begin_call(p);
+    QrotCall call(p);
     qrot_optimal(p, true, a.p, b.p);
     p->sync();
     HIP_CHECK(hipMemcpy(beta, b.p, p->m * sizeof(double), hipMemcpyDeviceToHost));
@@ -1081,7 +1095,7 @@ int regot_qrot_optimal_alpha(regot_problem* p, const double* beta, double* alpha
     HIP_CHECK(hipSetDevice(p->device));
     DBuf<double> a(p->n), b(p->m);
     HIP_CHECK(hipMemcpyAsync(b.p, beta, p->m * sizeof(double), hipMemcpyHostToDevice, p->stream));
-    qrot_begin_call(p);
+    QrotCall call(p);
     qrot_optimal(p, false, b.p, a.p);
     p->sync();
     HIP_CHECK(hipMemcpy(alpha, a.p, p->n * sizeof(double), hipMemcpyDeviceToHost));

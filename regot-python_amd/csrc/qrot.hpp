@@ -57,7 +57,7 @@ struct QrotScratch {
     std::unique_ptr<QrotHess> hess;
     // M transposed (m x n, pitch ldt) for the column roots: a workspace of the
     // call that is running (mt_state 0: not formed, 1: formed, -1: no room),
-    // formed again by each call since the caller may own M
+    // formed again by each call since the caller may own M (QrotCall)
     DBuf<unsigned char> mt;
     long ldt = 0;
     int mt_state = 0;
@@ -161,8 +161,21 @@ void apply_qrot_hess(regot_problem* p, QrotHess& H, const double* x, double tau,
 // gamma (n + m), src/qrot_problem.cpp:226-258.
 double qrot_obj_grad(regot_problem* p, const double* gamma, double* grad, double tau,
                      double* gnorm2);
-// Forget the transpose of the last call (its M may have changed since).
-void qrot_begin_call(regot_problem* p);
+// One call of the C-ABI that may form the transpose.  Its contents are forgotten
+// at the end (M may change before the next call) and its memory stays with the
+// handle up to kQrotKeep bytes: allocating and freeing 256 MiB takes 0.3 ms, a
+// fifth of a three-iteration solve of such a matrix, 4 GiB 0.6 ms, which is less
+// than one iteration on it.
+constexpr size_t kQrotKeep = static_cast<size_t>(512) << 20;
+struct QrotCall {
+    regot_problem* p;
+    explicit QrotCall(regot_problem* q) : p(q) {}
+    QrotCall(const QrotCall&) = delete;
+    QrotCall& operator=(const QrotCall&) = delete;
+    ~QrotCall();
+};
+// Row pitch of M' in elements.
+long qrot_transpose_pitch(int bulk, int n);
 // optimal_beta (cols = true: out = beta (m) given alpha = pot) or
 // optimal_alpha (cols = false: out = alpha (n) given beta = pot), device.
 void qrot_optimal(regot_problem* p, bool cols, const double* pot, double* out);

@@ -428,3 +428,34 @@ def test_qrot_primal_infinite_costs(gpu_lib):
     f0 = 0.5 * (D * D).sum() - reg * (alpha @ a + beta @ b)
     assert abs(f - f0) < 1e-13 * max(1.0, abs(f0)) and np.all(np.isfinite(g))
     assert prim == np.inf or np.isnan(prim)
+
+
+# the transpose of M that the column roots read belongs to the call: what stays
+# with the handle is bounded, and few rows are not padded to 256 bytes each
+@pytest.mark.parametrize("n,m,bulk", [(13000, 13500, "fp32"), (4, 3000000, "fp32"),
+                                      (3, 2000000, "fp64")])
+def test_qrot_transpose_is_given_back(gpu_lib, n, m, bulk):
+    import torch
+    dt = torch.float32 if bulk == "fp32" else torch.float64
+    ld = (m + 63) // 64 * 64
+    g = torch.Generator(device="cuda")
+    g.manual_seed(1)
+    M = torch.rand(n, ld, device="cuda", generator=g, dtype=dt)
+    reg = 0.1
+    a, b = np.full(n, 1.0 / n), np.full(m, 1.0 / m)
+    alpha = np.random.default_rng(0).uniform(0.0, 0.1, n)
+    torch.cuda.synchronize()
+    print("qrot transpose %dx%d %s" % (n, m, bulk), flush=True)
+    with gpu_lib.Problem.from_device(M.data_ptr(), n, m, np.float32 if bulk == "fp32"
+                                     else np.float64, a, b, reg, ldm=ld) as P:
+        P.qrot_optimal_alpha(np.zeros(m))     # the vectors and partial sums
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        beta = P.qrot_optimal_beta(alpha)
+        kept = before - torch.cuda.mem_get_info()[0]
+    size = n * m * (4 if bulk == "fp32" else 8)
+    assert kept <= min(1.5 * size, 512 << 20) + (64 << 20)
+    # sum_i (beta_j + alpha_i - M_ij)_+ = reg b_j on a few columns
+    for j in range(0, m, m // 7):
+        s = np.maximum(beta[j] + alpha - M[:, j].double().cpu().numpy(), 0.0).sum()
+        assert abs(s - reg * b[j]) < 1e-9 * reg * b[j] + 1e-13
