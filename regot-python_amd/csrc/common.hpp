@@ -49,6 +49,35 @@ enum Status : int {
 
 #define KERNEL_CHECK() HIP_CHECK(hipGetLastError())
 
+// What a failed device allocation may have back before it is tried once more:
+// memory that the handle whose call runs on this thread keeps for later calls.
+struct Spare {
+    void* owner = nullptr;
+    void (*give_back)(void*) = nullptr;
+};
+inline thread_local Spare spare_memory;
+struct SpareScope {
+    Spare was;
+    SpareScope(void* owner, void (*give_back)(void*)) : was(spare_memory)
+    {
+        spare_memory = Spare{owner, give_back};
+    }
+    SpareScope(const SpareScope&) = delete;
+    SpareScope& operator=(const SpareScope&) = delete;
+    ~SpareScope() { spare_memory = was; }
+};
+
+inline hipError_t device_malloc(void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && spare_memory.give_back) {
+        (void)hipGetLastError();
+        spare_memory.give_back(spare_memory.owner);
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 // Device allocation (hipMalloc), released on destruction, or a part of a Slab.
 template <typename T>
 struct DBuf {
@@ -74,7 +103,7 @@ struct DBuf {
     {
         release();
         if (count == 0) count = 1;
-        hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T));
+        hipError_t e = device_malloc(reinterpret_cast<void**>(&p), count * sizeof(T));
         if (e != hipSuccess) {
             p = nullptr;
             fail(E_NOMEM, "hipMalloc of %zu bytes failed: %s", count * sizeof(T),

@@ -163,7 +163,7 @@ int regot_implicit_grad(regot_problem* p, const double* gamma, int loss, double 
         if (loss != 0 && loss != 1) fail(E_INVALID, "loss must be 0 (entropic) or 1 (sharp)");
         if (G_dtype != REGOT_F32 && G_dtype != REGOT_F64) fail(E_INVALID, "bad G dtype");
         if (ldg < p->m) fail(E_INVALID, "ldg %lld < m %d", ldg, p->m);
-        HIP_CHECK(hipSetDevice(p->device));
+        HandleCall handle(p);
         const int n = p->n, m = p->m;
         const long N = static_cast<long>(n) + m - 1;
         hipStream_t s = p->stream;

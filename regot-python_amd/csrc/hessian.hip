@@ -419,7 +419,7 @@ void hess_ensure_transpose(regot_problem* p)
     const size_t esz = p->bulk == 0 ? 4 : 8;
     const long align_el = 256 / static_cast<long>(esz);
     p->ldt = (p->n + align_el - 1) / align_el * align_el;
-    HIP_CHECK(hipMalloc(&p->dMT, static_cast<size_t>(p->m) * p->ldt * esz));
+    HIP_CHECK(device_malloc(&p->dMT, static_cast<size_t>(p->m) * p->ldt * esz));
     launch_transpose(p->bulk, p->dM, p->ldm, p->n, p->m, p->dMT, p->ldt, p->stream);
 }
 
@@ -550,7 +550,7 @@ static void prepare(regot_problem* p, SparseHessian& H, const double* d_gamma, c
     H.rcnt.ensure(n + 1);   // also receives an (n+1)-entry scan
     H.zcnt.ensure(n);
     H.mf = false;
-    H.compact = false;
+    H.cg_copy = 0;
     launch_split_gamma(d_gamma, n, m, H.vn, H.vm, s);
     hipLaunchKernelGGL(k_hess_diag, dim3(ceil_div(std::max(n, m), 256)), dim3(256), 0, s, d_grad,
                        p->a.p, p->b.p, n, m, p->reg, H.h1.p, H.h2.p);
@@ -790,11 +790,13 @@ struct CgSide {
 constexpr long long kCgLdsMin = 1000000;
 
 // What the products of cg_lds.hip read, formed once per build.  False: FP32
-// bulk and no memory for the compact copies (12 bytes per entry).
+// bulk and no memory for the compact copies (asked for once per build).
 static bool cg_entries(regot_problem* p, SparseHessian& H, CgEntries* e)
 {
     if (p->bulk != 0) return true;
-    if (!H.compact) {
+    if (H.cg_copy < 0) return false;
+    if (H.cg_copy == 0) {
+        H.cg_copy = 2;
         try {
             H.rval32.ensure(H.nnz);
             H.cval32.ensure(H.nnz);
@@ -802,11 +804,13 @@ static bool cg_entries(regot_problem* p, SparseHessian& H, CgEntries* e)
             H.rowind16.ensure(H.nnz);
         } catch (const Error&) {
             (void)hipGetLastError();
+            H.free_cg_copy();
+            H.cg_copy = -1;
             return false;
         }
         launch_cg_compact(H.rval, H.colind, H.nnz, p->reg, H.rval32, H.colind16, p->stream);
         launch_cg_compact(H.cval, H.rowind, H.nnz, p->reg, H.cval32, H.rowind16, p->stream);
-        H.compact = true;
+        H.cg_copy = 1;
     }
     e->rval32 = H.rval32;
     e->cval32 = H.cval32;
@@ -855,11 +859,6 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
         }
     }
     const double* dinv = jacobi ? H.cg_dinv.p : nullptr;
-    CgEntries ent;
-    // the kernels of cg_lds.hip are the 64-lane form
-    const bool lds = !H.mf && (lpr_r == 64 || lpr_c == 64) && H.nnz >= kCgLdsMin &&
-                     cg_lds_ok(n, m1, p->ncu) && cg_entries(p, H, &ent);
-    const bool lds_r = lds && lpr_r == 64, lds_c = lds && lpr_c == 64;
 
     // per side: x = x0 (or 0), r = rhs - Delta x, u = D^-1 r (or r),
     // w = Delta u (in q), p = s = 0 (beta_0 = 0)
@@ -916,6 +915,12 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
         a.dinv = dinv;
         a.rep = c.rep->d;
     }
+    // After the last allocation of the call, which may take the copies' memory.
+    // The kernels of cg_lds.hip are the 64-lane form.
+    CgEntries ent;
+    const bool lds = !H.mf && (lpr_r == 64 || lpr_c == 64) && H.nnz >= kCgLdsMin &&
+                     cg_lds_ok(n, m1, p->ncu) && cg_entries(p, H, &ent);
+    const bool lds_r = lds && lpr_r == 64, lds_c = lds && lpr_c == 64;
     const CgArgs& a0 = S[0].a;
     const CgArgs& a1 = S[nr - 1].a;
     auto begin_of = [](const CgArgs& a) { return CgBegin{a.part, a.scal, a.ctl, a.rep}; };
@@ -1170,7 +1175,6 @@ int set_error(int code, const char* what);
 static void hess_check(regot_problem* p, bool need_built)
 {
     if (!p) fail(E_INVALID, "null problem handle");
-    HIP_CHECK(hipSetDevice(p->device));
     if (need_built && (!p->hess || (!p->hess->mf && !p->hess->rowptr.p)))
         fail(E_STATE, "no sparsified Hessian: call regot_sparsified_hess* first");
 }
@@ -1190,6 +1194,7 @@ int regot_sparsified_hess(regot_problem* p, const double* gamma, double delta,
 {
     CAPI_BEGIN
     hess_check(p, false);
+    HandleCall handle(p);
     if (!gamma) fail(E_INVALID, "null gamma");
     upload_and_grad(p, gamma);
     hess_threshold(p, p->gamma, p->grad, delta, density_hint);
@@ -1202,6 +1207,7 @@ int regot_sparsified_hess_with_density(regot_problem* p, const double* gamma, do
 {
     CAPI_BEGIN
     hess_check(p, false);
+    HandleCall handle(p);
     if (!gamma) fail(E_INVALID, "null gamma");
     upload_and_grad(p, gamma);
     hess_topk(p, p->gamma, p->grad, density);
@@ -1222,6 +1228,7 @@ int regot_hess_info(regot_problem* p, long long* nnz_stored, long long* nnz_zero
 {
     CAPI_BEGIN
     hess_check(p, true);
+    HandleCall handle(p);
     if (nnz_stored) *nnz_stored = p->hess->nnz;
     if (nnz_zero) *nnz_zero = p->hess->nnz_zero;
     if (density) *density = p->hess->density();
@@ -1233,6 +1240,7 @@ int regot_hess_export(regot_problem* p, double* h1, double* h2, int* colptr, int
 {
     CAPI_BEGIN
     hess_check(p, true);
+    HandleCall handle(p);
     SparseHessian& H = *p->hess;
     if (H.mf)
         fail(E_STATE, "the Hessian was built matrix-free and holds no CSR / CSC "
@@ -1257,6 +1265,7 @@ int regot_hess_apply_delta(regot_problem* p, const double* x, double shift, doub
 {
     CAPI_BEGIN
     hess_check(p, true);
+    HandleCall handle(p);
     const int m1 = p->m - 1;
     p->cin.ensure(m1);
     launch_copy(p->stage(x, m1), p->cin, m1, p->stream);
@@ -1269,6 +1278,7 @@ int regot_hess_apply_hs(regot_problem* p, const double* x, double* res)
 {
     CAPI_BEGIN
     hess_check(p, true);
+    HandleCall handle(p);
     const long N = p->n + p->m - 1;
     p->cin.ensure(N);
     p->cout.ensure(N);
@@ -1285,6 +1295,7 @@ int regot_hess_cg2(regot_problem* p, const double* rhs0, const double* rhs1, dou
 {
     CAPI_BEGIN
     hess_check(p, true);
+    HandleCall handle(p);
     if (!rhs0 || !rhs1 || !res0 || !res1 || !iters) fail(E_INVALID, "null argument");
     const long N = p->n + p->m - 1;
     DBuf<double> d0(N), d1(N), r0(N), r1(N);
@@ -1307,6 +1318,7 @@ int regot_hess_cg(regot_problem* p, const double* rhs, double shift, double tol,
 {
     CAPI_BEGIN
     hess_check(p, true);
+    HandleCall handle(p);
     const long N = p->n + p->m - 1;
     p->cin.ensure(N);
     p->cout.ensure(N);

@@ -236,7 +236,7 @@ int regot_primal_val(regot_problem* p, const double* gamma, double* value)
 {
     CAPI_BEGIN
     if (!p || !gamma || !value) fail(E_INVALID, "null argument");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     const int N = p->n + p->m - 1;
     HIP_CHECK(hipMemcpyAsync(p->gamma, gamma, N * sizeof(double), hipMemcpyHostToDevice,
                              p->stream));
@@ -250,7 +250,7 @@ int regot_round_plan(regot_problem* p, const double* gamma, double* plan)
 {
     CAPI_BEGIN
     if (!p || !gamma || !plan) fail(E_INVALID, "null argument");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     const int n = p->n, m = p->m;
     HIP_CHECK(hipMemcpyAsync(p->gamma, gamma, (n + m - 1) * sizeof(double),
                              hipMemcpyHostToDevice, p->stream));

@@ -455,10 +455,10 @@ int set_error(int code, const char* what)
     catch (const std::exception& e) { return set_error(E_INTERNAL, e.what()); }            \
     return OK;
 
-static void check_handle(const regot_problem* p)
+static regot_problem* check_handle(regot_problem* p)
 {
     if (!p) fail(E_INVALID, "null problem handle");
-    HIP_CHECK(hipSetDevice(p->device));
+    return p;
 }
 
 extern "C" {
@@ -537,7 +537,7 @@ int regot_problem_dims(const regot_problem* p, int* n, int* m, int* bulk)
 int regot_optimal_alpha(regot_problem* p, const double* beta_h, double* alpha_h)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     if (!beta_h || !alpha_h) fail(E_INVALID, "null vector");
     launch_copy(p->stage(beta_h, p->m), p->beta, p->m, p->stream);
     RowEpi e;
@@ -551,7 +551,7 @@ int regot_optimal_alpha(regot_problem* p, const double* beta_h, double* alpha_h)
 int regot_optimal_beta(regot_problem* p, const double* alpha_h, double* beta_h)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     if (!beta_h || !alpha_h) fail(E_INVALID, "null vector");
     launch_copy(p->stage(alpha_h, p->n), p->alpha, p->n, p->stream);
     ColEpi c;
@@ -564,7 +564,7 @@ int regot_optimal_beta(regot_problem* p, const double* alpha_h, double* beta_h)
 int regot_dual_obj(regot_problem* p, const double* gamma_h, double* obj)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     if (!gamma_h || !obj) fail(E_INVALID, "null pointer");
     *obj = p->dev_obj(p->stage_gamma(gamma_h));
     CAPI_END
@@ -573,7 +573,7 @@ int regot_dual_obj(regot_problem* p, const double* gamma_h, double* obj)
 int regot_dual_obj_grad(regot_problem* p, const double* gamma_h, double* obj, double* grad_h)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     if (!gamma_h || !obj || !grad_h) fail(E_INVALID, "null pointer");
     const long N = p->n + p->m - 1;
     *obj = p->dev_obj_grad(p->stage_gamma(gamma_h), p->stage_out(N), nullptr);
@@ -584,7 +584,7 @@ int regot_dual_obj_grad(regot_problem* p, const double* gamma_h, double* obj, do
 int regot_get_plan(regot_problem* p, const double* gamma_h, double* plan)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     if (!gamma_h || !plan) fail(E_INVALID, "null pointer");
     const long N = p->n + p->m - 1;
     HIP_CHECK(hipMemcpyAsync(p->gamma, gamma_h, N * sizeof(double), hipMemcpyHostToDevice,
@@ -606,7 +606,7 @@ int regot_get_plan(regot_problem* p, const double* gamma_h, double* plan)
 int regot_profile_enable(regot_problem* p, int on)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     p->prof = (on != 0);
     CAPI_END
 }
@@ -614,7 +614,7 @@ int regot_profile_enable(regot_problem* p, int on)
 int regot_profile_get(regot_problem* p, int kind, long long* launches, double* total_ms)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     if (kind < 0 || kind > 5) fail(E_INVALID, "profile kind %d", kind);
     p->prof_collect();
     if (launches) *launches = p->prof_slot[kind].launches;
@@ -625,7 +625,7 @@ int regot_profile_get(regot_problem* p, int kind, long long* launches, double* t
 int regot_profile_reset(regot_problem* p)
 {
     CAPI_BEGIN
-    check_handle(p);
+    HandleCall handle(check_handle(p));
     p->prof_collect();
     for (auto& s : p->prof_slot) {
         s.launches = 0;

@@ -223,6 +223,10 @@ struct regot_problem {
     // Row sums land in rsum, column sums in csum.  Returns f; *gnorm2 = ||g||^2.
     double dev_obj_grad(const double* d_gamma, double* d_grad, double* gnorm2);
 
+    // Free what the handle (a regot_problem) keeps only to save later calls work
+    // (the QROT transpose, the compact CG entries); they are formed again.
+    static void give_back(void* handle);
+
     void sync();
     void prof_begin(int kind, hipEvent_t* stop_out);
     void prof_end(int kind, hipEvent_t stop);
@@ -235,3 +239,17 @@ struct regot_problem {
     // a later commit.
     void prof_drop_after(long last);
 };
+
+namespace regot {
+
+// One call of the C-ABI on a handle: its device, and its spare memory for
+// allocations that fail.
+struct HandleCall {
+    SpareScope spare;
+    explicit HandleCall(regot_problem* p) : spare(p, &regot_problem::give_back)
+    {
+        HIP_CHECK(hipSetDevice(p->device));
+    }
+};
+
+}  // namespace regot

@@ -60,6 +60,23 @@ long qrot_transpose_pitch(int bulk, int n)
     return (n + al - 1) / al * al;
 }
 
+}  // namespace regot
+
+// In a running call, too: a transpose in use is not formed again (the call's
+// further column roots are passes over M), and a CG forms its compact entries
+// after its last allocation.  hipFree waits for the kernels that read them.
+void regot_problem::give_back(void* handle)
+{
+    regot_problem* p = static_cast<regot_problem*>(handle);
+    if (p->qrot && p->qrot->mt.p) {
+        p->qrot->mt.release();
+        if (p->qrot->mt_state > 0) p->qrot->mt_state = -1;
+    }
+    if (p->hess && (p->hess->cg_copy == 0 || p->hess->cg_copy == 1)) p->hess->free_cg_copy();
+}
+
+namespace regot {
+
 QrotCall::~QrotCall()
 {
     if (!p->qrot) return;
@@ -1038,7 +1055,7 @@ int regot_qrot_solve(regot_problem* p, int solver, double tol, int max_iter, int
     *out = nullptr;
     if (solver < 0 || solver > 8) fail(E_INVALID, "unknown QROT solver %d", solver);
     if (max_iter < 0) fail(E_INVALID, "max_iter must be >= 0");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     regot_opts o;
     if (opts) {
         o = *opts;
@@ -1065,7 +1082,7 @@ int regot_qrot_obj_grad(regot_problem* p, const double* gamma, double tau, doubl
 {
     CAPI_BEGIN
     if (!p || !gamma || !f) fail(E_INVALID, "null argument");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     const long N = static_cast<long>(p->n) + p->m;
     DBuf<double> g(N), gr(N);
     HIP_CHECK(hipMemcpyAsync(g.p, gamma, N * sizeof(double), hipMemcpyHostToDevice, p->stream));
@@ -1078,7 +1095,7 @@ int regot_qrot_optimal_beta(regot_problem* p, const double* alpha, double* beta)
 {
     CAPI_BEGIN
     if (!p || !alpha || !beta) fail(E_INVALID, "null argument");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     DBuf<double> a(p->n), b(p->m);
     HIP_CHECK(hipMemcpyAsync(a.p, alpha, p->n * sizeof(double), hipMemcpyHostToDevice, p->stream));
     QrotCall call(p);
@@ -1092,7 +1109,7 @@ int regot_qrot_optimal_alpha(regot_problem* p, const double* beta, double* alpha
 {
     CAPI_BEGIN
     if (!p || !alpha || !beta) fail(E_INVALID, "null argument");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     DBuf<double> a(p->n), b(p->m);
     HIP_CHECK(hipMemcpyAsync(b.p, beta, p->m * sizeof(double), hipMemcpyHostToDevice, p->stream));
     QrotCall call(p);
@@ -1106,7 +1123,7 @@ int regot_qrot_primal_val(regot_problem* p, const double* gamma, double* value)
 {
     CAPI_BEGIN
     if (!p || !gamma || !value) fail(E_INVALID, "null argument");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     const long N = static_cast<long>(p->n) + p->m;
     DBuf<double> g(N);
     HIP_CHECK(hipMemcpyAsync(g.p, gamma, N * sizeof(double), hipMemcpyHostToDevice, p->stream));
@@ -1121,7 +1138,7 @@ int regot_qrot_hess_solve(regot_problem* p, const double* gamma, const double* r
     CAPI_BEGIN
     if (!p || !gamma || !rhs || !out) fail(E_INVALID, "null argument");
     if (!(shift >= 0.0) || !(tau >= 0.0)) fail(E_INVALID, "shift and tau must be >= 0");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     const long N = static_cast<long>(p->n) + p->m;
     DBuf<double> g(N), r(N), x(N);
     HIP_CHECK(hipMemcpyAsync(g.p, gamma, N * sizeof(double), hipMemcpyHostToDevice, p->stream));

@@ -372,7 +372,7 @@ int regot_solve(regot_problem* p, int solver, double tol, int max_iter, int verb
     if (!out) fail(E_INVALID, "out is null");
     *out = nullptr;
     if (max_iter < 0) fail(E_INVALID, "max_iter must be >= 0");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     regot_opts o;
     if (opts)
         o = *opts;
@@ -447,7 +447,7 @@ int regot_result_plan(regot_problem* p, const regot_result* r, double* plan)
     if (r->qrot && !r->plan.p) {
         CAPI_BEGIN
         if (!plan) fail(E_INVALID, "plan is null");
-        HIP_CHECK(hipSetDevice(p->device));
+        HandleCall handle(p);
         qrot_plan_host(p, r->dual.data(), plan);
         CAPI_END
     }
@@ -468,7 +468,7 @@ int regot_result_verify(regot_problem* p, const regot_result* r, double* mar_err
     if (!p || !r) fail(E_INVALID, "null handle");
     if (p->n != r->n || p->m != r->m) fail(E_INVALID, "problem and result sizes differ");
     if (r->qrot) fail(E_INVALID, "verify applies to EROT results");
-    HIP_CHECK(hipSetDevice(p->device));
+    HandleCall handle(p);
     const int n = p->n, m = p->m;
     hipStream_t s = p->stream;
     HIP_CHECK(hipMemcpyAsync(p->gamma, r->dual.data(), (n + m - 1) * sizeof(double),

@@ -52,11 +52,20 @@ struct SparseHessian {
     DBuf<double> h1, h2;
     DBuf<int> rowptr, colind, colptr, rowind;
     DBuf<double> rval, cval;
-    // the entries as the large CG products read them (CgEntries), valid while
-    // compact is set
+    // the entries as the large CG products read them (CgEntries), 12 bytes each,
+    // formed by a build's first CG: 0 not formed, 1 formed, 2 being allocated,
+    // -1 no room
     DBuf<float> rval32, cval32;
     DBuf<unsigned short> colind16, rowind16;
-    bool compact = false;
+    int cg_copy = 0;
+    void free_cg_copy()
+    {
+        rval32.release();
+        cval32.release();
+        colind16.release();
+        rowind16.release();
+        cg_copy = 0;
+    }
     // work
     DBuf<double> tau, rho;
     DBuf<int> rcnt, ccnt, zcnt, csc_work;

@@ -15,7 +15,7 @@ def run_host_check(name, tmp_path):
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__",
                     "-I" + os.path.join(ROCM, "include"), "-I" + os.path.join(ROOT, "include"),
                     "-I" + os.path.join(ROOT, "regot-python_amd", "csrc"),
-                    os.path.join(ROOT, "tests", "host", name + ".cpp"), "-o", exe],
+                    os.path.join(ROOT, "tests", "host", name + ".cpp"), "-pthread", "-o", exe],
                    check=True, capture_output=True, text=True, timeout=120)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
@@ -35,3 +35,8 @@ def test_staging_memory_of_wide_problems(tmp_path):
 @needs_gxx
 def test_grids_of_wide_problems(tmp_path):
     run_host_check("grid_check", tmp_path)
+
+
+@needs_gxx
+def test_failed_allocations_take_the_handles_spare_memory(tmp_path):
+    run_host_check("spare_check", tmp_path)
