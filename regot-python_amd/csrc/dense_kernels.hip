@@ -131,16 +131,20 @@ __device__ void bcd_decide(const BcdState& st)
     // FP64: 267 us per iteration, now 264).
     constexpr int U = 8;
     const double2* cp2 = reinterpret_cast<const double2*>(cp);
-    for (int q = threadIdx.x; q < st.ntiles; q += 256 * U) {
+    int q0 = threadIdx.x;
+    for (; q0 + 256 * (U - 1) < st.ntiles; q0 += 256 * U) {
         double2 x[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) x[u] = cp2[min(q + 256 * u, st.ntiles - 1)];
+        for (int u = 0; u < U; u++) x[u] = cp2[q0 + 256 * u];
 #pragma unroll
-        for (int u = 0; u < U; u++)
-            if (q + 256 * u < st.ntiles) {
-                v[3] += x[u].x;
-                v[4] += x[u].y;
-            }
+        for (int u = 0; u < U; u++) {
+            v[3] += x[u].x;
+            v[4] += x[u].y;
+        }
+    }
+    for (; q0 < st.ntiles; q0 += 256) {
+        v[3] += cp[2 * q0];
+        v[4] += cp[2 * q0 + 1];
     }
     block_sums_256<5>(v);
     if (threadIdx.x != 0) return;
