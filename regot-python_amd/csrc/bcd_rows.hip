@@ -279,6 +279,11 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
         }
     }
 
+    // The records of up to 64 rows pass between lanes of wave 0 without a barrier;
+    // the wave's LDS stores and loads stay in program order.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
     // pitch is a multiple of 16: whole vectors, also past m
     double* pw = part + static_cast<long>(blockIdx.x) * pitch + col0;
 #pragma unroll
