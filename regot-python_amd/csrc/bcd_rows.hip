@@ -102,6 +102,7 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
     constexpr bool F64 = sizeof(TA) == 8;
     constexpr double LO = F64 ? 0x1p-400 : 0x1p-20, HI = F64 ? 0x1p400 : 0x1p20;
     static_assert(NW * R <= 64, "one lane per wave total");
+    static_assert(R <= 4, "FP32 terms of a column between FP64 additions");
     __shared__ double red[2][NW * R];
     __shared__ double redx[NW];
     __shared__ double rsum[NW][3];
@@ -259,7 +260,7 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
                         acc[c][v] = fma(static_cast<double>(e[r][c][v]),
                                         static_cast<double>(wr[r]), acc[c][v]);
                 } else {
-                    // at most R <= 8 FP32 terms between FP64 additions
+                    // R <= 4 FP32 terms between FP64 additions
                     TA x = e[0][c][v] * wr[0];
 #pragma unroll
                     for (int r = 1; r < R; r++) x = fma(e[r][c][v], wr[r], x);

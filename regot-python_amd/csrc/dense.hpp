@@ -32,11 +32,10 @@ struct ColEpi {
     const double* b = nullptr;
     const double* colpot = nullptr;  // beta used for column sums / the shift guess
     double* colsum = nullptr;        // sum_i exp((alpha_i + beta_j - M_ij)/reg)
-    // Column gradient: with beta_out, b_j * expm1(beta_out_j/reg + ln2 lse2 - log b_j)
-    // (the FP64 rounding residual of the update); otherwise colsum_j - b_j.
-    double* resid = nullptr;
-    // Per tile t of 16 columns (j < m-1 only): [2t] = sum resid_j^2,
-    // [2t+1] = sum beta_j b_j with beta = beta_out if set, else colpot.
+    // Per tile t of 16 columns (j < m-1 only): [2t] = sum resid_j^2, [2t+1] = sum
+    // beta_j b_j with beta = beta_out if set, else colpot.  resid_j: with beta_out,
+    // b_j * expm1(beta_out_j/reg + ln2 lse2 - log b_j) (the FP64 rounding residual
+    // of the update); otherwise colsum_j - b_j.
     // In BCD mode the half selected by the parity of k+1 is written.
     double* tilepart = nullptr;
     double reg = 1.0;

@@ -279,7 +279,7 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
     if (valid) {
         if (epi.lse2) epi.lse2[j] = L;
         double cs = 0.0;
-        if (epi.colsum || (epi.resid && !epi.beta_out)) {
+        if (epi.colsum || (epi.tilepart && !epi.beta_out)) {
             cs = exp2(cp * k + L);
             if (epi.colsum) epi.colsum[j] = cs;
         }
@@ -291,7 +291,6 @@ __global__ __launch_bounds__(256) void k_col_combine(const double* __restrict__ 
         } else {
             g = cs - bj;
         }
-        if (epi.resid) epi.resid[j] = g;
         if (j < m - 1) {
             r2 = g * g;
             bb = pot * bj;

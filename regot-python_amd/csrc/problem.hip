@@ -177,8 +177,6 @@ void regot_problem::setup(int n_, int m_, const void* M, int M_dtype, int bulk_,
     slab.add(csum, m);
     slab.add(gamma, static_cast<size_t>(n) + m);
     slab.add(grad, static_cast<size_t>(n) + m);
-    slab.add(scal, 64);
-    slab.add(ctl, 16);
     slab.add(part, static_cast<size_t>(nblk) * m);
     slab.make();
     HIP_CHECK(hipMemcpyAsync(a, a_h, n * sizeof(double), hipMemcpyHostToDevice, stream));

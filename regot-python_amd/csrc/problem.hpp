@@ -81,7 +81,7 @@ void launch_log_check(const double* x, double* y, long count, hipStream_t s);
 // Buffers of the on-device BCD loop, kept across solves on one handle.
 struct BcdWork {
     Slab slab;
-    DBuf<double> ap0, ap1, be0, be1, gcol, rpart, cpart, stall;
+    DBuf<double> ap0, ap1, be0, be1, rpart, cpart, stall;
     DBuf<double> fpart;         // column sums of the single-read pass (blocks x m)
     DBuf<int> ctl;
     MappedRing<double> hf, hg;
@@ -137,8 +137,7 @@ struct regot_problem {
     regot::DBuf<double> a, b, loga, logb;
 
     // scratch for the operator entry points and the drivers
-    regot::DBuf<double> alpha, beta, rsum, csum, gamma, grad, part, scal;
-    regot::DBuf<int> ctl;
+    regot::DBuf<double> alpha, beta, rsum, csum, gamma, grad, part;
     int nblk = 1;
     int ntiles = 1;
     std::unique_ptr<regot::BcdWork> bcd;

@@ -421,15 +421,14 @@ void sweep(regot_problem* p, const double* alpha, const double* beta, const Qrot
                            w.eb.p, rows, rowpart, colpart, scal);
         KERNEL_CHECK();
     };
-    constexpr int CW = MODE == SW_COLS ? 4 : 2;       // widest strip of the mode
     constexpr int RW = MODE == SW_GRAD ? 4 : 2;
     const int C = sweep_c(m, MODE);
     if (C == 1)
         nt ? go(k_qrot_sweep<TM, MODE, 1, 4, true>) : go(k_qrot_sweep<TM, MODE, 1, 4, false>);
     else if (C == 2)
         nt ? go(k_qrot_sweep<TM, MODE, 2, RW, true>) : go(k_qrot_sweep<TM, MODE, 2, RW, false>);
-    else
-        nt ? go(k_qrot_sweep<TM, MODE, CW, 2, true>) : go(k_qrot_sweep<TM, MODE, CW, 2, false>);
+    else if constexpr (MODE == SW_COLS)
+        nt ? go(k_qrot_sweep<TM, MODE, 4, 2, true>) : go(k_qrot_sweep<TM, MODE, 4, 2, false>);
 }
 
 template <int MODE>

@@ -88,7 +88,6 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
         w.slab.add(w.ap1, n);
         w.slab.add(w.be0, m);
         w.slab.add(w.be1, m);
-        w.slab.add(w.gcol, m);
         w.slab.add(w.rpart, 3L * std::max(nrb, nfb));
         w.slab.add(w.cpart, 4L * p->ntiles);
         w.slab.add(w.ctl, 4);
@@ -118,7 +117,6 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
     };
 
     ColEpi c0;
-    c0.resid = w.gcol;
     c0.tilepart = w.cpart;
     {
         FlagScope fs(p->precise, precise);
@@ -216,7 +214,6 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             st.beta = bk;
             ColEpi c;
             c.beta_out = bk1;
-            c.resid = w.gcol;
             c.tilepart = w.cpart;
             if (fused && (kk > 0 || !o.x0)) {
                 st.nrb = nfb;
@@ -305,7 +302,6 @@ void solve_bcd(regot_problem* p, double tol, int max_iter, int verbose, const re
             double* bk = (k0 & 1) ? w.be1.p : w.be0.p;
             ColEpi c;
             c.beta_out = bk;
-            c.resid = w.gcol;
             c.tilepart = w.cpart + 2L * p->ntiles * (k0 & 1);
             p->col_pass((k0 & 1) ? w.ap1.p : w.ap0.p, bk, c);
         }
