@@ -155,24 +155,28 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
 #pragma unroll
         for (int v = 0; v < V; v++) acc[c][v] = 0.0;
 
+    // A shift of 1e30 makes every term 0.  The repeats of the last row have weight
+    // 0 and must not have an infinite term; an infinite potential (a row without a
+    // finite cost) or one that is not a number (a warm start's) says nothing of the
+    // row's size, and the range test finds a shift if there is a finite term.
+    auto shift_at = [&](long i) {
+        const double s = row_shift(la, al, k);
+        return (i + lr < r1 && __builtin_isfinite(s)) ? s : 1e30;
+    };
+    double next_shl = shift_at(r0);
+
     auto step = [&](VT (&cur)[R][NC], VT (&nxt)[R][NC], long i0, int slot) {
-        if (!ONE) load_rows<TM, NC, R, NT>(M, ldm, i0 + R, r1, off, nxt);
         const double la0 = la, al0 = al, av0 = av;
-        double shl = row_shift(la, al, k);
+        double shl = next_shl;
         const bool row_in = lane < NW * R && i0 + lr < r1;
-        // A shift of 1e30 makes every term 0.  The repeats of the last row have
-        // weight 0 and must not have an infinite term; an infinite potential (a
-        // row without a finite cost) or one that is not a number (a warm start's)
-        // says nothing of the row's size, and the range test below finds a shift
-        // if there is a finite term.
-        shl = (row_in && __builtin_isfinite(shl)) ? shl : 1e30;
         if (!ONE) {
-            // the next step's row data
+            // the next step's row data, then its rows
             long i = i0 + R + lr;
             i = (i < r1) ? i : r1 - 1;
             la = loga[i];
             al = alpha[i];
             av = a[i];
+            load_rows<TM, NC, R, NT>(M, ldm, i0 + R, r1, off, nxt);
         }
         TA e[R][NC][V];
         double tot;
@@ -267,6 +271,8 @@ __global__ __launch_bounds__(T) void k_bcd_rows(
                     acc[c][v] += static_cast<double>(x);
                 }
             }
+        // off the next step's path (the row data came before its rows)
+        if (!ONE) next_shl = shift_at(i0 + R);
     };
 
     if (ONE) {
