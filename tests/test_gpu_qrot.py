@@ -427,6 +427,8 @@ def test_qrot_primal_infinite_costs(gpu_lib):
     D = np.maximum(0.6 - M, 0.0)
     f0 = 0.5 * (D * D).sum() - reg * (alpha @ a + beta @ b)
     assert abs(f - f0) < 1e-13 * max(1.0, abs(f0)) and np.all(np.isfinite(g))
+    # (row 3 and column 5 are met to rounding here, so the mass is 0, a NaN, or not;
+    # test_qrot_primal_of_forbidden_entries pins the value where it is not rounding)
     assert prim == np.inf or np.isnan(prim)
 
 
@@ -459,3 +461,25 @@ def test_qrot_transpose_is_given_back(gpu_lib, n, m, bulk):
     for j in range(0, m, m // 7):
         s = np.maximum(beta[j] + alpha - M[:, j].double().cpu().numpy(), 0.0).sum()
         assert abs(s - reg * b[j]) < 1e-9 * reg * b[j] + 1e-13
+
+
+def test_qrot_primal_of_forbidden_entries(gpu_lib):
+    # The rounding's rank-one term err_a err_b' / |err_a|_1 puts mass on an infinite
+    # cost, and the primal value is +inf, where both of its marginals are short of
+    # mass.
+    n, m, reg = 40, 330, 0.1
+    M, a, b = cloud_problem(n, m, d=4, seed=1)
+    finite = M.copy()
+    M[3, 5] = np.inf
+    with gpu_lib.Problem(M, a, b, reg) as P:
+        # no plan at all: every marginal is short by all of its mass
+        assert P.qrot_primal_val(np.zeros(n + m)) == np.inf
+        # ample plan but for row 3 and column 5, which have none
+        alpha, beta = np.full(n, 0.6), np.full(m, 0.6)
+        alpha[3], beta[5] = -5.0, -5.0
+        assert P.qrot_primal_val(np.concatenate([alpha, beta])) == np.inf
+        # a finite twin: T = 0, so the plan is a b' / sum a
+        with gpu_lib.Problem(finite, a, b, reg) as Q:
+            got = Q.qrot_primal_val(np.zeros(n + m))
+    want = a @ finite @ b + 0.5 * reg * (a @ a) * (b @ b)
+    assert abs(got - want) < 1e-13 * abs(want)
