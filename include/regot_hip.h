@@ -154,6 +154,11 @@ int regot_hess_info(regot_problem* p, long long* nnz_stored, long long* nnz_zero
  * Products, CG and the drivers' iterates agree with the stored form to
  * rounding (the sums run in another order). */
 int regot_set_hess_storage(regot_problem* p, int mode);
+/* Products of the CG with the gathered vector in LDS: they run from min_entries
+ * stored entries on (default 1000000; min_entries < 0 leaves the line where it
+ * is).  *products (nullable) = the products of that form launched so far on this
+ * handle.  Both forms give the same bits. */
+int regot_cg_lds(regot_problem* p, long long min_entries, long long* products);
 /* Copy h1 (n), h2 (m-1), CSC (colptr m, rowind nnz, cval nnz) and CSR
  * (rowptr n+1, colind nnz, rval nnz) to host; NULL skips an array.
  * (Hessian::to_spmat, src/sinkhorn_hess.cpp:57-96, builds the same matrix.) */

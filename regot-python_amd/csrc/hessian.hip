@@ -781,14 +781,6 @@ struct CgSide {
     CgArgs a;
 };
 
-// Stored entries from which the products keep their vector in LDS.  Below, the
-// copy of the vector costs more than the gathers: a solve of some 20 iterations
-// took per iteration, its set-up and copies included, from global memory and
-// from LDS: 0.72 M entries (6000^2 FP32) 35.8 and 37.0 us, 1.34 M (8192^2) 56.3
-// and 44.7, 1.80 M (6000^2) 49.3 and 38.9, 2.25 M (15000^2) 99.7 and 72.7, in
-// FP64 1.34 M (8192^2) 55.7 and 49.0.
-constexpr long long kCgLdsMin = 1000000;
-
 // What the products of cg_lds.hip read, formed once per build.  False: FP32
 // bulk and no memory for the compact copies (asked for once per build).
 static bool cg_entries(regot_problem* p, SparseHessian& H, CgEntries* e)
@@ -918,7 +910,7 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
     // After the last allocation of the call, which may take the copies' memory.
     // The kernels of cg_lds.hip are the 64-lane form.
     CgEntries ent;
-    const bool lds = !H.mf && (lpr_r == 64 || lpr_c == 64) && H.nnz >= kCgLdsMin &&
+    const bool lds = !H.mf && (lpr_r == 64 || lpr_c == 64) && H.nnz >= p->cg_lds_min &&
                      cg_lds_ok(n, m1, p->ncu) && cg_entries(p, H, &ent);
     const bool lds_r = lds && lpr_r == 64, lds_c = lds && lpr_c == 64;
     const CgArgs& a0 = S[0].a;
@@ -960,6 +952,7 @@ static void cg_delta_sides(regot_problem* p, int nr, CgSide* S, double shift, do
                 hipLaunchKernelGGL(k_cg_cols_mf, dim3(nbc), dim3(256), 0, s, a0, H.mf_part.p,
                                    H.mf_nwg);
             } else {
+                p->cg_lds_products += lds_r + lds_c;
                 if (lds_r)
                     launch_cg_rows_lds(a0, a1, ent, nr, p->ncu, s);
                 else
@@ -1221,6 +1214,15 @@ int regot_set_hess_storage(regot_problem* p, int mode)
     if (!p) fail(E_INVALID, "null problem handle");
     if (mode < -1 || mode > 1) fail(E_INVALID, "storage mode must be -1, 0 or 1 (got %d)", mode);
     p->hess_storage = mode;
+    CAPI_END
+}
+
+int regot_cg_lds(regot_problem* p, long long min_entries, long long* products)
+{
+    CAPI_BEGIN
+    if (!p) fail(E_INVALID, "null problem handle");
+    if (min_entries >= 0) p->cg_lds_min = min_entries;
+    if (products) *products = p->cg_lds_products;
     CAPI_END
 }
 

@@ -13,6 +13,14 @@ namespace regot {
 
 struct SparseHessian;  // sparse.hpp
 
+// Stored entries from which the products of a CG keep their vector in LDS.  Below,
+// the copy of the vector costs more than the gathers: a solve of some 20
+// iterations took per iteration, its set-up and copies included, from global
+// memory and from LDS: 0.72 M entries (6000^2 FP32) 35.8 and 37.0 us, 1.34 M
+// (8192^2) 56.3 and 44.7, 1.80 M (6000^2) 49.3 and 38.9, 2.25 M (15000^2) 99.7 and
+// 72.7, in FP64 1.34 M (8192^2) 55.7 and 49.0.
+constexpr long long kCgLdsMin = 1000000;
+
 // FP64 BLAS-1 helpers on device vectors (vec_kernels.hip).  Reductions run in
 // one workgroup in a fixed order, so they are reproducible.
 void vec_axpy(double* y, double alpha, const double* x, long count, hipStream_t s);
@@ -180,6 +188,10 @@ struct regot_problem {
     // dense enough, the Hessian C-ABI stores CSR / CSC; 0 always stored; 1
     // matrix-free wherever the bulk and shape allow.
     int hess_storage = -1;
+    // CG products with the vector in LDS (cg_lds.hip): from so many stored entries
+    // on, and those launched so far
+    long long cg_lds_min = regot::kCgLdsMin;
+    long long cg_lds_products = 0;
 
     // profiling of the hot passes: [0] row pass, [1] column pass (partial +
     // combine), [2] single-read BCD pass, [3] its column-sum combine, [4] and

@@ -404,6 +404,14 @@ class Problem:
         stored; 1: matrix-free wherever it applies (hess_export then fails)."""
         check(lib().regot_set_hess_storage(self._h, int(mode)))
 
+    def cg_lds(self, min_entries=-1):
+        """Run the CG's products with their vector in LDS from min_entries stored
+        entries on (negative: leave the line, 1000000 by default); the products of
+        that form launched so far.  Both forms give the same bits."""
+        done = _lib.ctypes.c_longlong()
+        check(lib().regot_cg_lds(self._h, int(min_entries), _lib.ctypes.byref(done)))
+        return done.value
+
     def hess_info(self):
         """(stored nnz, FP64-zero kept entries, Hessian density)"""
         a = _lib.ctypes.c_longlong()

@@ -134,3 +134,47 @@ def test_cg_products_with_vector_in_lds(gpu_lib, bulk, n, m, density):
             assert np.linalg.norm(res) <= tol * np.linalg.norm(rhs) + drift
             top = (r[:n] - S @ x[n:]) / d1
             assert np.allclose(x[:n], top, rtol=1e-12, atol=1e-12 * np.abs(top).max())
+
+
+# 64 lanes per row in both products (up to 8192 rows, or many entries a row), in the
+# columns alone (18431 x 11000, 0.5%) or the rows' (2050 x 18433), sets below the usual line, a row and a column
+# more than a multiple of 4 per workgroup, the longest vector
+@pytest.mark.parametrize("bulk,n,m,density,both", [
+    ("fp32", 3001, 3503, 0.1, True), ("fp64", 3001, 3503, 0.1, True),
+    ("fp32", 1025, 258, 0.02, True), ("fp64", 700, 901, 0.03, True),
+    ("fp32", 16387, 2050, 0.12, True), ("fp64", 2050, 18433, 0.02, False),
+    ("fp32", 18431, 11000, 0.005, False), ("fp32", 5, 3, 1.0, True)])
+def test_cg_products_in_lds_give_the_same_bits(gpu_lib, bulk, n, m, density, both):
+    reg = 0.02
+    M, a, b = cloud_problem(n, m, d=8, seed=83)
+    if bulk == "fp32":
+        M = M.astype(np.float32)
+    rng = np.random.default_rng(10)
+    N = n + m - 1
+    print("cg lds bits %dx%d %s" % (n, m, bulk), flush=True)
+    with gpu_lib.Problem(M, a, b, reg) as P:
+        P.set_hess_storage(0)
+        P.sparsified_hess_with_density(near_optimum(P), density)
+        shift = 1e-3 * P.hess_export()["h2"].max()
+        r0, r1 = rng.standard_normal(N), rng.standard_normal(N)
+        # a cap inside a batch of iterations, both ends of a solve, a pair
+        runs = [lambda: P.hess_cg(r0, shift, tol=1e-10, max_iter=2000),
+                lambda: P.hess_cg(r1, shift, tol=1e-10, max_iter=5),
+                lambda: P.hess_cg2(r0, r1, shift, tol=1e-10, max_iter=2000)]
+        P.cg_lds(1 << 62)
+        c0 = P.cg_lds()
+        old = [f() for f in runs]
+        c1 = P.cg_lds()
+        P.cg_lds(0)
+        new = [f() for f in runs]
+        c2 = P.cg_lds()
+    assert c1 == c0
+    # both products, or one, of every iteration; what is enqueued past the stop
+    # counts too
+    its = old[0][1] + old[1][1] + max(old[2][1])
+    assert c2 - c1 >= (2 if both else 1) * its > 0
+    if not both:
+        assert c2 - c1 < 2 * its
+    for x, y in zip(old[:2], new[:2]):
+        assert np.array_equal(x[0], y[0]) and x[1:] == y[1:]
+    assert np.array_equal(old[2][0], new[2][0]) and old[2][1:] == new[2][1:]
