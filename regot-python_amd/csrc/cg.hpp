@@ -6,6 +6,9 @@
 
 namespace regot {
 
+// ctl: [0] done, [1] iterations when done, [2] how the set-up ended it (k_cg_begin).
+// scal: [0..1] alpha by parity, [2..3] gamma by parity, [4] r.r of the last update,
+// [5] stop threshold, [6] rhs.rhs, [7] w.u of the set-up.
 struct CgArgs {
     const int* rowptr;
     const int* colind;

@@ -59,10 +59,7 @@ __global__ void k_sub_div(const double* w, const double* y, const double* h1, do
 // gamma_i / alpha_{i-1}); alpha_0, gamma_0 come from the set-up and beta_0 = 0.
 // The iteration index is a launch argument (the host enqueues at most
 // max_iter iterations); alpha and gamma are kept in two slots by parity so
-// no kernel reads a slot that it writes.
-// ctl: [0] done, [1] iterations when done.  scal: [0..1] alpha by parity,
-// [2..3] gamma by parity, [4] r.r of the last update, [5] stop threshold,
-// [6] rhs norm^2.
+// no kernel reads a slot that it writes.  The state is CgArgs (cg.hpp).
 
 // dinv_j = 1 / (h2_j + shift - sum_i sigma_ij^2 / (h1_i + shift)), the diagonal
 // of Delta (>= shift since sigma_ij <= h1_i and sum_i sigma_ij <= h2_j); one
@@ -92,9 +89,8 @@ __global__ __launch_bounds__(256) void k_delta_diag(const int* __restrict__ colp
     }
 }
 
-// u = dinv .* r (or r), partials of r.u and r.r per 1024 entries.
 // r as given, or (rhs set) r = rhs from a zero start: then also x = 0.  p = s =
-// 0, u = D^-1 r (or r); part = the workgroup's sums of r.u and r.r.
+// 0, u = D^-1 r (or r); part = the sums of r.u and r.r per 1024 entries.
 __global__ __launch_bounds__(256) void k_pcg_start(double* __restrict__ r,
                                                    const double* __restrict__ rhs,
                                                    const double* __restrict__ dinv, int m1,

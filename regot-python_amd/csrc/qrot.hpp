@@ -1,6 +1,6 @@
 // qrot.hpp -- quadratically regularised OT (QROT) on the device: the dual
-// passes (qrot_kernels.hip), the rounded primal value (primal_kernels.hip)
-// and the host drivers (qrot.cpp).  The QROT dual variable is
+// passes (qrot_kernels.hip), the roots (qrot_root.hip), the objective and the
+// rounded primal value (qrot_sweep.hip) and the host drivers (qrot.cpp).  The QROT dual variable is
 // gamma = [alpha (n); beta (m)]: no elimination of beta_m.
 #pragma once
 
