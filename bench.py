@@ -66,7 +66,7 @@ def measured_traffic(kernel, n):
         return None
     k = rec["kernels"]
     names = {"row_pass": ["k_row_pass<float, float, 4, true>"],
-             "col_pass": ["k_col_partial<float, float>", "k_col_combine<true, false>"],
+             "col_pass": ["k_col_partial<float, float>", "k_col_combine<true, false, 16>"],
              "bcd_fused": ["k_bcd_fused<8, true, 2>"]}[kernel]
     if not all(x in k for x in names):
         return None
